@@ -18,6 +18,7 @@
 
 #include "qo_device.hpp"
 #include "qo_internal.hpp"
+#include "qo_sort.hpp"
 #include "qo_split.hpp"
 
 namespace qo {
@@ -34,9 +35,11 @@ struct alignas(32) GEntry {
 };
 static_assert(sizeof(GEntry) == 32, "entry size");
 
-__global__ void k_gtable_init(GEntry *t, size_t n) {
+// Empties the global table and zeroes the call's `nc` counters.
+__global__ void k_gtable_init(GEntry *t, size_t n, uint64_t *counters, uint32_t nc) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     size_t stride = (size_t)gridDim.x * blockDim.x;
+    if (i < nc) counters[i] = 0;
     for (; i < n; i += stride) {
         GEntry e;
         e.key = kEmptyKey;
@@ -813,6 +816,72 @@ __global__ void k_gtable_gather(const GEntry *rows, const uint64_t *list, const 
     if (blockIdx.x == 0 && threadIdx.x == 0) *d_num = *overflow ? ~uint64_t(0) : g;
 }
 
+// The end of a group-by with at most kFinishGroups groups in one launch: one
+// work-group lists the occupied entries of the global table and the finished
+// rows as (key, source), sorts the list in LDS and writes the output columns.
+// One CU reads the table (32 B per entry, at least two entries per group), so
+// the time grows with the capacity: against the collect / list / sort / gather
+// launches a group-by of 200,000 rows takes 23.7 us instead of 32.7 with 16
+// groups, 35.7 instead of 43.6 with 1024, 54.9 instead of 58.4 with 2048, and
+// 78.5 instead of 75.0 with 4096 (so the limit is 2048).
+template <int ITEMS>
+__global__ __launch_bounds__(kBlockSortThreads) void k_groupby_finish(const GEntry *__restrict__ t, uint32_t entries,
+                                                                      const GEntry *__restrict__ rows,
+                                                                      const uint64_t *d_rows, uint32_t cap,
+                                                                      const uint32_t *overflow, int32_t *okey,
+                                                                      int64_t *ocount, int64_t *osum, int32_t *omin,
+                                                                      int32_t *omax, uint64_t *d_num) {
+    __shared__ BlockSort<ITEMS, false> S;
+    __shared__ uint32_t s_n;
+    constexpr uint32_t kRow = 1u << 31;  // source is a finished row, not a table entry
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    const uint64_t nrows = *d_rows;
+    const uint32_t r = nrows < cap ? (uint32_t)nrows : cap;
+    for (uint32_t i = threadIdx.x; i < r; i += kBlockSortThreads)
+        S.key[i] = ((uint64_t)(rows[i].key ^ 0x80000000u) << 32) | (i | kRow);
+    constexpr uint32_t kU = 4;  // entries in flight per thread
+    for (uint32_t i0 = 0; i0 < entries; i0 += kU * kBlockSortThreads) {
+        uint64_t c[kU];
+        uint32_t k[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+            const uint32_t i = i0 + u * kBlockSortThreads + threadIdx.x;
+            c[u] = i < entries ? t[i].cnt : 0;
+            k[u] = i < entries ? t[i].key : 0;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) {
+            const uint64_t m = ballot(c[u] != 0);
+            if (m == 0) continue;  // wave-uniform
+            uint32_t base = 0;
+            if (lane_id() == 0) base = atomicAdd(&s_n, popc(m));
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            const uint32_t at = r + base + popc(m & lanemask_lt());
+            if (c[u] != 0 && at < cap)
+                S.key[at] = ((uint64_t)(k[u] ^ 0x80000000u) << 32) | (i0 + u * kBlockSortThreads + threadIdx.x);
+        }
+    }
+    __syncthreads();
+    const uint64_t total = nrows + s_n;
+    const uint32_t g = total < cap ? (uint32_t)total : cap;
+    if (threadIdx.x == 0) *d_num = *overflow ? ~uint64_t(0) : total;
+    if (g == 0) return;  // whole block
+    block_sort<ITEMS, false>(S, g, 32, 64);
+    for (uint32_t i = threadIdx.x; i < g; i += kBlockSortThreads) {
+        const uint64_t v = S.key[i];
+        const uint32_t src = (uint32_t)v;
+        const GEntry &e = (src & kRow) ? rows[src & ~kRow] : t[src];
+        okey[i] = (int32_t)((uint32_t)(v >> 32) ^ 0x80000000u);
+        ocount[i] = (int64_t)e.cnt;
+        osum[i] = (int64_t)e.sum;
+        omin[i] = e.mn;
+        omax[i] = e.mx;
+    }
+}
+
+constexpr size_t kFinishGroups = 2048;
+
 struct GroupbyPlan {
     uint64_t gmask;
     size_t entries;
@@ -898,9 +967,8 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
     uint64_t *list = b.list;
     void *rws = b.rws;
     uint32_t *overflow = reinterpret_cast<uint32_t *>(counters + 1);
-    QO_TRY(launch_fill_u64(counters, 0, 4, st));
     const unsigned ig = grid_for(p.entries, 256, (unsigned)props().cu_count * 16);
-    k_gtable_init<<<ig, 256, 0, st>>>(gt, p.entries);
+    k_gtable_init<<<ig, 256, 0, st>>>(gt, p.entries, counters, 4);
     QO_LAUNCHED();
     if (n && pp.on) {
         const uint32_t nb = 1u << pp.s.L;
@@ -968,6 +1036,18 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
         }
 #undef QO_GBH
         QO_LAUNCHED();
+    }
+    if (group_capacity > 0 && group_capacity <= kFinishGroups) {
+        const uint32_t entries = (uint32_t)p.entries, cap = (uint32_t)group_capacity;
+        if (group_capacity <= kBlockSortThreads)
+            k_groupby_finish<1><<<1, kBlockSortThreads, 0, st>>>(gt, entries, b.rows, counters, cap, overflow, okey,
+                                                                 ocount, osum, omin, omax, d_num);
+        else
+            k_groupby_finish<2><<<1, kBlockSortThreads, 0, st>>>(gt, entries, b.rows, counters, cap, overflow, okey,
+                                                                 ocount, osum, omin, omax, d_num);
+        static_assert(kFinishGroups <= 2 * kBlockSortThreads, "the list fits the block sort");
+        QO_LAUNCHED();
+        return QO_OK;
     }
     unsigned long long *d_rows = reinterpret_cast<unsigned long long *>(counters);
     const unsigned cg = grid_for(p.entries, 256 * kCollectJ, (unsigned)props().cu_count * 4);

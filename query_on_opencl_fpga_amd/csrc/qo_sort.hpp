@@ -5,6 +5,8 @@
 
 #include <cstdint>
 
+#include "qo_device.hpp"
+
 namespace qo {
 
 constexpr int kSortItems = 16;
@@ -65,6 +67,120 @@ __host__ __device__ __forceinline__ int32_t join_sort_key_key(uint64_t k) {
 }
 __host__ __device__ __forceinline__ int32_t join_sort_key_spay(uint64_t k) {
     return (int32_t)((uint32_t)k ^ 0x80000000u);
+}
+
+// Lanes of this wave that are active and hold the same 8-bit digit.
+QO_DEV uint64_t match_digit(uint32_t d, bool valid) {
+    uint64_t m = ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        uint64_t bb = ballot((d >> b) & 1u);
+        m &= ((d >> b) & 1u) ? bb : ~bb;
+    }
+    return m;
+}
+
+// One-block stable radix sort of up to kBlockSortThreads * ITEMS 64-bit keys
+// (and 32-bit values) that lie in LDS.  What bounds it is the chain of passes:
+// a pass reads the block's keys, ranks them with wave ballots, scans 16 x 256
+// digit counts and scatters them back, about 2 us each at one key per thread
+// and 7 us at eight.  A launch per step of a pass (histogram, scan, placement)
+// takes 13 to 17 us per pass for arrays of this size.  Digits in which all
+// keys agree get no pass, so a narrow key range costs nothing.
+constexpr int kBlockSortThreads = 1024;
+constexpr int kBlockSortWaves = kBlockSortThreads / kWave;
+
+template <int ITEMS, bool HAS_VAL>
+struct BlockSort {
+    static constexpr uint32_t kMax = (uint32_t)kBlockSortThreads * ITEMS;
+    uint64_t key[kMax];
+    uint32_t val[HAS_VAL ? kMax : 1];
+    uint32_t cnt[kBlockSortWaves][256];
+    uint32_t dpre[256];
+    uint32_t w[kBlockSortWaves];
+    uint64_t diff[kBlockSortWaves];
+};
+
+// Sorts S.key[0, n) (and S.val) by bits [lo_bit, hi_bit) (whole 8-bit digits
+// from lo_bit).  All threads call it after a barrier that follows the writes of
+// S; on return (after a barrier) S holds the sorted array.
+template <int ITEMS, bool HAS_VAL>
+QO_DEV void block_sort(BlockSort<ITEMS, HAS_VAL> &S, uint32_t n, int lo_bit, int hi_bit) {
+    const unsigned w = wave_id(), lane = lane_id();
+    // Wave w owns positions [w * 64 J, (w + 1) * 64 J): all waves share a short array.
+    const int J = (int)((n + kBlockSortThreads - 1) / kBlockSortThreads);
+    const uint32_t wb = w * (uint32_t)J * kWave;
+    uint64_t k[ITEMS];
+    uint32_t v[ITEMS], rank[ITEMS];
+    // Bits in which any key differs from the first.
+    uint64_t diff = 0;
+    const uint64_t first = S.key[0];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+        const uint32_t idx = wb + j * kWave + lane;
+        if (j < J && idx < n) diff |= S.key[idx] ^ first;
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) diff |= __shfl_xor(diff, o, kWave);
+    if (lane == 0) S.diff[w] = diff;
+    __syncthreads();
+    diff = 0;
+#pragma unroll
+    for (int i = 0; i < kBlockSortWaves; ++i) diff |= S.diff[i];
+    for (int sh = lo_bit; sh < hi_bit; sh += 8) {
+        if (((diff >> sh) & 255u) == 0) continue;  // block-uniform
+#pragma unroll
+        for (int i = 0; i < 256 / kWave; ++i) S.cnt[w][i * kWave + lane] = 0;
+        wave_lockstep();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            if (j >= J) break;
+            const uint32_t idx = wb + j * kWave + lane;
+            const bool valid = idx < n;
+            k[j] = valid ? S.key[idx] : 0;
+            if (HAS_VAL) v[j] = valid ? S.val[idx] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            if (j >= J) break;
+            const bool valid = wb + j * kWave + lane < n;
+            const uint32_t d = (uint32_t)(k[j] >> sh) & 255u;
+            const uint64_t m = match_digit(d, valid);
+            const uint32_t pre = S.cnt[w][d];
+            const uint32_t r = popc(m & lanemask_lt());
+            wave_lockstep();  // every lane has read its digit's count before the leaders advance it
+            if (valid && r == 0) S.cnt[w][d] = pre + popc(m);
+            wave_lockstep();
+            rank[j] = pre + r;
+        }
+        __syncthreads();
+        uint32_t tot = 0;
+        if (threadIdx.x < 256) {
+            uint32_t c[kBlockSortWaves];
+#pragma unroll
+            for (int i = 0; i < kBlockSortWaves; ++i) c[i] = S.cnt[i][threadIdx.x];
+#pragma unroll
+            for (int i = 0; i < kBlockSortWaves; ++i) {
+                S.cnt[i][threadIdx.x] = tot;
+                tot += c[i];
+            }
+        }
+        // Threads 0..255 come first in the block, so their exclusive scan is the digit start.
+        const uint32_t start = block_excl_scan<kBlockSortWaves>(tot, S.w);
+        if (threadIdx.x < 256) S.dpre[threadIdx.x] = start;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            if (j >= J) break;
+            if (wb + j * kWave + lane < n) {
+                const uint32_t d = (uint32_t)(k[j] >> sh) & 255u;
+                const uint32_t p = S.dpre[d] + S.cnt[w][d] + rank[j];
+                S.key[p] = k[j];
+                if (HAS_VAL) S.val[p] = v[j];
+            }
+        }
+        __syncthreads();
+    }
 }
 
 }  // namespace qo

@@ -1,0 +1,53 @@
+"""GPU: the one-work-group sort of small arrays and the one-launch end of a
+group-by, at the edges of their size ranges, against the oracle (exact)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+SIZES = [1, 2, 63, 64, 65, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 8192, 8193]
+
+
+@pytest.mark.parametrize("bits", [0, 7, 20, 32])
+@pytest.mark.parametrize("n", SIZES)
+def test_small_sort_records(qo, orc, n, bits):
+    """Stable over ties (0 bits: one key), digits that all keys share, full-range keys."""
+    rec = np.empty((n, 2), np.uint32)
+    rec[:, 0] = np.arange(n)
+    y = orc.gen_uniform_u32(n, 5, 1, 0, 0)
+    rec[:, 1] = (y & np.uint32((1 << bits) - 1 if bits < 32 else 0xFFFFFFFF)) + np.uint32(0x7F0000 if bits < 32 else 0)
+    assert np.array_equal(qo.operators.sort_records(rec), orc.sort_records(rec))
+
+
+@pytest.mark.parametrize("span", [1, 9, 1 << 31])
+@pytest.mark.parametrize("m", SIZES)
+def test_small_sort_join_rows(qo, orc, m, span):
+    """Signed keys around zero, runs longer than 64 rows (span 1 and 9), repeated s_payloads."""
+    k = (orc.gen_uniform_u32(m, 6, 0, 0, span).astype(np.int64) - span // 2).astype(np.int32)
+    sp = orc.gen_uniform_u32(m, 6, 1, 0, 0).astype(np.int32)
+    sp[::3] = -5
+    rp = k * np.int32(3) + np.int32(1)  # a function of the key: rows that tie are identical
+    got = qo.operators.sort_join_rows(k, rp, sp)
+    exp = orc.sort_join_rows(k, rp, sp)
+    for g, e in zip(got, exp):
+        assert np.array_equal(g, e)
+
+
+@pytest.mark.parametrize("groups,n", [(1, 5000), (1023, 5000), (1024, 40000), (1025, 40000), (2048, 70001),
+                                      (2049, 70001), (2048, (1 << 20) + 3)])
+def test_group_finish_edges(qo, orc, groups, n):
+    """Capacities around the one-launch end's limits, with the empty-marker key; the last size takes the
+    partitioned path, whose groups arrive as finished rows."""
+    k = orc.gen_uniform_u32(n, 7, 0, 0, groups).astype(np.int64) * 7919 - 12345
+    k[k == -12345 + 7919 * (groups - 1)] = -1
+    k = k.astype(np.int32)
+    v = orc.gen_uniform_u32(n, 7, 1, 0, 0).astype(np.int32)
+    for g, e in zip(qo.operators.groupby_agg(k, v, groups), orc.groupby_agg(k, v)):
+        assert np.array_equal(g, e)
+
+
+@pytest.mark.parametrize("cap", [1, 100, 1024, 1500])
+def test_group_finish_over_capacity(qo, orc, cap):
+    """More keys than the outputs hold: the count says so (or that the table overflowed)."""
+    k = orc.gen_uniform_u32(60000, 8, 0, 0, 50000).astype(np.int32)
+    with pytest.raises(qo._lib.QoError):
+        qo.operators.groupby_agg(k, k, cap)
