@@ -565,11 +565,22 @@ int launch_radix_rows_segments(uint64_t *keys, uint32_t *vals, uint64_t *kalt, u
     return QO_OK;
 }
 
-static void radix_carve(size_t n, bool with_vals, Carver &cv, uint64_t **kalt, uint32_t **valt, RowsBufs *rb) {
+// Long runs the list holds: enough that listing every one and sorting each in a
+// work-group stays cheaper than the eight full-width passes.
+static uint32_t long_runs_cap(size_t m) { return (uint32_t)(4096 + m / 1024); }
+// Longest run that one work-group sorts on its own (4.9 ns per row).
+static uint64_t long_run_limit(size_t m) { return (1u << 14) + m / 256; }
+
+static void radix_carve(size_t n, bool with_vals, Carver &cv, uint64_t **kalt, uint32_t **valt, RowsBufs *rb,
+                        uint32_t **runs = nullptr) {
     const uint32_t tiles = radix_tiles(n) + 1;
     *kalt = cv.take<uint64_t>(n ? n : 1);
     *valt = with_vals ? cv.take<uint32_t>(n ? n : 1) : nullptr;
     *rb = rows_carve(tiles, cv);
+    if (with_vals) {
+        uint32_t *list = cv.take<uint32_t>(long_runs_cap(n));
+        if (runs) *runs = list;
+    }
 }
 
 size_t radix_workspace_bytes(size_t n, bool with_vals) {
@@ -777,7 +788,7 @@ int sort_join_rows_ws(int32_t *key, int32_t *rpay, int32_t *spay, size_t m, void
     uint32_t *v32 = cv.take<uint32_t>(m);
     void *rws = cv.take<char>(radix_workspace_bytes(m, true));
     unsigned g = grid_for(m, 256, (unsigned)props().cu_count * 8);
-    uint32_t *flag = cv.take<uint32_t>(1);
+    uint32_t *flag = cv.take<uint32_t>(2);
     k_pack_join<<<g, 256, 0, st>>>(key, spay, rpay, m, k64, v32);
     QO_LAUNCHED();
     return sort_packed_join_rows(k64, v32, m, rws, key, rpay, spay, st, 64, flag);
@@ -793,8 +804,9 @@ size_t sort_join_rows_ws_bytes(size_t m) { return m * 12 + 2048 + radix_workspac
 // counts the run's rows that order before it (smaller s_payload, or equal and
 // earlier: stable) and writes itself to the output columns at run start + that
 // count.  Rows of runs that start outside the block's range are left to the
-// block that owns the start; a run longer than kFixRun sets *long_flag and is
-// not written.
+// block that owns the start; a run longer than kFixRun is not written: its
+// start goes to the list of long runs (k_fix_long), or, without a list, it sets
+// the flag.
 constexpr uint32_t kFixTile = 4096;
 constexpr uint32_t kFixRun = 64;
 constexpr uint32_t kFixWin = kFixTile + kFixRun;
@@ -802,9 +814,17 @@ constexpr uint32_t kFixThreads = 512;  // four blocks per CU (34 KB LDS each), 8
 constexpr uint32_t kFixRounds = (kFixWin + kFixThreads - 1) / kFixThreads;
 constexpr uint32_t kFixChunks = kFixWin / kWave + 2;  // marks of the window's chunks and one past it
 
+// Where the run pass leaves the runs longer than kFixRun.
+struct LongRuns {
+    uint32_t *flag;            // set: the rows need the full-width sort
+    uint32_t *n = nullptr;     // starts of the long runs (counted past cap too)
+    uint32_t *list = nullptr;  // null: a long run sets the flag
+    uint32_t cap = 0;
+};
+
 // Block work of the run pass: positions [t0, t0 + kFixTile) of m rows (k, v).
 QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__restrict__ v, size_t m, size_t t0,
-                          const RowOut &out, uint32_t *long_flag) {
+                          const RowOut &out, const LongRuns &lr) {
     static_assert(kFixWin % kWave == 0, "window of whole chunks");
     __shared__ uint32_t s_hi[kFixWin];
     __shared__ uint32_t s_lo[kFixWin + 4];  // 4 words of slack for the unrolled rank loop
@@ -837,6 +857,13 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
     }
     __syncthreads();
     bool long_run = false;
+    auto is_long = [&](uint32_t i, uint32_t s) {
+        long_run = true;
+        if (lr.list && i == s) {  // the run's first row lists it
+            const uint32_t at = atomicAdd(lr.n, 1u);
+            if (at < lr.cap) lr.list[at] = (uint32_t)(t0 + s);
+        }
+    };
     for (uint32_t i = threadIdx.x; i < len; i += kFixThreads) {
         const uint32_t c = i / kWave;  // uniform across the wave
         const uint64_t at_or_below = lane == kWave - 1 ? ~0ull : (2ull << lane) - 1;
@@ -860,11 +887,11 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
         } else if (s_mark[c + 1]) {
             e = (c + 1) * kWave + (uint32_t)__builtin_ctzll(s_mark[c + 1]);
         } else {
-            long_run = true;
+            is_long(i, s);
             continue;
         }
         if (e - s > kFixRun) {
-            long_run = true;
+            is_long(i, s);
             continue;
         }
         const uint32_t xl = s_lo[i];
@@ -882,12 +909,170 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
         out.spay[dst] = join_sort_key_spay(x);
         out.rpay[dst] = (int32_t)v[t0 + i];
     }
-    if (long_run) atomicOr(long_flag, 1u);
+    if (long_run && !lr.list) atomicOr(lr.flag, 1u);
 }
 
 __global__ __launch_bounds__(kFixThreads) void k_fix_runs(const uint64_t *__restrict__ k, const uint32_t *__restrict__ v,
-                                                          size_t m, RowOut out, uint32_t *long_flag) {
-    fix_runs_tile(k, v, m, (size_t)blockIdx.x * kFixTile, out, long_flag);
+                                                          size_t m, RowOut out, LongRuns lr) {
+    fix_runs_tile(k, v, m, (size_t)blockIdx.x * kFixTile, out, lr);
+}
+
+// The long runs of k_fix_runs, one work-group each in turn.  A run of up to
+// kLongLds rows is sorted by s_payload in LDS; a longer one, up to `longest`
+// rows, by four digit passes of this work-group between its places in (k, v)
+// and (kalt, valt), which no other run uses; a run longer still, or more runs
+// than the list holds, sets the flag (the full-width sort reads (k, v), where
+// every run is complete in some order at any time).  Bound by the passes' chain
+// of dependent LDS steps, with one work-group per run.  Before it, one key of
+// more than 64 rows sent all rows through eight more passes: 3,000,045 S rows
+// with 200,003 unevenly referenced dense keys (hottest key ~4000 rows) 557 ->
+// 376 us for the whole join, 60,000,045 with 4,000,003 3.94 -> 3.40 ms.
+constexpr int kLongItems = 6;
+constexpr uint32_t kLongLds = kLongItems * kBlockSortThreads;
+
+// End of the run of equal key that starts at s; `longest` rows at most are
+// looked at (s + longest + 1 is returned for a longer run).
+QO_DEV uint64_t run_end(const uint64_t *k, size_t m, uint64_t s, uint64_t longest, uint32_t *s_min) {
+    const uint32_t key = (uint32_t)(k[s] >> 32);
+    auto differs = [&](uint64_t p) { return p >= m || (uint32_t)(k[p] >> 32) != key; };
+    for (uint64_t from = s; from <= s + longest; from += (uint64_t)kBlockSortThreads * kWave) {
+        if (threadIdx.x == 0) *s_min = ~0u;
+        __syncthreads();
+        if (differs(from + (uint64_t)(threadIdx.x + 1) * kWave)) atomicMin(s_min, threadIdx.x);
+        __syncthreads();
+        const uint32_t c = *s_min;
+        __syncthreads();
+        if (c == ~0u) continue;  // block-uniform
+        const uint64_t p0 = from + (uint64_t)c * kWave;  // the end lies in (p0, p0 + 64]
+        if (threadIdx.x == 0) *s_min = kWave;
+        __syncthreads();
+        if (threadIdx.x < kWave && differs(p0 + threadIdx.x + 1)) atomicMin(s_min, threadIdx.x + 1);
+        __syncthreads();
+        const uint64_t e = p0 + *s_min;
+        __syncthreads();
+        return e;
+    }
+    return s + longest + 1;
+}
+
+__global__ __launch_bounds__(kBlockSortThreads) void k_fix_long(uint64_t *k, uint32_t *v, uint64_t *kalt,
+                                                                uint32_t *valt, size_t m, uint64_t longest, RowOut out,
+                                                                LongRuns lr) {
+    __shared__ BlockSort<kLongItems, false> S;
+    __shared__ uint32_t s_hist[4][256];
+    __shared__ uint32_t s_min;
+    const uint32_t n = *lr.n;
+    if (n > lr.cap) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *lr.flag = 1u;
+        return;  // whole block
+    }
+    const unsigned w = wave_id(), lane = lane_id();
+    for (uint32_t r = blockIdx.x; r < n; r += gridDim.x) {
+        const uint64_t s = lr.list[r];
+        const uint64_t e = run_end(k, m, s, longest, &s_min);
+        const uint64_t len = e - s;
+        const int32_t key = join_sort_key_key(k[s]);
+        if (len > longest) {
+            if (threadIdx.x == 0) *lr.flag = 1u;
+            continue;
+        }
+        if (len <= kLongLds) {
+            // Sorted as s_payload (order-preserving) << 32 | r_payload.
+            for (uint32_t i = threadIdx.x; i < (uint32_t)len; i += kBlockSortThreads)
+                S.key[i] = (k[s + i] << 32) | v[s + i];
+            __syncthreads();
+            block_sort<kLongItems, false>(S, (uint32_t)len, 32, 64);
+            for (uint32_t i = threadIdx.x; i < (uint32_t)len; i += kBlockSortThreads) {
+                const uint64_t x = S.key[i];
+                out.key[s + i] = key;
+                out.spay[s + i] = (int32_t)((uint32_t)(x >> 32) ^ 0x80000000u);
+                out.rpay[s + i] = (int32_t)(uint32_t)x;
+            }
+            __syncthreads();  // S is reused
+            continue;
+        }
+        // Digit counts of the four passes, then per pass the tiles in order.
+        for (uint32_t i = threadIdx.x; i < 1024; i += kBlockSortThreads) (&s_hist[0][0])[i] = 0;
+        __syncthreads();
+        for (uint64_t i = threadIdx.x; i < len; i += kBlockSortThreads) {
+            const uint32_t x = (uint32_t)k[s + i];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) atomicAdd(&s_hist[p][(x >> (8 * p)) & 255u], 1u);
+        }
+        uint64_t *ks = k + s, *kd = kalt + s;
+        uint32_t *vs = v + s, *vd = valt + s;
+        for (int p = 0; p < 4; ++p) {
+            __syncthreads();
+            const uint32_t c = threadIdx.x < 256 ? s_hist[p][threadIdx.x] : 0u;
+            const uint32_t start = block_excl_scan<kBlockSortWaves>(c, S.w);
+            if (threadIdx.x < 256) S.dpre[threadIdx.x] = start;
+            if (threadIdx.x == 0) s_min = 0;
+            __syncthreads();
+            if (c == (uint32_t)len) s_min = 1u;
+            __syncthreads();
+            if (s_min) continue;  // one digit: nothing moves
+            for (uint64_t t0 = 0; t0 < len; t0 += kLongLds) {
+                for (int i = 0; i < 256 / kWave; ++i) S.cnt[w][i * kWave + lane] = 0;
+                __syncthreads();
+                const uint32_t rem = (uint32_t)(len - t0 < kLongLds ? len - t0 : kLongLds);
+                uint64_t x[kLongItems];
+                uint32_t y[kLongItems], rank[kLongItems];
+#pragma unroll
+                for (int j = 0; j < kLongItems; ++j) {
+                    const uint32_t i = (w * kLongItems + j) * kWave + lane;
+                    x[j] = i < rem ? ks[t0 + i] : 0;
+                    y[j] = i < rem ? vs[t0 + i] : 0;
+                }
+#pragma unroll
+                for (int j = 0; j < kLongItems; ++j) {
+                    const bool valid = (w * kLongItems + j) * kWave + lane < rem;
+                    const uint32_t d = (uint32_t)(x[j] >> (8 * p)) & 255u;
+                    const uint64_t mk = match_digit(d, valid);
+                    const uint32_t pre = S.cnt[w][d];
+                    const uint32_t q = popc(mk & lanemask_lt());
+                    wave_lockstep();  // every lane has read its digit's count before the leaders advance it
+                    if (valid && q == 0) S.cnt[w][d] = pre + popc(mk);
+                    wave_lockstep();
+                    rank[j] = pre + q;
+                }
+                __syncthreads();
+                if (threadIdx.x < 256) {
+                    uint32_t run = S.dpre[threadIdx.x];
+#pragma unroll
+                    for (int i = 0; i < kBlockSortWaves; ++i) {
+                        const uint32_t u = S.cnt[i][threadIdx.x];
+                        S.cnt[i][threadIdx.x] = run;
+                        run += u;
+                    }
+                    S.dpre[threadIdx.x] = run;
+                }
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < kLongItems; ++j) {
+                    if ((w * kLongItems + j) * kWave + lane >= rem) continue;
+                    const uint32_t d = (uint32_t)(x[j] >> (8 * p)) & 255u;
+                    const uint32_t at = S.cnt[w][d] + rank[j];
+                    kd[at] = x[j];
+                    vd[at] = y[j];
+                }
+                __syncthreads();  // the counts are reused by the next tile
+            }
+            __threadfence();  // the next pass reads what other waves wrote
+            __syncthreads();
+            uint64_t *const kt = ks;
+            ks = kd;
+            kd = kt;
+            uint32_t *const vt = vs;
+            vs = vd;
+            vd = vt;
+        }
+        for (uint64_t i = threadIdx.x; i < len; i += kBlockSortThreads) {
+            out.key[s + i] = key;
+            out.spay[s + i] = join_sort_key_spay(ks[i]);
+            out.rpay[s + i] = (int32_t)vs[i];
+        }
+        __syncthreads();
+    }
 }
 
 // Segmented form: block b is global tile b of the segments (kSortTile rows per
@@ -901,7 +1086,7 @@ __global__ __launch_bounds__(kFixThreads) void k_fix_runs_seg(const uint64_t *__
     if (n > sg.cap) n = sg.cap;
     const size_t t0 = (size_t)(blockIdx.x - sg.tile0) * kFixTile;
     if (t0 >= n) return;  // whole block
-    fix_runs_tile(k + sg.base, v + sg.base, n, t0, outs[si], long_flag);
+    fix_runs_tile(k + sg.base, v + sg.base, n, t0, outs[si], LongRuns{long_flag});
 }
 
 int launch_fix_runs_segments(const uint64_t *keys, const uint32_t *vals, const RadixSeg *d_segs, int nseg,
@@ -934,19 +1119,26 @@ int sort_packed_join_rows(uint64_t *k64, uint32_t *v32, size_t m, void *rws, int
     uint64_t *kalt = nullptr;
     uint32_t *valt = nullptr;
     RowsBufs rb{};
-    radix_carve(m, true, cv, &kalt, &valt, &rb);
+    uint32_t *runs = nullptr;
+    radix_carve(m, true, cv, &kalt, &valt, &rb, &runs);
     const RadixSeg seg{0, m, nullptr, 0, radix_tiles(m)};
     bool in_alt = false;
     QO_TRY(launch_radix_rows(k64, v32, kalt, valt, seg, 32, hi_bit, rb, st, &in_alt, nullptr));
-    QO_TRY(launch_fill_u32(flag, 0, 1, st));
+    QO_TRY(launch_fill_u32(flag, 0, 2, st));
     const size_t blocks = (m + kFixTile - 1) / kFixTile;
-    k_fix_runs<<<(unsigned)blocks, kFixThreads, 0, st>>>(in_alt ? kalt : k64, in_alt ? valt : v32, m, out, flag);
+    const LongRuns lr{flag, flag + 1, runs, long_runs_cap(m)};
+    uint64_t *ks = in_alt ? kalt : k64, *kd = in_alt ? k64 : kalt;
+    uint32_t *vs = in_alt ? valt : v32, *vd = in_alt ? v32 : valt;
+    k_fix_runs<<<(unsigned)blocks, kFixThreads, 0, st>>>(ks, vs, m, out, lr);
+    QO_LAUNCHED();
+    k_fix_long<<<(unsigned)props().cu_count * 2, kBlockSortThreads, 0, st>>>(ks, vs, kd, vd, m, long_run_limit(m), out,
+                                                                           lr);
     QO_LAUNCHED();
     uint32_t long_run = 0;
     QO_HIP(hipMemcpyAsync(&long_run, flag, 4, hipMemcpyDeviceToHost, st));
     QO_HIP(hipStreamSynchronize(st));
     if (!long_run) return QO_OK;
-    // Some key has more than kFixRun rows: sort all rows on the full width
+    // Very long runs, or very many long ones: sort all rows on the full width
     // (the result does not depend on the rows' current order).
     if (in_alt) {
         QO_HIP(hipMemcpyAsync(k64, kalt, m * 8, hipMemcpyDeviceToDevice, st));

@@ -51,3 +51,22 @@ def test_group_finish_over_capacity(qo, orc, cap):
     k = orc.gen_uniform_u32(60000, 8, 0, 0, 50000).astype(np.int32)
     with pytest.raises(qo._lib.QoError):
         qo.operators.groupby_agg(k, k, cap)
+
+
+@pytest.mark.parametrize("m,hot", [(60000, 65), (60000, 6144), (60000, 6145), (200000, 17000), (200000, 40000),
+                                   (400000, 64)])
+def test_join_rows_long_runs(qo, orc, m, hot):
+    """Keys of more than 64 rows: sorted in LDS (to 6144 rows), by passes of one work-group, or, past its limit, on
+    the full width; many long runs and several hot keys; constant and negative s_payloads."""
+    rng = np.random.default_rng(m + hot)
+    k = rng.integers(-m, m, m).astype(np.int32)
+    k[:hot] = 12
+    k[hot:hot + 300] = -7
+    if hot == 64:
+        k = rng.integers(0, m // 75, m).astype(np.int32)   # most keys past 64 rows: more runs than the list holds
+    k = rng.permutation(k)
+    sp = rng.integers(-(1 << 31), (1 << 31) - 1, m, dtype=np.int64).astype(np.int32)
+    sp[k == -7] = 5
+    rp = k * np.int32(3) + np.int32(1)
+    for g, e in zip(qo.operators.sort_join_rows(k, rp, sp), orc.sort_join_rows(k, rp, sp)):
+        assert np.array_equal(g, e)
