@@ -459,15 +459,26 @@ int qo_hj_filter_sort(void *table, size_t table_bytes, const int32_t *rkey, cons
     QO_ENTER();
     QO_REQUIRE(table && h_count, "null pointer");
     hipStream_t st = stream_of(s);
+    int status = QO_OK;
+    void *ws = workspace(st, join_build_ws_bytes(table_bytes, nr), &status);
+    if (!ws) return status;
+    QO_TRY(launch_join_build(table, table_bytes, rkey, rpay, nr, ws, st));
+    bool done = false;
+    QO_TRY(sorted_join_try(table, table_bytes, rkey, rpay, nr, skey, spay, sfilt, ns, flo, fhi, okey, orpay, ospay,
+                           out_capacity, h_count, st, &done));
+    if (done) {
+        if (*h_count > out_capacity) return set_error(QO_ERR_CAPACITY, "join produced %llu rows, capacity %zu",
+                                                      (unsigned long long)*h_count, out_capacity);
+        return QO_OK;
+    }
     // The probe writes sort-ready rows (join_sort_key(key, s_payload), r_payload)
     // that the sort orders in place and unpacks into the output columns, so no
-    // separate pack pass runs.  Build buckets, probe buckets and the sort's
-    // workspace share one region in stream order.
-    const size_t stage_bytes = std::max({join_build_ws_bytes(table_bytes, nr), join_probe_ws_bytes(table_bytes, ns),
-                                         radix_workspace_bytes(out_capacity, true)});
+    // separate pack pass runs.  Probe buckets and the sort's workspace share one
+    // region in stream order.
+    const size_t stage_bytes = std::max(join_probe_ws_bytes(table_bytes, ns),
+                                        radix_workspace_bytes(out_capacity, true));
     const size_t rows = out_capacity ? out_capacity : 1;
-    int status = QO_OK;
-    void *ws = workspace(st, stage_bytes + rows * 12 + 2048, &status);
+    ws = workspace(st, stage_bytes + rows * 12 + 2048, &status);
     if (!ws) return status;
     Carver cv(ws);
     uint64_t *d_count = cv.take<uint64_t>(1);
@@ -475,7 +486,6 @@ int qo_hj_filter_sort(void *table, size_t table_bytes, const int32_t *rkey, cons
     uint64_t *k64 = cv.take<uint64_t>(rows);
     uint32_t *v32 = cv.take<uint32_t>(rows);
     void *sws = cv.take<char>(stage_bytes);
-    QO_TRY(launch_join_build(table, table_bytes, rkey, rpay, nr, sws, st));
     JoinOut out;
     out.cap = out_capacity;
     out.k64 = k64;

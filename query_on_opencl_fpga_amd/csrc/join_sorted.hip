@@ -1,0 +1,755 @@
+// Sorted filtered join by key order (qo_hj_filter_sort, unique build keys).
+//
+// The generic path probes in arrival order and then sorts the joined rows with
+// radix passes, each of which reads and writes all of them.  Here S is split by
+// key value instead of by hash: bucket f holds the S tuples (and the build
+// tuples) with key - kmin in [f << sh, (f + 1) << sh), small enough that one
+// work-group joins it in LDS and writes its rows in their final order, so the
+// rows move twice (one split, or two) before they are written once.
+//
+//  * k_sj_sample: 16384 S tuples give the host the expected number of rows, how
+//    evenly their keys spread over the build range, the hottest key and whether
+//    every tuple finds a match.
+//  * k_sj_split1 / k_sj_split2: S (filter fused; keys outside the build range
+//    dropped) into up to 256 buckets, each again into up to 256.
+//  * k_sj_finish: per bucket, looks every tuple up, counts the matches per
+//    (build key, s_payload interval) in LDS, scans the counts, places the rows
+//    and ranks each in its bin's run.
+// A key-range table (dense keys) serves the lookup directly: the bucket's slots
+// are a contiguous table slice and the slot is the key's rank.  For other keys
+// the build tuples are split the same way and ordered in LDS by bins of the
+// bucket's key interval.  A bucket that overflows (skew that the sample did not
+// show) sets a flag; nothing is written then and the generic path runs.
+//
+// Whole calls, generic path -> this one: 2^28 S rows, half selected, 2^24 dense
+// build keys 5.64 -> 2.40 ms (split 0.96, second split 0.55, finish 0.64, build
+// 0.2); 12,000,008 S rows, half selected, 1,500,001 spread 31-bit keys 684 ->
+// 352 us; 16384 S rows, half selected, 4096 spread keys 204 -> 125 us.
+#include <algorithm>
+#include <cmath>
+
+#include "qo_internal.hpp"
+#include "qo_join.hpp"
+#include "qo_split.hpp"
+
+namespace qo {
+
+// Offset of a key in the build keys' span (monotone in the signed key).
+struct KeySpan {
+    uint32_t kmin, last;  // smallest build key, largest - smallest
+    QO_DEV bool operator()(int32_t key, uint32_t &d) const {
+        d = (uint32_t)key - kmin;
+        return d <= last;
+    }
+};
+
+struct FlagOverflow {
+    uint32_t *flag;
+    QO_DEV void operator()(uint64_t) const { *flag = 1u; }  // kSjOverflow
+};
+
+constexpr uint32_t kSjSamples = 16384;
+constexpr uint32_t kSjBins = 256;
+constexpr int kSjHotBits = 16;
+
+// What the host plans from: the table's state and the sample's counts.
+struct SjInfo {
+    uint32_t mode, dups;   // dups: repeated keys or (-1, -1) build tuples
+    int32_t rmin, rmax;
+    uint32_t pass, match;  // sampled tuples that pass the filter inside the build range; those with a match
+    uint32_t hot, pad;     // most samples with one key (to the collisions of kSjHotBits hash bits)
+    uint32_t pmin, pmax;   // ~smallest and largest sampled s_payload, both as value ^ 2^31
+    uint32_t bin[kSjBins];
+};
+
+QO_DEV int span_bin_shift(uint32_t last) { return last < kSjBins ? 0 : 24 - __clz((int)last); }
+
+// Thread i samples tuple i of an even grid over S, jittered inside its cell.
+// `keys` counts the samples by key hash (zeroed, like *info, beforehand).
+constexpr int kSjSampleThreads = 1024;  // few blocks: their counts meet in same-address atomics
+template <bool HAS_FILTER>
+__global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader *__restrict__ hdr, const int32_t *__restrict__ skey,
+                                                   const int32_t *__restrict__ spay,
+                                                   const int32_t *__restrict__ sfilt, size_t ns, int32_t flo,
+                                                   int32_t fhi, SjInfo *info, uint32_t *keys) {
+    __shared__ uint32_t s_bin[kSjBins];
+    __shared__ uint32_t s_pass, s_match, s_hot, s_pmin, s_pmax;
+    if (threadIdx.x < kSjBins) s_bin[threadIdx.x] = 0;
+    if (threadIdx.x == 0) s_pass = s_match = s_hot = s_pmin = s_pmax = 0;
+    const uint32_t i = blockIdx.x * kSjSampleThreads + threadIdx.x;
+    const uint64_t cell = ns >= kSjSamples ? ns / kSjSamples : 1;
+    const uint64_t at = ns >= kSjSamples ? (uint64_t)i * cell + hash32(i) % cell : i;
+    const uint32_t last = (uint32_t)hdr->rmax - (uint32_t)hdr->rmin;
+    const KeySpan span{(uint32_t)hdr->rmin, last};
+    bool in = at < ns;
+    const int32_t key = in ? skey[at] : 0;
+    const int32_t filt = HAS_FILTER && in ? sfilt[at] : 0;
+    const uint32_t pay = in ? (uint32_t)spay[at] ^ 0x80000000u : 0u;
+    uint32_t d = 0;
+    in = in && span(key, d) && (!HAS_FILTER || (filt >= flo && filt <= fhi));
+    __syncthreads();
+    uint32_t hot = 0;
+    bool match = false;
+    if (in) {
+        atomicAdd(&s_bin[(d >> span_bin_shift(last)) & (kSjBins - 1)], 1u);
+        hot = 1 + atomicAdd(&keys[hash32((uint32_t)key) >> (32 - kSjHotBits)], 1u);
+        // A repeated build key makes chains long, and the join generic: no walk then.
+        if (hdr->has_dups == 0)
+            match = join_count(reinterpret_cast<const uint64_t *>(hdr + 1), hdr->cap, JoinHash::of(hdr), 0, key) != 0;
+    }
+    const uint64_t m = ballot(in), mm = ballot(match);
+    hot = wave_max(hot);
+    const uint32_t pmin = wave_max(in ? ~pay : 0u), pmax = wave_max(in ? pay : 0u);
+    if (lane_id() == 0 && m) {
+        atomicAdd(&s_pass, popc(m));
+        atomicAdd(&s_match, popc(mm));
+        atomicMax(&s_hot, hot);
+        atomicMax(&s_pmin, pmin);
+        atomicMax(&s_pmax, pmax);
+    }
+    __syncthreads();
+    if (threadIdx.x < kSjBins && s_bin[threadIdx.x]) atomicAdd(&info->bin[threadIdx.x], s_bin[threadIdx.x]);
+    if (threadIdx.x == 0 && s_pass) {
+        atomicAdd(&info->pass, s_pass);
+        atomicAdd(&info->match, s_match);
+        atomicMax(&info->hot, s_hot);
+        atomicMax(&info->pmin, s_pmin);
+        atomicMax(&info->pmax, s_pmax);
+    }
+    if (i == 0) {
+        info->mode = hdr->mode;
+        info->dups = hdr->has_dups | hdr->sentinel_count | hdr->overflow;
+        info->rmin = hdr->rmin;
+        info->rmax = hdr->rmax;
+    }
+}
+
+constexpr int kSjPartBits = 8;
+using SjSplitLds = SplitLdsT<1u << kSjPartBits>;
+
+// Columns -> `parts` buckets of (key - kmin) >> shift.
+template <bool HAS_FILTER, class Layout>
+__global__ __launch_bounds__(kSplitThreads) void k_sj_split1(const int32_t *__restrict__ kcol,
+                                                             const int32_t *__restrict__ pcol,
+                                                             const int32_t *__restrict__ fcol, size_t n, int32_t flo,
+                                                             int32_t fhi, bool vec, KeySpan span, int shift,
+                                                             uint32_t parts, uint64_t *__restrict__ bucket, Layout out,
+                                                             uint32_t *ctr, FlagOverflow overflow) {
+    __shared__ SjSplitLds sh;
+    int32_t key[kSplitJ][4], pay[kSplitJ][4];
+    uint32_t pass[kSplitJ];
+    load_s_tile<kSplitJ, HAS_FILTER, kSplitThreads>(kcol, pcol, fcol, n, flo, fhi, vec, blockIdx.x, key, pay, pass);
+#pragma unroll
+    for (int j = 0; j < kSplitJ; ++j)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            uint32_t d;
+            if (!span(key[j][k], d)) pass[j] &= ~(1u << k);
+        }
+    split_block<kSplitJ>(key, pay, pass, span, shift, parts, 0, bucket, out, ctr, sh, overflow);
+}
+
+// Bucket b of the first split (its XCD regions) -> fine buckets (b << b2) +
+// part.  Block order as in the L2 probe: work-group i runs on XCD i % 8, which
+// walks its own buckets one after another, so that one L2 completes the lines
+// of a fine bucket's runs.
+__global__ __launch_bounds__(kSplitThreads) void k_sj_split2(const uint64_t *__restrict__ in, uint64_t incap,
+                                                             const uint32_t *inctr, uint32_t nb1, uint32_t tpr,
+                                                             KeySpan span, int shift, int b2,
+                                                             uint64_t *__restrict__ bucket, FixedLayout out,
+                                                             uint32_t *ctr, FlagOverflow overflow) {
+    __shared__ SjSplitLds sh;
+    const uint32_t x = blockIdx.x & 7u, q = blockIdx.x >> 3;
+    const uint32_t per = kXcdRegions * tpr;
+    const uint32_t b = (q / per) * 8u + x, rem = q % per;
+    if (b >= nb1) return;
+    const uint32_t reg = b * kXcdRegions + rem / tpr;
+    uint64_t n = inctr[reg * kCtrStride];
+    if (n > incap) n = incap;
+    const uint64_t e0 = (uint64_t)(rem % tpr) * kSplitTile;
+    if (e0 >= n) return;  // whole block: no barrier has been reached
+    const uint32_t m = (uint32_t)(n - e0 < kSplitTile ? n - e0 : kSplitTile);
+    int32_t key[kSplitJ][4], pay[kSplitJ][4];
+    uint32_t pass[kSplitJ];
+    load_pairs<kSplitJ, kSplitThreads>(in + (size_t)reg * incap + e0, m, key, pay, pass);
+    split_block<kSplitJ>(key, pay, pass, span, shift, 1u << b2, b << b2, bucket, out, ctr, sh, overflow);
+}
+
+constexpr uint32_t kSjRankRun = 256;  // longest run whose rows are ranked one against another
+constexpr int kSjItems = 6;           // S tuples per thread
+
+// Interval of the s_payload's range, by which a build key's matches are
+// counted: 2^sb intervals of [pmin, pmin + 2^bits), monotone in the s_payload
+// (values outside the sampled range fall into the first or last one).
+struct PayloadBins {
+    uint32_t pmin;  // value ^ 2^31
+    int bits;
+    QO_DEV uint32_t operator()(uint32_t pay, int sb) const {
+        const uint32_t x = pay ^ 0x80000000u;
+        const uint32_t t = x < pmin ? 0u : (x - pmin) >> (bits > sb ? bits - sb : 0);
+        return min(t, (1u << sb) - 1u);
+    }
+};
+
+// A bucket's work-group has NT threads: at most kRows S tuples and kSlots
+// build keys (dense: key slots), two per thread.  Rows are counted in kBins
+// (build key, s_payload interval) bins, so that a run left to be ranked is a row
+// or two long.  32 waves fill a CU: two work-groups of 1024 or four of 512, each
+// 1024 threads with at most 80 KB of LDS.
+template <bool DENSE, int NT>
+struct SjLds {
+    static constexpr int kItems = kSjItems;
+    static constexpr uint32_t kRows = (uint32_t)kItems * NT;
+    static constexpr uint32_t kSlots = 2 * NT;
+    static constexpr int kBinBits = __builtin_ctz(kSlots);  // bins of a sparse bucket's key interval
+    static constexpr int kPer = DENSE ? 8 : 4;
+    static constexpr uint32_t kBins = (uint32_t)kPer * NT;
+    uint32_t cnt[kBins + 1];  // matches per bin, then where its run starts
+    uint32_t pay[kSlots];
+    int32_t spay[kRows];
+    uint16_t slot[kRows];  // build key << sb | s_payload interval
+    uint64_t bits[DENSE ? kSlots / 64 : 1];       // dense: slots that hold a key
+    uint32_t off[DENSE ? 1 : kSlots];             // sparse: key offsets of the build tuples, ascending
+    uint32_t bin[DENSE ? 1 : kSlots + 1];         // sparse: where each bin's build tuples start
+    uint32_t w[NT / kWave];
+    uint64_t base;
+    uint32_t tile, long_run;
+};
+
+struct SjBuckets {
+    const uint64_t *bucket;
+    uint64_t cap;
+    const uint32_t *ctr;
+    QO_DEV uint32_t count(uint32_t f) const {
+        const uint64_t c = ctr[(size_t)f * kCtrStride];
+        return (uint32_t)(c < cap ? c : cap);
+    }
+};
+
+// Rows of the bucket (s.spay, s.slot; total of them) into (slot, s_payload)
+// order by digit passes in place: every row is in registers before any is
+// written back.  For buckets with a run too long to rank row against row; the
+// run starts in s.cnt give way to the waves' digit counts.
+template <bool DENSE, int NT>
+QO_DEV void sj_sort_rows(SjLds<DENSE, NT> &s, uint32_t total, int sb) {
+    constexpr int IT = kSjItems;
+    constexpr int kWaves = NT / kWave;
+    static_assert(kWaves * 256 * sizeof(uint16_t) <= sizeof(s.cnt), "digit counts");
+    uint16_t(*cnt)[256] = reinterpret_cast<uint16_t(*)[256]>(s.cnt);
+    const unsigned w = wave_id(), lane = lane_id();
+    for (int pass = 0; pass < 6; ++pass) {  // 4 digits of the s_payload, 2 of the slot (11 bits)
+        __syncthreads();
+        for (int i = 0; i < 256 / kWave; ++i) cnt[w][i * kWave + lane] = 0;
+        uint32_t x[IT], at[IT];  // at: order within the wave's digit | slot << 13 | digit << 24
+        static_assert(SjLds<DENSE, NT>::kRows <= 1u << 13 && 2 * NT <= 1 << 11, "fields of at");
+        wave_lockstep();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            const uint32_t i = (w * IT + j) * kWave + lane;
+            const bool valid = i < total;
+            x[j] = valid ? (uint32_t)s.spay[i] : 0u;
+            const uint32_t l = valid ? (uint32_t)s.slot[i] >> sb : 0u;
+            const uint32_t d = (pass < 4 ? (x[j] ^ 0x80000000u) >> (8 * pass) : l >> (8 * (pass - 4))) & 255u;
+            const uint64_t m = match_digit(d, valid);
+            const uint32_t pre = cnt[w][d], r = popc(m & lanemask_lt());
+            wave_lockstep();  // every lane has read its digit's count before the leaders advance it
+            if (valid && r == 0) cnt[w][d] = (uint16_t)(pre + popc(m));
+            wave_lockstep();
+            at[j] = (pre + r) | (l << 13) | (d << 24);
+        }
+        __syncthreads();
+        uint32_t tot = 0;
+        if (threadIdx.x < 256) {
+#pragma unroll
+            for (int i = 0; i < kWaves; ++i) {
+                const uint32_t c = cnt[i][threadIdx.x];
+                cnt[i][threadIdx.x] = (uint16_t)tot;
+                tot += c;
+            }
+        }
+        const uint32_t start = block_excl_scan<kWaves>(tot, s.w);
+        if (threadIdx.x < 256)
+#pragma unroll
+            for (int i = 0; i < kWaves; ++i) cnt[i][threadIdx.x] = (uint16_t)(cnt[i][threadIdx.x] + start);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            if ((w * IT + j) * kWave + lane >= total) continue;
+            const uint32_t p = cnt[w][at[j] >> 24] + (at[j] & 0x1FFFu);
+            s.spay[p] = (int32_t)x[j];
+            s.slot[p] = (uint16_t)(((at[j] >> 13) & 0x7FFu) << sb);
+        }
+    }
+}
+
+// Exclusive scan of c[0, PER * NT) in place, PER entries per thread;
+// c[PER * NT] := the total, which is returned.  Barriers before and after.
+template <int NT, int PER>
+QO_DEV uint32_t sj_scan(uint32_t *c, uint32_t *s_w) {
+    __syncthreads();
+    uint32_t v[PER], sum = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        v[u] = c[PER * threadIdx.x + u];
+        sum += v[u];
+    }
+    uint32_t at = block_excl_scan<NT / kWave>(sum, s_w);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        c[PER * threadIdx.x + u] = at;
+        at += v[u];
+    }
+    if (threadIdx.x == NT - 1) c[PER * NT] = at;
+    __syncthreads();
+    return c[PER * NT];
+}
+
+// off[f]: where the rows of bucket f start when every S tuple of a bucket has
+// a match (off[nb]: their number, also in *d_count).  Block b scans the 2^b2
+// buckets of first-split bucket b behind the totals of the first-split buckets
+// before it (A: nsub regions each).
+__global__ __launch_bounds__(256) void k_sj_offsets(SjBuckets A, uint32_t nsub, SjBuckets S, uint32_t nb, int b2,
+                                                    uint32_t *__restrict__ off, uint64_t *d_count) {
+    __shared__ uint32_t s_w[4];
+    __shared__ uint32_t s_before;
+    if (threadIdx.x == 0) s_before = 0;
+    __syncthreads();
+    uint32_t before = 0;
+    if (threadIdx.x < blockIdx.x)  // at most 256 first-split buckets
+        for (uint32_t r = 0; r < nsub; ++r) before += A.count(threadIdx.x * nsub + r);
+    before = wave_sum(before);
+    if (lane_id() == 0 && before) atomicAdd(&s_before, before);
+    const uint32_t per = b2 ? 1u << b2 : nb, f0 = blockIdx.x * per;  // per <= 256
+    const uint32_t f = f0 + threadIdx.x;
+    const uint32_t c = threadIdx.x < per && f < nb ? S.count(f) : 0u;
+    const uint32_t ex = block_excl_scan256(c, s_w);
+    __syncthreads();
+    if (threadIdx.x < per && f < nb) {
+        off[f] = s_before + ex;
+        if (f == nb - 1) {
+            off[nb] = s_before + ex + c;
+            *d_count = s_before + ex + c;
+        }
+    }
+}
+
+// ALL: the bucket's rows start at off[f] (every tuple is expected to match; one
+// that does not sets kSjMiss in *flag, and the launch without ALL is needed).
+// Otherwise the buckets are taken by ticket and a look-back gives the start.
+//
+// Bound by vector instructions and by the latency between its barriers, then by
+// HBM (2^28 rows: 2.8 GB in 0.64 ms).  What was measured at that size: rows
+// ranked within whole key runs (mean 8 rows, but a wave waits for its longest)
+// 0.84 ms, 185 vector instructions per row; within (key, s_payload interval)
+// bins 0.64 ms.  Work-groups of 1024 threads with ticket and look-back 1.04 ms.
+constexpr uint32_t kSjOverflow = 1u, kSjMiss = 2u;
+template <bool DENSE, int NT, bool ALL>
+__global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, uint32_t nb, int sh,
+                                                             KeySpan span, PayloadBins pbins,
+                                                             const uint64_t *__restrict__ slots, SoaEmit emit, uint32_t *flag, const uint32_t *__restrict__ off,
+                                                             uint64_t *status, uint32_t *ticket, uint64_t *d_count,
+                                                             DevCtl *ctl) {
+    using Lds = SjLds<DENSE, NT>;
+    constexpr int IT = Lds::kItems;
+    __shared__ Lds s;
+    // In the ALL form the flag and the bucket's place are three scalar loads in
+    // flight together, and the tuples' loads wait for them only.
+    const uint32_t fl = *flag;
+    const uint32_t o0 = ALL ? off[blockIdx.x] : 0u, o1 = ALL ? off[blockIdx.x + 1] : 0u;
+    if (fl & kSjOverflow) return;  // the generic path runs
+    if (threadIdx.x == 0) {
+        if (!ALL) s.tile = atomicAdd(ticket, 1u);
+        s.long_run = 0;
+    }
+#pragma unroll
+    for (int u = 0; u < Lds::kPer; ++u) s.cnt[threadIdx.x + u * NT] = 0;
+    if (!DENSE) {
+        s.bin[threadIdx.x] = 0;
+        s.bin[threadIdx.x + NT] = 0;
+    }
+    __syncthreads();
+    const uint32_t f = ALL ? blockIdx.x : s.tile;
+    if (f >= nb) return;  // whole block; one block per bucket, so never taken
+    const uint32_t n = ALL ? o1 - o0 : S.count(f);
+    const uint32_t base_d = f << sh;  // offset of the bucket's first key
+    const uint64_t *src = S.bucket + (size_t)f * S.cap;
+    uint64_t v[IT];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        const uint32_t i = (uint32_t)j * NT + threadIdx.x;
+        v[j] = i < n ? ld_stream(src + i) : 0ull;
+    }
+    int sb;  // log2 of the s_payload intervals per build key
+    if (DENSE) {
+        sb = __builtin_ctz(Lds::kBins) - sh;
+        const uint32_t nslots = 1u << sh;  // <= kSlots; a slice lies inside the table (2^p slots, sh <= p)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t i = (uint32_t)u * NT + threadIdx.x;
+            const uint64_t w = i < nslots ? ld_stream(slots + base_d + i) : kEmptySlot;
+            s.pay[i] = (uint32_t)(w >> 32);
+            const uint64_t m = ballot(w != kEmptySlot);
+            if (lane_id() == 0) s.bits[i / kWave] = m;
+        }
+        __syncthreads();
+    } else {
+        // Build tuples of the bucket, ordered by key: counted by bin, placed bin
+        // by bin, then ranked among their bin's.
+        const uint32_t nr = R.count(f);
+        sb = 31 - __clz((int)(Lds::kBins / (nr ? nr : 1u)));
+        const uint64_t *rsrc = R.bucket + (size_t)f * R.cap;
+        const int bsh = sh > Lds::kBinBits ? sh - Lds::kBinBits : 0;
+        uint32_t d[2], p[2], at[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const uint32_t i = (uint32_t)u * NT + threadIdx.x;
+            const uint64_t w = i < nr ? ld_stream(rsrc + i) : 0ull;
+            d[u] = (uint32_t)w - span.kmin - base_d;
+            p[u] = (uint32_t)(w >> 32);
+            at[u] = i < nr ? atomicAdd(&s.bin[d[u] >> bsh], 1u) : 0u;
+        }
+        sj_scan<NT, 2>(s.bin, s.w);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            if ((uint32_t)u * NT + threadIdx.x < nr) s.off[s.bin[d[u] >> bsh] + at[u]] = d[u];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if ((uint32_t)u * NT + threadIdx.x >= nr) continue;
+            const uint32_t b0 = s.bin[d[u] >> bsh], b1 = s.bin[(d[u] >> bsh) + 1];
+            uint32_t before = 0;
+            for (uint32_t i = b0; i < b1; ++i) before += s.off[i] < d[u];
+            at[u] = b0 + before;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if ((uint32_t)u * NT + threadIdx.x >= nr) continue;
+            s.off[at[u]] = d[u];
+            s.pay[at[u]] = p[u];
+        }
+        __syncthreads();
+    }
+    // Lookup: rank of the tuple's build key in the bucket, and its arrival order
+    // among that key's matches: slot | order << 16, or kMiss.
+    constexpr uint32_t kMiss = ~0u;
+    uint32_t pk[IT];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        pk[j] = kMiss;
+        if ((uint32_t)j * NT + threadIdx.x >= n) continue;
+        const uint32_t d = (uint32_t)v[j] - span.kmin - base_d;
+        uint32_t l = kMiss;
+        if (DENSE) {
+            if ((s.bits[d / kWave] >> (d % kWave)) & 1u) l = d;
+        } else {
+            const int bsh = sh > Lds::kBinBits ? sh - Lds::kBinBits : 0;
+            const uint32_t b1 = s.bin[(d >> bsh) + 1];
+            for (uint32_t i = s.bin[d >> bsh]; i < b1; ++i)
+                if (s.off[i] == d) l = i;
+        }
+        if (l != kMiss) {
+            const uint32_t bin = (l << sb) | pbins((uint32_t)(v[j] >> 32), sb);
+            const uint32_t order = atomicAdd(&s.cnt[bin], 1u);
+            pk[j] = bin | (order << 16);
+            if (order >= kSjRankRun) s.long_run = 1u;
+        }
+    }
+    const uint32_t total = sj_scan<NT, Lds::kPer>(s.cnt, s.w);
+    if (ALL) {
+        if (total != n) {  // block-uniform
+            if (threadIdx.x == 0) atomicOr(flag, kSjMiss);
+            return;
+        }
+    } else if (threadIdx.x == 0 && f > 0) {
+        st_agent(&status[f], kFlagAgg | total);  // successors need not wait for the placement
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+        if (pk[j] == kMiss) continue;
+        const uint32_t l = pk[j] & 0xFFFFu, p = s.cnt[l] + (pk[j] >> 16);
+        s.spay[p] = (int32_t)(v[j] >> 32);
+        s.slot[p] = (uint16_t)l;
+    }
+    __syncthreads();
+    if (s.long_run) {  // block-uniform
+        sj_sort_rows<DENSE, NT>(s, total, sb);
+    } else {
+        // Position i of the rows in bin order: its rank in its bin's run by
+        // s_payload, four rows of the run per step (reads past the run's end stay
+        // inside the struct).
+        uint32_t dst[IT];  // final position | slot << 16
+        int32_t x[IT];
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            const uint32_t i = (uint32_t)j * NT + threadIdx.x;
+            dst[j] = 0;
+            if (i >= total) continue;
+            const uint32_t l = s.slot[i];
+            x[j] = s.spay[i];
+            const uint32_t b0 = s.cnt[l], b1 = s.cnt[l + 1];
+            uint32_t before = 0;
+            for (uint32_t q = b0; q < b1; q += 4) {
+                const int32_t y0 = s.spay[q], y1 = s.spay[q + 1], y2 = s.spay[q + 2], y3 = s.spay[q + 3];
+                before += (y0 < x[j] || (y0 == x[j] && q < i)) ? 1u : 0u;
+                before += (q + 1 < b1 && (y1 < x[j] || (y1 == x[j] && q + 1 < i))) ? 1u : 0u;
+                before += (q + 2 < b1 && (y2 < x[j] || (y2 == x[j] && q + 2 < i))) ? 1u : 0u;
+                before += (q + 3 < b1 && (y3 < x[j] || (y3 == x[j] && q + 3 < i))) ? 1u : 0u;
+            }
+            dst[j] = (b0 + before) | (l << 16);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+            if ((uint32_t)j * NT + threadIdx.x >= total) continue;
+            s.spay[dst[j] & 0xFFFFu] = x[j];
+            s.slot[dst[j] & 0xFFFFu] = (uint16_t)(dst[j] >> 16);
+        }
+    }
+    if (!ALL && threadIdx.x < kWave) {
+        const uint64_t e = lookback(status, f, total, ctl);
+        if (threadIdx.x == 0) s.base = e;
+    }
+    __syncthreads();
+    const uint64_t base = ALL ? o0 : s.base;
+    const uint32_t kbase = span.kmin + base_d;
+    emit.template flush_rows<NT>(base, total, [&](uint32_t i, int32_t &k, int32_t &r, int32_t &p) {
+        const uint32_t l = (uint32_t)s.slot[i] >> sb;
+        k = (int32_t)(kbase + (DENSE ? l : s.off[DENSE ? 0 : l]));
+        r = (int32_t)s.pay[l];
+        p = s.spay[i];
+    });
+    if (!ALL && f == nb - 1 && threadIdx.x == 0) *d_count = base + total;
+}
+
+// ---------------------------------------------------------------------------
+// Host plan.
+// ---------------------------------------------------------------------------
+struct SjSide {            // one input's buckets
+    uint64_t capA = 0;     // pairs per region of the first split (two splits only)
+    uint64_t capB = 0;     // pairs per fine bucket
+};
+struct SjPlan {
+    bool on = false, dense = false, all = false;
+    int nt = 0;            // threads of the finishing work-groups
+    KeySpan span{};
+    PayloadBins pay{};
+    int sh = 0, b2 = 0;    // bucket = offset >> sh; b2 > 0: two splits, first by offset >> (sh + b2)
+    uint32_t nb = 0, nb1 = 0, parts1 = 0;
+    SjSide s, r;
+};
+
+// Fewer S tuples than this are probed and sorted by the generic path, whose
+// small sort is one launch.
+constexpr size_t kSjMinRows = size_t(1) << 14;
+constexpr uint64_t kSjMaxBuckets = 1u << (2 * kSjPartBits);
+
+// A fine bucket has room for all the rows a work-group takes, whatever the
+// expected number: a hot key of some thousand rows still fits.
+static SjSide sj_side(const SjPlan &p, double rows, uint32_t limit) {
+    SjSide o;
+    o.capB = limit;
+    if (p.b2) {
+        const double span = (double)p.span.last + 1.0;
+        const double a = std::min(rows, rows * std::ldexp(1.0, p.sh + p.b2) / span) / kXcdRegions;
+        o.capA = ((uint64_t)(a * 1.25 + 8.0 * std::sqrt(a)) + kSplitTile + 31) / 32 * 32;
+    }
+    return o;
+}
+
+// Buckets for work-groups of nt threads: the widest whose rows (and build
+// keys) fit with room to spare beside a hot key's, and narrow enough to give a
+// small join a few work-groups per CU.
+static bool sj_buckets(SjPlan &p, int nt, double rows, double hot, size_t nr) {
+    const double limit = (double)kSjItems * nt, span = (double)p.span.last + 1.0;
+    const double room = 0.9 * limit - hot;
+    if (room < 0.1 * limit) return false;
+    const double want = std::min({0.75 * limit, room, std::max(512.0, rows / 512.0)});
+    p.nt = nt;
+    p.sh = 0;
+    while (p.sh < 31) {
+        const double w = std::ldexp(1.0, p.sh + 1);
+        if (rows * w / span > want || w / 2 >= span) break;  // 2^sh <= the smallest power of two >= span
+        if (p.dense ? w > 2.0 * nt : (double)nr * w / span > 1.5 * nt) break;
+        ++p.sh;
+    }
+    const uint64_t nb = ((uint64_t)p.span.last >> p.sh) + 1;
+    if (nb > kSjMaxBuckets || rows * std::ldexp(1.0, p.sh) / span > std::min(room, 0.8 * limit)) return false;
+    p.nb = (uint32_t)nb;
+    int bits = 0;
+    while ((1u << bits) < p.nb) ++bits;
+    p.b2 = bits <= kSjPartBits ? 0 : bits / 2;
+    p.nb1 = ((p.nb - 1) >> p.b2) + 1;
+    p.parts1 = 1;
+    while (p.parts1 < p.nb1) p.parts1 *= 2;
+    p.s = sj_side(p, rows, (uint32_t)limit);
+    if (!p.dense) p.r = sj_side(p, (double)nr, 2u * (uint32_t)nt);
+    return true;
+}
+
+static SjPlan sj_plan(const SjInfo &info, size_t nr, size_t ns) {
+    SjPlan p;
+    if (info.dups || info.rmin > info.rmax || info.pass == 0) return p;
+    const uint32_t last = (uint32_t)info.rmax - (uint32_t)info.rmin;
+    // Even spread: no bin of the sample far above the mean of the bins in use.
+    const int bsh = last < kSjBins ? 0 : 24 - __builtin_clz(last);
+    const double mean = (double)info.pass / ((last >> bsh) + 1);
+    const uint32_t top = *std::max_element(info.bin, info.bin + kSjBins);
+    if (top > 1.5 * mean + 6.0 * std::sqrt(mean) + 4.0) return p;
+    const double per = (double)ns / (double)std::min<size_t>(ns, kSjSamples);  // tuples a sample stands for
+    const double rows = std::min((double)ns, std::max(1.0, per * (info.pass + 4.0 * std::sqrt((double)info.pass))));
+    // A key seen up to 6 times in the sample may be chance (or a collision); the
+    // largest of many counts lies above its own mean.
+    const double hot = info.hot <= 6 ? 0.0 : per * (info.hot - std::sqrt((double)info.hot));
+    p.dense = info.mode == kJoinKeyRange;
+    p.all = info.match == info.pass;
+    p.span = KeySpan{(uint32_t)info.rmin, last};
+    p.pay = PayloadBins{~info.pmin, 32 - __builtin_clz((info.pmax - ~info.pmin) | 1u)};
+    p.on = sj_buckets(p, 512, rows, hot, nr) || sj_buckets(p, 1024, rows, hot, nr);
+    return p;
+}
+
+struct SjSideBufs {
+    uint32_t *ctrA = nullptr, *ctrB = nullptr;
+    uint64_t *a = nullptr, *b = nullptr;
+};
+struct SjBufs {
+    uint64_t *res = nullptr;  // [0] rows, [1] overflow flag
+    uint32_t *ticket = nullptr, *off = nullptr;
+    uint64_t *status = nullptr;
+    SjSideBufs s, r;
+    size_t clear_words = 0;   // from res on: zeroed before the splits
+};
+
+static SjBufs sj_carve(const SjPlan &p, Carver &cv) {
+    SjBufs b;
+    const size_t fine = (size_t)p.nb1 << p.b2;
+    b.res = cv.take<uint64_t>(2);
+    const size_t from = cv.off - 16;
+    b.ticket = cv.take<uint32_t>(1);
+    b.status = cv.take<uint64_t>(p.nb);
+    auto counters = [&](SjSideBufs &o) {
+        o.ctrB = cv.take<uint32_t>(fine * kCtrStride);
+        if (p.b2) o.ctrA = cv.take<uint32_t>((size_t)p.parts1 * kXcdRegions * kCtrStride);
+    };
+    counters(b.s);
+    if (!p.dense) counters(b.r);
+    b.clear_words = (cv.off - from) / 4;
+    b.off = cv.take<uint32_t>(p.nb + 1);
+    auto data = [&](SjSideBufs &o, const SjSide &side) {
+        if (p.b2) o.a = cv.take<uint64_t>((size_t)p.nb1 * kXcdRegions * side.capA);
+        o.b = cv.take<uint64_t>(fine * side.capB);
+    };
+    data(b.s, p.s);
+    if (!p.dense) data(b.r, p.r);
+    return b;
+}
+
+template <bool HAS_FILTER>
+static int sj_split(const SjPlan &p, const SjSide &side, const SjSideBufs &b, uint32_t *flag, const int32_t *key,
+                    const int32_t *pay, const int32_t *filt, size_t n, int32_t flo, int32_t fhi, hipStream_t st) {
+    const bool vec = (((uintptr_t)key | (uintptr_t)pay | (HAS_FILTER ? (uintptr_t)filt : 0)) & 15u) == 0;
+    const size_t tiles = (n + kSplitTile - 1) / kSplitTile;
+    QO_REQUIRE(tiles < 0x7FFFFFFFull, "join input too large");
+    const FlagOverflow ovf{flag};
+    if (!p.b2) {
+        k_sj_split1<HAS_FILTER><<<(unsigned)tiles, kSplitThreads, 0, st>>>(
+            key, pay, filt, n, flo, fhi, vec, p.span, p.sh, p.parts1, b.b, FixedLayout{side.capB}, b.ctrB, ovf);
+        QO_LAUNCHED();
+        return QO_OK;
+    }
+    k_sj_split1<HAS_FILTER><<<(unsigned)tiles, kSplitThreads, 0, st>>>(key, pay, filt, n, flo, fhi, vec, p.span,
+                                                                      p.sh + p.b2, p.parts1, b.a, XcdLayout{side.capA},
+                                                                      b.ctrA, ovf);
+    QO_LAUNCHED();
+    const uint32_t tpr = (uint32_t)((side.capA + kSplitTile - 1) / kSplitTile);
+    const uint64_t grid = (uint64_t)((p.nb1 + 7) / 8) * 8 * kXcdRegions * tpr;
+    QO_REQUIRE(grid < 0x7FFFFFFFull, "join input too large");
+    k_sj_split2<<<(unsigned)grid, kSplitThreads, 0, st>>>(b.a, side.capA, b.ctrA, p.nb1, tpr, p.span, p.sh, p.b2, b.b,
+                                                          FixedLayout{side.capB}, b.ctrB, ovf);
+    QO_LAUNCHED();
+    return QO_OK;
+}
+
+
+int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
+                    const int32_t *skey, const int32_t *spay, const int32_t *sfilt, size_t ns, int32_t flo,
+                    int32_t fhi, int32_t *okey, int32_t *orpay, int32_t *ospay, size_t out_capacity, uint64_t *rows,
+                    hipStream_t st, bool *done) {
+    *done = false;
+    if (nr == 0 || ns < kSjMinRows || ns >= 0xFFFFFFFFull || tune_get(TUNE_JOIN_PART, ns).param != PART_AUTO)
+        return QO_OK;
+    const JoinHeader *hdr = static_cast<const JoinHeader *>(table);
+    int status = QO_OK;
+    constexpr size_t kWords = sizeof(SjInfo) / 4 + (size_t(1) << kSjHotBits);
+    void *ws = workspace(st, kWords * 4 + 256, &status);
+    if (!ws) return status;
+    SjInfo *d_info = static_cast<SjInfo *>(ws);
+    uint32_t *d_keys = reinterpret_cast<uint32_t *>(d_info + 1);
+    SjInfo info;
+    QO_TRY(launch_fill_u32(d_info, 0, kWords, st));
+    if (sfilt)
+        k_sj_sample<true><<<kSjSamples / kSjSampleThreads, kSjSampleThreads, 0, st>>>(hdr, skey, spay, sfilt, ns, flo, fhi, d_info, d_keys);
+    else
+        k_sj_sample<false><<<kSjSamples / kSjSampleThreads, kSjSampleThreads, 0, st>>>(hdr, skey, spay, sfilt, ns, flo, fhi, d_info, d_keys);
+    QO_LAUNCHED();
+    QO_HIP(hipMemcpyAsync(&info, d_info, sizeof(info), hipMemcpyDeviceToHost, st));
+    QO_HIP(hipStreamSynchronize(st));
+    const SjPlan p = sj_plan(info, nr, ns);
+    if (!p.on) return QO_OK;
+    Carver size(nullptr);
+    sj_carve(p, size);
+    ws = workspace(st, size.off + 256, &status);
+    if (!ws) return status;
+    Carver cv(ws);
+    const SjBufs b = sj_carve(p, cv);
+    uint32_t *flag = reinterpret_cast<uint32_t *>(b.res + 1);
+    QO_TRY(launch_fill_u32(b.res, 0, b.clear_words, st));
+    if (sfilt) QO_TRY(sj_split<true>(p, p.s, b.s, flag, skey, spay, sfilt, ns, flo, fhi, st));
+    else QO_TRY(sj_split<false>(p, p.s, b.s, flag, skey, spay, nullptr, ns, 0, 0, st));
+    if (!p.dense) QO_TRY(sj_split<false>(p, p.r, b.r, flag, rkey, rpay, nullptr, nr, 0, 0, st));
+    const SoaEmit out{okey, orpay, ospay, out_capacity};
+    const SjBuckets sb{b.s.b, p.s.capB, b.s.ctrB}, rb{b.r.b, p.r.capB, b.r.ctrB};
+    const uint64_t *slots = reinterpret_cast<const uint64_t *>(hdr + 1);
+    uint64_t res[2];
+    for (bool all = p.all;; all = false) {
+        if (all) {
+            k_sj_offsets<<<p.b2 ? p.nb1 : 1u, 256, 0, st>>>(SjBuckets{nullptr, p.s.capA, b.s.ctrA}, kXcdRegions, sb,
+                                                            p.nb, p.b2, b.off, b.res);
+            QO_LAUNCHED();
+        }
+#define QO_SJ_FINISH(D, T, A)                                                                                       \
+    k_sj_finish<D, T, A><<<p.nb, T, 0, st>>>(sb, rb, p.nb, p.sh, p.span, p.pay, slots, out, flag, b.off, b.status, b.ticket, \
+                                             b.res, dev_ctl())
+        if (p.dense) {
+            if (p.nt == 512) {
+                if (all) QO_SJ_FINISH(true, 512, true);
+                else QO_SJ_FINISH(true, 512, false);
+            } else {
+                if (all) QO_SJ_FINISH(true, 1024, true);
+                else QO_SJ_FINISH(true, 1024, false);
+            }
+        } else {
+            if (p.nt == 512) {
+                if (all) QO_SJ_FINISH(false, 512, true);
+                else QO_SJ_FINISH(false, 512, false);
+            } else {
+                if (all) QO_SJ_FINISH(false, 1024, true);
+                else QO_SJ_FINISH(false, 1024, false);
+            }
+        }
+#undef QO_SJ_FINISH
+        QO_LAUNCHED();
+        QO_HIP(hipMemcpyAsync(res, b.res, sizeof(res), hipMemcpyDeviceToHost, st));
+        QO_HIP(hipStreamSynchronize(st));
+        const uint32_t f = (uint32_t)res[1];
+        if (f & kSjOverflow) return QO_OK;  // nothing was written
+        // An unmatched tuple: the rows start elsewhere, so they are all written again.
+        if (!(all && (f & kSjMiss))) break;
+    }
+    *rows = res[0];
+    *done = true;
+    return QO_OK;
+}
+
+}  // namespace qo

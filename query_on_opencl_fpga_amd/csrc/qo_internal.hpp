@@ -208,6 +208,17 @@ int launch_join_probe(const void *table, size_t table_bytes, const int32_t *skey
                       const int32_t *sfilt, size_t ns, int32_t flo, int32_t fhi, const JoinOut &out,
                       uint64_t *d_count, void *ws, hipStream_t st);
 
+// Sorted join against the table built from (rkey, rpay), by a split in key
+// order (join_sorted.hip).  *done = false when its conditions do not hold
+// (repeated build keys, few or unevenly spread S keys, a bucket that
+// overflowed): nothing was written and the probe and sort have to run.  Else
+// *rows is the match count and the first out_capacity rows are written.  Uses
+// the stream's workspace (slot 0) and synchronises the stream.
+int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
+                    const int32_t *skey, const int32_t *spay, const int32_t *sfilt, size_t ns, int32_t flo,
+                    int32_t fhi, int32_t *okey, int32_t *orpay, int32_t *ospay, size_t out_capacity, uint64_t *rows,
+                    hipStream_t st, bool *done);
+
 }  // namespace qo
 
 #define QO_HIP(call)                                                                                \

@@ -157,9 +157,9 @@ using SplitLds = SplitLdsT<kMaxSplit>;
 // marks element k of group j) into `parts` buckets by
 // part = (hs(key) >> shift) & (parts - 1); bucket index = bucket0 + part,
 // placed by `out` in `bucket`; ctr holds one fill cursor per bucket.
-template <int J, class Layout, class Overflow, class Lds>
+template <int J, class Hash, class Layout, class Overflow, class Lds>
 QO_DEV void split_block(const int32_t (&key)[J][4], const int32_t (&pay)[J][4], const uint32_t (&pass)[J],
-                        const JoinHash &hs, int shift, uint32_t parts, uint32_t bucket0,
+                        const Hash &hs, int shift, uint32_t parts, uint32_t bucket0,
                         uint64_t *__restrict__ bucket, const Layout &out, uint32_t *ctr, Lds &sh,
                         const Overflow &overflow) {
     const uint32_t mask = parts - 1;
