@@ -10,6 +10,9 @@
 // memory, per-query digit starts up front, then per pass a tile histogram, a
 // segmented column scan and the placement) orders every query's matches; its
 // last pass writes each query's output columns.
+// Small queries are joined before all that by the sorted join of
+// batch_sorted.hip; the stages above then run only on the queries it left, and
+// return at once when it left none.
 // The stage sequence (fills included, no memset nodes) is captured once into a
 // graph at creation and replayed by qo_batch_launch.
 //
@@ -41,9 +44,17 @@ QO_DEV int query_of(const BQuery *q, int nq, uint32_t t) {
     return lo;
 }
 
-__global__ void k_b_init(const BQuery *q, int nq) {
+// run_if (this kernel and the next ones): return at once unless *run_if != 0;
+// skip[q] != 0: query q is done.  Both may be null.
+__global__ void k_b_fill(uint64_t *dst, size_t n, const uint32_t *run_if) {
+    if (run_if && *run_if == 0) return;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = kEmptySlot;
+}
+
+__global__ void k_b_init(const BQuery *q, int nq, const uint32_t *run_if) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nq) return;
+    if (i >= nq || (run_if && *run_if == 0)) return;
     JoinHeader *h = q[i].hdr;
     h->cap = q[i].table_cap;
     h->has_dups = 0;
@@ -73,9 +84,11 @@ __global__ void k_b_init(const BQuery *q, int nq) {
 #define QO_TILE_LOOP_END }
 
 __global__ __launch_bounds__(256) void k_b_build(const BQuery *q, int nq, uint32_t total, uint32_t *ticket,
-                                                 uint32_t build_tile) {
+                                                 uint32_t build_tile, const uint32_t *run_if, const uint32_t *skip) {
+    if (run_if && *run_if == 0) return;
     QO_TILE_LOOP(ticket, total, t)
     const int qi = query_of<0>(q, nq, t);
+    if (skip && skip[qi]) continue;  // block-uniform
     const BQuery &Q = q[qi];
     const uint64_t r0 = (uint64_t)(t - Q.rtile0) * build_tile;
     const uint64_t r1 = r0 + build_tile < Q.nr ? r0 + build_tile : Q.nr;
@@ -90,7 +103,9 @@ __global__ __launch_bounds__(256) void k_b_build(const BQuery *q, int nq, uint32
 // VGPRs the kernel ran 2 and took 48.3 ms per 512-query batch, with the bound
 // (168 VGPRs, a few spilled) 39.7 ms.
 __global__ __launch_bounds__(256, 3) void k_b_probe(const BQuery *q, int nq, uint32_t total, uint32_t *ticket,
-                                                 uint64_t *mkeys, uint32_t *mvals, uint32_t group) {
+                                                 uint64_t *mkeys, uint32_t *mvals, uint32_t group,
+                                                 const uint32_t *run_if, const uint32_t *skip) {
+    if (run_if && *run_if == 0) return;
     __shared__ uint32_t s_tot[tile_offsets_words(kProbeJ, 4)];
     __shared__ uint64_t s_base;
     __shared__ JoinStage stage;
@@ -98,6 +113,7 @@ __global__ __launch_bounds__(256, 3) void k_b_probe(const BQuery *q, int nq, uin
     QO_TILE_LOOP(ticket, groups, tg)
     for (uint32_t t = tg * group; t < total && t < (tg + 1) * group; ++t) {
     const int qi = query_of<1>(q, nq, t);
+    if (skip && skip[qi]) continue;  // block-uniform
     const BQuery &Q = q[qi];
     const uint64_t *slots = reinterpret_cast<const uint64_t *>(Q.hdr + 1);
     // Sort-ready rows (join_sort_key, r_payload); every query's rows start at a
@@ -117,7 +133,7 @@ __global__ __launch_bounds__(256, 3) void k_b_probe(const BQuery *q, int nq, uin
 // ---------------------------------------------------------------------------
 // Plan of one join batch: sizes, then (after binding an arena) device pointers.
 // ---------------------------------------------------------------------------
-int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p) {
+int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p, bool sorted) {
     QO_REQUIRE(nq >= 1 && queries, "bad batch arguments");
     p.nq = nq;
     p.hq.assign(nq, BQuery{});
@@ -130,6 +146,7 @@ int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p) {
     p.pbuild_q.clear();
     p.part_ws_bytes = 0;
     uint64_t rt = 0, stt = 0, mt = 0;
+    std::vector<char> generic(nq, !sorted);
     // Launch parameters by the size class of the batch's mean build side.
     uint64_t rsum = 0;
     for (int i = 0; i < nq; ++i) rsum += queries[i].nr;
@@ -167,6 +184,7 @@ int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p) {
             p.pbuild_q.push_back(i);
             p.part_ws_bytes = std::max(p.part_ws_bytes, bws);
         }
+        if (partitioned || bws || tune_get(TUNE_JOIN_PART, (size_t)u.ns).param != PART_AUTO) generic[i] = 1;
         q.vec = ((uintptr_t)u.skey % 16 == 0 && (uintptr_t)u.spay % 16 == 0 &&
                  (!u.sfilt || (uintptr_t)u.sfilt % 16 == 0)) ? 1u : 0u;
         q.rtile0 = (uint32_t)rt;
@@ -191,6 +209,7 @@ int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p) {
     p.stt = (uint32_t)stt;
     p.mt = (uint32_t)mt;
     p.small_words = 64 + (size_t)nq * 2;
+    bj_plan_init(queries, nq, generic, p.sj);
     return QO_OK;
 }
 
@@ -208,6 +227,9 @@ static void plan_carve(JoinBatchPlan &p, Carver &cv) {
     p.d_outs = cv.take<RowOut>(p.nq);
     p.sort_ws = cv.take<char>(radix_rows_seg_bytes(p.mt, p.nq, (uint32_t)p.hchunks.size()));
     p.part_ws = p.part_ws_bytes ? cv.take<char>(p.part_ws_bytes) : nullptr;
+    p.counts = cv.take<unsigned long long>(p.nq);
+    p.long_list = p.sj.all_on ? cv.take<SegPos>(p.total_match / 64 + 1) : nullptr;
+    bj_plan_carve(p.sj, cv);
 }
 
 size_t join_plan_bytes(JoinBatchPlan &p) {
@@ -222,7 +244,7 @@ void join_plan_bind(JoinBatchPlan &p, void *arena) {
     // Tables the persistent build fills come first, those of partitioned builds after.
     uint64_t slot_off = 0, pslot_off = p.fill_slots;
     size_t pb = 0;
-    p.counts = reinterpret_cast<unsigned long long *>(p.small + 64);
+    p.gcounts = reinterpret_cast<unsigned long long *>(p.small + 64);
     for (int i = 0; i < p.nq; ++i) {
         BQuery &q = p.hq[i];
         const bool pbuild = pb < p.pbuild_q.size() && p.pbuild_q[pb] == i;
@@ -230,7 +252,7 @@ void join_plan_bind(JoinBatchPlan &p, void *arena) {
         uint64_t &off = pbuild ? pslot_off : slot_off;
         q.hdr = reinterpret_cast<JoinHeader *>(p.slots_all + off);
         off += 32 + q.table_cap;
-        q.count = p.counts + i;
+        q.count = p.gcounts + i;
         p.hs[i] = RadixSeg{q.m_base, q.out_cap, reinterpret_cast<const uint64_t *>(q.count), q.mtile0, q.nmtile};
     }
 }
@@ -244,18 +266,32 @@ int join_plan_upload(const JoinBatchPlan &p, hipStream_t st) {
     QO_HIP(hipMemcpyAsync(p.d_chunk0, p.hchunk0.data(), sizeof(uint32_t) * p.hchunk0.size(), hipMemcpyHostToDevice,
                           st));
     QO_HIP(hipMemcpyAsync(p.d_outs, p.houts.data(), sizeof(RowOut) * p.nq, hipMemcpyHostToDevice, st));
-    return QO_OK;
+    return bj_plan_upload(p.sj, st);
 }
 
 int join_plan_launch(const JoinBatchPlan &p, hipStream_t st) {
     const unsigned persist = (unsigned)props().cu_count * 8;
-    if (p.fill_slots) QO_TRY(launch_fill_u64(p.slots_all, kEmptySlot, p.fill_slots, st));
     QO_TRY(launch_fill_u32(p.small, 0, p.small_words, st));
-    k_b_init<<<(p.nq + 255) / 256, 256, 0, st>>>(p.d_q, p.nq);
+    // The sorted join of the small queries; the generic stages below run only if
+    // it left some, and only on those.
+    uint32_t *run_if = nullptr;
+    const uint32_t *skip = nullptr;
+    if (p.sj.any_on) {
+        run_if = p.small + 3;
+        skip = p.sj.skip;
+        QO_TRY(bj_plan_launch(p.sj, run_if, st));
+    }
+    if (p.fill_slots) {
+        k_b_fill<<<grid_for(p.fill_slots, 256, (unsigned)props().cu_count * 8), 256, 0, st>>>(p.slots_all, p.fill_slots,
+                                                                                            run_if);
+        QO_LAUNCHED();
+    }
+    k_b_init<<<(p.nq + 255) / 256, 256, 0, st>>>(p.d_q, p.nq, run_if);
     QO_LAUNCHED();
     uint32_t *tickets = p.small;
     if (p.rt) {
-        k_b_build<<<std::min<unsigned>(p.rt, persist), 256, 0, st>>>(p.d_q, p.nq, p.rt, tickets + 0, p.build_tile);
+        k_b_build<<<std::min<unsigned>(p.rt, persist), 256, 0, st>>>(p.d_q, p.nq, p.rt, tickets + 0, p.build_tile,
+                                                                     run_if, skip);
         QO_LAUNCHED();
     }
     for (int i : p.pbuild_q) {
@@ -267,7 +303,7 @@ int join_plan_launch(const JoinBatchPlan &p, hipStream_t st) {
     }
     if (p.stt) {
         k_b_probe<<<std::min<unsigned>(p.stt, persist), 256, 0, st>>>(p.d_q, p.nq, p.stt, tickets + 1, p.mkeys,
-                                                                      p.mvals, p.probe_group);
+                                                                      p.mvals, p.probe_group, run_if, skip);
         QO_LAUNCHED();
     }
     for (int i : p.part_q) {
@@ -285,22 +321,27 @@ int join_plan_launch(const JoinBatchPlan &p, hipStream_t st) {
     if (p.mt) {
         // Radix passes over the key bits only, then one pass that orders every
         // run of equal key by s_payload and writes the query's output columns.
-        // Should some key have more than 64 rows, the full-width sort (its
-        // kernels gated on that flag, so they return at once otherwise)
-        // rewrites the outputs.
-        uint32_t *long_flag = p.small + 2;
+        // Runs of more than 64 rows: with the sorted join able to take every
+        // query (so that each has at most a million rows and few come here), a
+        // work-group per run.  Otherwise the full-width sort, whose 42 launches
+        // are gated on a flag, rewrites the outputs.
+        uint32_t *long_words = p.small + 4;
         bool in_alt = false;
         QO_TRY(launch_radix_rows_segments(p.mkeys, p.mvals, p.kalt, p.valt, p.d_segs, p.nq, p.mt, p.d_chunks,
-                                           (uint32_t)p.hchunks.size(), p.d_chunk0, 32, 64, p.sort_ws, st, &in_alt));
+                                           (uint32_t)p.hchunks.size(), p.d_chunk0, 32, 64, p.sort_ws, st, &in_alt,
+                                           nullptr, run_if));
         uint64_t *ks = in_alt ? p.kalt : p.mkeys, *ka = in_alt ? p.mkeys : p.kalt;
         uint32_t *vs = in_alt ? p.valt : p.mvals, *va = in_alt ? p.mvals : p.valt;
-        QO_TRY(launch_fix_runs_segments(ks, vs, p.d_segs, p.nq, p.mt, p.d_outs, long_flag, st));
-        bool alt2 = false;
-        QO_TRY(launch_radix_rows_segments(ks, vs, ka, va, p.d_segs, p.nq, p.mt, p.d_chunks,
-                                           (uint32_t)p.hchunks.size(), p.d_chunk0, 0, 64, p.sort_ws, st, &alt2,
-                                           p.d_outs, long_flag));
+        QO_TRY(launch_fix_runs_segments(ks, vs, ka, va, p.d_segs, p.nq, p.mt, p.d_outs, long_words, p.long_list, st,
+                                        run_if));
+        if (!p.long_list) {
+            bool alt2 = false;
+            QO_TRY(launch_radix_rows_segments(ks, vs, ka, va, p.d_segs, p.nq, p.mt, p.d_chunks,
+                                               (uint32_t)p.hchunks.size(), p.d_chunk0, 0, 64, p.sort_ws, st, &alt2,
+                                               p.d_outs, long_words));
+        }
     }
-    return QO_OK;
+    return bj_counts_launch(p.sj, p.gcounts, p.nq, p.counts, st);
 }
 
 }  // namespace qo
@@ -315,20 +356,28 @@ struct qo_batch {
 
 using namespace qo;
 
-extern "C" {
+namespace qo {
 
-int qo_batch_create(const qo_join_query *queries, int nq, qo_batch **out) {
+int batch_create(const qo_join_query *queries, int nq, bool sorted, qo_batch **out) {
     QO_ENTER();
     QO_REQUIRE(out, "null output");
     *out = nullptr;
     qo_batch *b = new qo_batch;
-    int rc = join_plan_init(queries, nq, b->plan);
+    int rc = join_plan_init(queries, nq, b->plan, sorted);
     if (rc != QO_OK) {
         delete b;
         return rc;
     }
-    const size_t bytes = join_plan_bytes(b->plan);
+    size_t bytes = join_plan_bytes(b->plan);
     hipError_t e = hipMalloc(&b->arena, bytes);
+    if (e != hipSuccess && b->plan.sj.any_on) {
+        // No room for the buckets of the sorted join: the generic stages alone.
+        (void)hipGetLastError();
+        b->arena = nullptr;
+        b->plan.sj = SjBatchPlan{};
+        bytes = join_plan_bytes(b->plan);
+        e = hipMalloc(&b->arena, bytes);
+    }
     if (e != hipSuccess) {
         delete b;
         return set_error(QO_ERR_NO_MEMORY, "batch arena of %zu bytes: %s", bytes, hipGetErrorString(e));
@@ -359,6 +408,14 @@ int qo_batch_create(const qo_join_query *queries, int nq, qo_batch **out) {
     }
     *out = b;
     return QO_OK;
+}
+
+}  // namespace qo
+
+extern "C" {
+
+int qo_batch_create(const qo_join_query *queries, int nq, qo_batch **out) {
+    return batch_create(queries, nq, true, out);
 }
 
 int qo_batch_launch(qo_batch *b, qo_stream s) {

@@ -29,7 +29,58 @@ struct BQuery {
     uint32_t pad;
 };
 
+// Device descriptor of a query for the sorted join of small queries
+// (batch_sorted.hip), and what a launch finds out about it.
+struct SjBQuery {
+    const int32_t *rkey, *rpay, *skey, *spay, *sfilt;
+    uint64_t nr, ns;
+    int32_t flo, fhi;
+    int32_t *okey, *orpay, *ospay;
+    uint64_t out_cap;
+    uint32_t bucket0, nbmax;  // its buckets: [bucket0, bucket0 + nbmax)
+    uint32_t svec, rvec;      // columns 16-byte aligned
+    uint32_t on;              // 0: left to the generic stages
+    uint32_t pad;
+};
+struct SjBState {             // zero before a launch
+    uint32_t rmin_inv, rmax;  // ~smallest and largest build key, biased by 2^31
+    uint32_t pass;            // sampled S tuples that pass the filter
+    uint32_t pmin_inv, pmax;  // ~smallest and largest sampled s_payload, biased
+    uint32_t kmin, last, sh, nb, pay_bits;
+    uint32_t from;            // first of its buckets in the list of those in use
+    uint32_t overflow, repeated, missed, ticket;
+    uint64_t rows;            // matches
+};
+struct SjBucket {             // a bucket in use: S and build tuples, rows before it if every tuple matches
+    uint32_t q, f, n, nr, at, pad[3];
+};
+struct SjBatchPlan {
+    std::vector<SjBQuery> q;
+    std::vector<uint2> stiles, rtiles;  // (query, tile) of every split tile
+    uint32_t buckets = 0;
+    bool any_on = false, all_on = false;
+    SjBQuery *d_q = nullptr;
+    uint2 *d_stiles = nullptr, *d_rtiles = nullptr;
+    SjBucket *list = nullptr;     // the buckets in use, words[0] of them
+    uint32_t *skip = nullptr, *words = nullptr;  // words[1]: some query has unmatched tuples
+    SjBState *state = nullptr;
+    uint32_t *sctr = nullptr, *rctr = nullptr;
+    uint64_t *status = nullptr, *sbuckets = nullptr, *rbuckets = nullptr;
+    size_t clear_words = 0;
+};
+// generic[i]: query i is left to the generic stages.
+void bj_plan_init(const qo_join_query *queries, int nq, const std::vector<char> &generic, SjBatchPlan &p);
+void bj_plan_carve(SjBatchPlan &p, Carver &cv);
+int bj_plan_upload(const SjBatchPlan &p, hipStream_t st);
+// Joins the queries; afterwards skip[q] != 0 for those done, and *any (zeroed
+// before) is set when the generic stages have one left.
+int bj_plan_launch(const SjBatchPlan &p, uint32_t *any, hipStream_t st);
+// counts[q] = the matches of q, from the sorted join or the generic counters.
+int bj_counts_launch(const SjBatchPlan &p, const unsigned long long *generic, int nq, unsigned long long *counts,
+                     hipStream_t st);
+
 struct JoinBatchPlan {
+    SjBatchPlan sj;  // the queries' sorted join (any_on = false: none)
     int nq = 0;
     std::vector<BQuery> hq;
     std::vector<RadixSeg> hs;
@@ -63,12 +114,14 @@ struct JoinBatchPlan {
     uint32_t *d_chunk0 = nullptr;
     RowOut *d_outs = nullptr;
     void *sort_ws = nullptr;
+    SegPos *long_list = nullptr;  // long runs of the generic sort (all queries small)
     void *part_ws = nullptr;
-    unsigned long long *counts = nullptr;
+    unsigned long long *gcounts = nullptr;  // match counters of the generic stages (in `small`)
+    unsigned long long *counts = nullptr;   // match count per query
 };
 
-// Sizes the plan (host only).
-int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p);
+// Sizes the plan (host only).  `sorted`: small queries take the sorted join.
+int join_plan_init(const qo_join_query *queries, int nq, JoinBatchPlan &p, bool sorted = false);
 // Device bytes the plan needs.
 size_t join_plan_bytes(JoinBatchPlan &p);
 // Places the plan's buffers in `arena` and fills the per-query device pointers.
@@ -77,5 +130,9 @@ void join_plan_bind(JoinBatchPlan &p, void *arena);
 int join_plan_upload(const JoinBatchPlan &p, hipStream_t st);
 // Enqueues every stage (fills, build, probe, segmented sort, unpack) on st.
 int join_plan_launch(const JoinBatchPlan &p, hipStream_t st);
+
+// qo_batch_create; without `sorted` every query takes the generic stages (the
+// autotuner measures their parameters).
+int batch_create(const qo_join_query *queries, int nq, bool sorted, qo_batch **out);
 
 }  // namespace qo

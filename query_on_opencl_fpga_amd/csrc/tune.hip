@@ -26,6 +26,7 @@
 #include <functional>
 #include <vector>
 
+#include "qo_batch.hpp"
 #include "qo_internal.hpp"
 #include "qo_measure.hpp"
 
@@ -176,7 +177,7 @@ int make_workload(int op, size_t n, hipStream_t st, Workload &w) {
         w.prepare = [&w] {
             if (w.batch) qo_batch_destroy(w.batch);
             w.batch = nullptr;
-            return qo_batch_create(w.jq.data(), (int)w.jq.size(), &w.batch);
+            return batch_create(w.jq.data(), (int)w.jq.size(), false, &w.batch);
         };
         w.release = [&w] {
             if (w.batch) qo_batch_destroy(w.batch);
