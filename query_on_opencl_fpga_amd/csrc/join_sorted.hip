@@ -278,37 +278,70 @@ struct SjPlan {
 constexpr size_t kSjMinRows = size_t(1) << 14;
 constexpr uint64_t kSjMaxBuckets = 1u << (2 * kSjPartBits);
 
+// What the sample says about S: expected rows, and the most of them in an
+// aligned interval of 2^shift key offsets.
+struct SjSpread {
+    const SjInfo &info;
+    double rows, per, hot, span;  // per: tuples a sample stands for; hot: rows of the hottest key
+    int bsh;                      // a bin of the sample covers 2^bsh offsets
+    bool even;
+    SjSpread(const SjInfo &in, uint32_t last, size_t ns) : info(in) {
+        per = (double)ns / (double)std::min<size_t>(ns, kSjSamples);
+        rows = std::min((double)ns, std::max(1.0, per * (in.pass + 4.0 * std::sqrt((double)in.pass))));
+        // A key seen up to 6 times in the sample may be chance (or a collision); the
+        // largest of many counts lies above its own mean.
+        hot = in.hot <= 6 ? 0.0 : per * (in.hot - std::sqrt((double)in.hot));
+        span = (double)last + 1.0;
+        bsh = last < kSjBins ? 0 : 24 - __builtin_clz(last);
+        // Even: no bin far above the mean of the bins in use, as far as the sample can tell.
+        const double mean = (double)in.pass / ((last >> bsh) + 1);
+        const uint32_t top = *std::max_element(in.bin, in.bin + kSjBins);
+        even = top <= 1.5 * mean + 6.0 * std::sqrt(mean) + 4.0;
+    }
+    double most(int shift) const {
+        const double part = std::min(1.0, std::ldexp(1.0, shift) / span);
+        if (even) return rows * part + hot;
+        // Uneven: the fullest group of bins, or the fullest bin's share.
+        const uint32_t group = shift > bsh ? 1u << std::min(8, shift - bsh) : 1u;
+        uint32_t top = 0;
+        for (uint32_t b = 0; b < kSjBins; b += group) {
+            uint32_t c = 0;
+            for (uint32_t u = 0; u < group; ++u) c += info.bin[b + u];
+            top = std::max(top, c);
+        }
+        const double m = per * (top + 2.0 * std::sqrt((double)top));
+        return shift >= bsh ? m : m * std::ldexp(1.0, shift - bsh) + hot;
+    }
+};
+
 // A fine bucket has room for all the rows a work-group takes, whatever the
-// expected number: a hot key of some thousand rows still fits.
-static SjSide sj_side(const SjPlan &p, double rows, uint32_t limit) {
+// expected number: a hot key of some thousand rows still fits.  `most`: rows
+// expected in the fullest bucket of the first split.
+static SjSide sj_side(const SjPlan &p, double most, uint32_t limit) {
     SjSide o;
     o.capB = limit;
-    if (p.b2) {
-        const double span = (double)p.span.last + 1.0;
-        const double a = std::min(rows, rows * std::ldexp(1.0, p.sh + p.b2) / span) / kXcdRegions;
-        o.capA = ((uint64_t)(a * 1.25 + 8.0 * std::sqrt(a)) + kSplitTile + 31) / 32 * 32;
-    }
+    if (p.b2) o.capA = ((uint64_t)(most / kXcdRegions * 1.25 + 8.0 * std::sqrt(most)) + kSplitTile + 31) / 32 * 32;
     return o;
 }
 
 // Buckets for work-groups of nt threads: the widest whose rows (and build
-// keys) fit with room to spare beside a hot key's, and narrow enough to give a
-// small join a few work-groups per CU.
-static bool sj_buckets(SjPlan &p, int nt, double rows, double hot, size_t nr) {
-    const double limit = (double)kSjItems * nt, span = (double)p.span.last + 1.0;
-    const double room = 0.9 * limit - hot;
-    if (room < 0.1 * limit) return false;
-    const double want = std::min({0.75 * limit, room, std::max(512.0, rows / 512.0)});
+// keys) fit with room to spare, and narrow enough to give a small join a few
+// work-groups per CU.
+static bool sj_buckets(SjPlan &p, int nt, const SjSpread &s, size_t nr) {
+    const double limit = (double)sj_items(p.dense, nt) * nt;
+    const double want = std::min(0.75 * limit, std::max(512.0, s.rows / 512.0));
     p.nt = nt;
     p.sh = 0;
     while (p.sh < 31) {
         const double w = std::ldexp(1.0, p.sh + 1);
-        if (rows * w / span > want || w / 2 >= span) break;  // 2^sh <= the smallest power of two >= span
-        if (p.dense ? w > 2.0 * nt : (double)nr * w / span > 1.5 * nt) break;
+        if (s.rows * w / s.span > want || w / 2 >= s.span) break;  // 2^sh <= the smallest power of two >= span
+        if (s.most(p.sh + 1) > 0.9 * limit) break;
+        if (p.dense ? w > 2.0 * nt : (double)nr * w / s.span > 1.5 * nt) break;
         ++p.sh;
     }
     const uint64_t nb = ((uint64_t)p.span.last >> p.sh) + 1;
-    if (nb > kSjMaxBuckets || rows * std::ldexp(1.0, p.sh) / span > std::min(room, 0.8 * limit)) return false;
+    // Of uneven keys no more buckets than a few per 1000 rows: most would be empty.
+    if (nb > kSjMaxBuckets || s.most(p.sh) > 0.9 * limit || (!s.even && nb > 1024 + s.rows / 256)) return false;
     p.nb = (uint32_t)nb;
     int bits = 0;
     while ((1u << bits) < p.nb) ++bits;
@@ -316,8 +349,11 @@ static bool sj_buckets(SjPlan &p, int nt, double rows, double hot, size_t nr) {
     p.nb1 = ((p.nb - 1) >> p.b2) + 1;
     p.parts1 = 1;
     while (p.parts1 < p.nb1) p.parts1 *= 2;
-    p.s = sj_side(p, rows, (uint32_t)limit);
-    if (!p.dense) p.r = sj_side(p, (double)nr, 2u * (uint32_t)nt);
+    p.s = sj_side(p, s.most(p.sh + p.b2), (uint32_t)limit);
+    if (!p.dense) {
+        const double even = (double)nr * std::min(1.0, std::ldexp(1.0, p.sh + p.b2) / s.span);
+        p.r = sj_side(p, s.even ? even : std::min((double)nr, 4.0 * even), 2u * (uint32_t)nt);
+    }
     return true;
 }
 
@@ -325,21 +361,12 @@ static SjPlan sj_plan(const SjInfo &info, size_t nr, size_t ns) {
     SjPlan p;
     if (info.dups || info.rmin > info.rmax || info.pass == 0) return p;
     const uint32_t last = (uint32_t)info.rmax - (uint32_t)info.rmin;
-    // Even spread: no bin of the sample far above the mean of the bins in use.
-    const int bsh = last < kSjBins ? 0 : 24 - __builtin_clz(last);
-    const double mean = (double)info.pass / ((last >> bsh) + 1);
-    const uint32_t top = *std::max_element(info.bin, info.bin + kSjBins);
-    if (top > 1.5 * mean + 6.0 * std::sqrt(mean) + 4.0) return p;
-    const double per = (double)ns / (double)std::min<size_t>(ns, kSjSamples);  // tuples a sample stands for
-    const double rows = std::min((double)ns, std::max(1.0, per * (info.pass + 4.0 * std::sqrt((double)info.pass))));
-    // A key seen up to 6 times in the sample may be chance (or a collision); the
-    // largest of many counts lies above its own mean.
-    const double hot = info.hot <= 6 ? 0.0 : per * (info.hot - std::sqrt((double)info.hot));
+    const SjSpread s(info, last, ns);
     p.dense = info.mode == kJoinKeyRange;
     p.all = info.match == info.pass;
     p.span = KeySpan{(uint32_t)info.rmin, last};
     p.pay = PayloadBins{~info.pmin, 32 - __builtin_clz((info.pmax - ~info.pmin) | 1u)};
-    p.on = sj_buckets(p, 512, rows, hot, nr) || sj_buckets(p, 1024, rows, hot, nr);
+    p.on = sj_buckets(p, 512, s, nr) || sj_buckets(p, 1024, s, nr);
     return p;
 }
 

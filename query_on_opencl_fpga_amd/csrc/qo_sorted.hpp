@@ -23,7 +23,9 @@ struct FlagOverflow {
 };
 
 constexpr uint32_t kSjRankRun = 256;  // longest run whose rows are ranked one against another
-constexpr int kSjItems = 6;           // S tuples per thread
+// S tuples per thread: six, and for the larger work-groups, which take the joins
+// with a hot key, as many as leave room for two of them per CU.
+constexpr int sj_items(bool dense, int nt) { return nt <= 512 ? 6 : dense ? 8 : 7; }
 
 // Interval of the s_payload's range, by which a build key's matches are
 // counted: 2^sb intervals of [pmin, pmin + 2^bits), monotone in the s_payload
@@ -45,11 +47,11 @@ struct PayloadBins {
 // 1024 threads with at most 80 KB of LDS.
 template <bool DENSE, int NT>
 struct SjLds {
-    static constexpr int kItems = kSjItems;
+    static constexpr int kItems = sj_items(DENSE, NT);
     static constexpr uint32_t kRows = (uint32_t)kItems * NT;
     static constexpr uint32_t kSlots = 2 * NT;
     static constexpr int kBinBits = __builtin_ctz(kSlots);  // bins of a sparse bucket's key interval
-    static constexpr int kPer = DENSE ? 8 : 4;
+    static constexpr int kPer = (DENSE ? 8 : 4) / (NT <= 512 ? 1 : 2);
     static constexpr uint32_t kBins = (uint32_t)kPer * NT;
     uint32_t cnt[kBins + 1];  // matches per bin, then where its run starts
     uint32_t pay[kSlots];
@@ -79,7 +81,7 @@ struct SjBuckets {
 // run starts in s.cnt give way to the waves' digit counts.
 template <bool DENSE, int NT>
 QO_DEV void sj_sort_rows(SjLds<DENSE, NT> &s, uint32_t total, int sb) {
-    constexpr int IT = kSjItems;
+    constexpr int IT = SjLds<DENSE, NT>::kItems;
     constexpr int kWaves = NT / kWave;
     static_assert(kWaves * 256 * sizeof(uint16_t) <= sizeof(s.cnt), "digit counts");
     uint16_t(*cnt)[256] = reinterpret_cast<uint16_t(*)[256]>(s.cnt);
@@ -175,7 +177,7 @@ QO_DEV void sj_bucket(SjLds<DENSE, NT> &s, const uint64_t *__restrict__ src, uin
                       const uint64_t *__restrict__ rsrc, uint32_t nr, const uint64_t *__restrict__ slots, uint32_t kbase,
                       int sh, const PayloadBins &pbins, const SoaEmit &emit, const Start &start) {
     using Lds = SjLds<DENSE, NT>;
-    constexpr int IT = kSjItems;
+    constexpr int IT = SjLds<DENSE, NT>::kItems;
     // The build side's loads go first: its work then runs while the S tuples are
     // still on their way.
     const uint32_t nb = DENSE ? 1u << sh : nr;  // slots of the slice, or build tuples
