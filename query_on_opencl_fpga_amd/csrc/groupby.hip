@@ -3,10 +3,11 @@
 // 1. Hash aggregation (qo_groupby_agg): every block keeps an LDS-resident
 //    partial table (key, COUNT, SUM, MIN, MAX) with linear probing; tuples whose
 //    key does not find an LDS slot within a few probes update a global
-//    open-addressing table directly.  At the end each block merges its LDS table
-//    into the global one (or, when it saw every tuple of its keys, appends its
-//    groups as finished rows); the rows are sorted by key and gathered into the
-//    SoA outputs.
+//    open-addressing table directly.  At the end the blocks' LDS tables are merged
+//    into the global one, by a launch that merges one key range of every block in
+//    LDS or, of few blocks, by global atomics (a block that saw every tuple of its
+//    keys appends its groups as finished rows); the rows are sorted by key and
+//    gathered into the SoA outputs.
 // 2. The reference's sort-based pipeline for drop-in callers: group start
 //    positions over Records sorted by .y (scanGroupLabel_kernel +
 //    groupByImpl_write_kernel, kernel/aggregation/1/group_by_cu_op_dp.cl:293-327,
@@ -183,10 +184,14 @@ QO_DEV void ltable_add(LTable<C> &L, int32_t k, int32_t v, int probes, GEntry *g
     }
     int s = (uint32_t)k == kEmptyKey ? -1 : l_slot<C, TWO>(L.key, (uint32_t)k, probes, skip);
     if (s >= 0) {
+        // MIN and MAX are read first: once a group has seen a few tuples hardly any
+        // changes them, and a read costs less than an LDS atomic (2^28 tuples, 1024
+        // groups: 476 -> 443 us; with Zipf sizes 663 -> 549; 16 groups 695 -> 504).
+        const int32_t lo = L.mn[s], hi = L.mx[s];
         atomicAdd(&L.cnt[s], cnt);
         atomicAdd(&L.sum[s], (unsigned long long)sum);
-        atomicMin(&L.mn[s], mn);
-        atomicMax(&L.mx[s], mx);
+        if (mn < lo) atomicMin(&L.mn[s], mn);
+        if (mx > hi) atomicMax(&L.mx[s], mx);
     } else {
         g_update(gt, gmask, (uint32_t)k, cnt, sum, mn, mx, overflow);
     }
@@ -203,6 +208,126 @@ QO_DEV void ltable_flush(const LTable<C> &L, GEntry *gt, uint64_t gmask, uint32_
         const int i = (j + rot) & (C - 1);
         if (L.cnt[i]) g_update(gt, gmask, L.key[i], L.cnt[i], L.sum[i], L.mn[i], L.mx[i], overflow);
     }
+}
+
+// ---------------------------------------------------------------------------
+// Merge of the blocks' LDS tables without global atomics per block and group.
+// Merging every table straight into the global one queues blocks x groups x 4
+// atomics on few cache lines, whose updates the L2 takes one after another: 4 M
+// rows in 1024 groups took 103 us at 256 blocks and 310 at 1024 (47.9 and 85.7
+// with the merge), 1 M rows 91 (41).  Instead each block writes its
+// groups out ordered by kMergeParts ranges of the key hash, and one work-group
+// per range merges that range of every block in LDS and updates the global table
+// once per group.
+// ---------------------------------------------------------------------------
+constexpr int kMergeBits = 7;
+constexpr uint32_t kMergeParts = 1u << kMergeBits;
+constexpr int kMergeThreads = 256;
+constexpr uint32_t kMergeMaxBlocks = 2048;
+constexpr int kMergeSlots = 1024;
+
+struct Partials {
+    GEntry *ent = nullptr;      // block b's groups at [b * C, ...), by range; null: no merge
+    uint32_t *start = nullptr;  // start[p * blocks + b]: where range p begins there; kMergeParts + 1 rows
+};
+
+// Writes the block's groups (after a barrier); all NT threads.
+template <int C, int NT>
+QO_DEV void ltable_partials(const LTable<C> &L, const Partials &out) {
+    static_assert(C % NT == 0 && NT >= (int)kMergeParts, "table size");
+    constexpr int kPer = C / NT;
+    __shared__ uint32_t s_cnt[kMergeParts], s_w[NT / kWave];
+    if (threadIdx.x < kMergeParts) s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t at[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = k * NT + threadIdx.x;
+        if (L.cnt[i]) at[k] = atomicAdd(&s_cnt[fib_slot(L.key[i], kMergeBits)], 1u);
+    }
+    __syncthreads();
+    const uint32_t c = threadIdx.x < kMergeParts ? s_cnt[threadIdx.x] : 0u;
+    const uint32_t ex = block_excl_scan<NT / kWave>(c, s_w);
+    if (threadIdx.x < kMergeParts) {
+        s_cnt[threadIdx.x] = ex;
+        out.start[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = ex;
+        if (threadIdx.x == kMergeParts - 1) out.start[(size_t)kMergeParts * gridDim.x + blockIdx.x] = ex + c;
+    }
+    __syncthreads();
+    GEntry *dst = out.ent + (size_t)blockIdx.x * C;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = k * NT + threadIdx.x;
+        if (!L.cnt[i]) continue;
+        GEntry e;
+        e.key = L.key[i];
+        e.mn = L.mn[i];
+        e.mx = L.mx[i];
+        e.pad = 0;
+        e.cnt = L.cnt[i];
+        e.sum = L.sum[i];
+        dst[s_cnt[fib_slot(e.key, kMergeBits)] + at[k]] = e;
+    }
+}
+
+// Range blockIdx.x of all `blocks` tables of C slots, merged into the global
+// table.  Counts stay below 2^32 (the launch's rule).
+__global__ __launch_bounds__(kMergeThreads) void k_groupby_merge(Partials in, uint32_t blocks, uint32_t C, GEntry *gt,
+                                                                 uint64_t gmask, uint32_t *overflow) {
+    constexpr uint32_t kPer = kMergeMaxBlocks / kMergeThreads;
+    __shared__ LTable<kMergeSlots> L;
+    __shared__ uint32_t s_pre[kMergeMaxBlocks + 1], s_from[kMergeMaxBlocks];
+    __shared__ uint32_t s_w[kMergeThreads / kWave];
+    const uint32_t *lo = in.start + (size_t)blockIdx.x * blocks, *hi = lo + blocks;
+    ltable_init<kMergeSlots>(L);
+    uint32_t c[kPer], sum = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) {
+        const uint32_t b = threadIdx.x * kPer + u;
+        const uint32_t f = b < blocks ? lo[b] : 0u;
+        c[u] = b < blocks ? hi[b] - f : 0u;
+        s_from[b] = f;
+        sum += c[u];
+    }
+    uint32_t at = block_excl_scan<kMergeThreads / kWave>(sum, s_w);
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) {
+        s_pre[threadIdx.x * kPer + u] = at;
+        at += c[u];
+    }
+    if (threadIdx.x == kMergeThreads - 1) s_pre[kMergeMaxBlocks] = at;
+    __syncthreads();
+    const uint32_t n = s_pre[kMergeMaxBlocks];
+    constexpr int kU = 4;  // entries in flight per thread
+    for (uint32_t e0 = threadIdx.x; e0 < n; e0 += kU * kMergeThreads) {
+        GEntry e[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const uint32_t i = e0 + u * kMergeThreads;
+            if (i >= n) continue;
+            uint32_t b = 0;  // last block whose entries start at or before i
+#pragma unroll
+            for (uint32_t step = kMergeMaxBlocks / 2; step; step /= 2)
+                if (s_pre[b + step] <= i) b += step;
+            e[u] = in.ent[(size_t)b * C + s_from[b] + (i - s_pre[b])];
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            if (e0 + u * kMergeThreads >= n) continue;
+            const int sl = l_slot<kMergeSlots>(L.key, e[u].key, 64, kMergeBits);  // tables hold no empty-marker key
+            if (sl >= 0) {
+                atomicAdd(&L.cnt[sl], (uint32_t)e[u].cnt);
+                atomicAdd(&L.sum[sl], e[u].sum);
+                atomicMin(&L.mn[sl], e[u].mn);
+                atomicMax(&L.mx[sl], e[u].mx);
+            } else {
+                g_update(gt, gmask, e[u].key, e[u].cnt, e[u].sum, e[u].mn, e[u].mx, overflow);
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kMergeSlots; i += kMergeThreads)
+        if (L.cnt[i]) g_update(gt, gmask, L.key[i], L.cnt[i], L.sum[i], L.mn[i], L.mx[i], overflow);
 }
 
 // Appends the block's LDS groups as finished rows (the block saw every tuple
@@ -331,8 +456,9 @@ QO_DEV void dom_merge(LTable<C> &L, const DomAcc &a, uint32_t dom, int probes, i
 template <int C, bool VEC, int NT, bool FILT = false>
 __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__ key, const int32_t *__restrict__ val,
                                                       size_t n, GEntry *gt, uint64_t gmask, int probes,
-                                                      uint32_t *overflow, const int32_t *__restrict__ filt = nullptr,
-                                                      int32_t flo = 0, int32_t fhi = 0) {
+                                                      uint32_t *overflow, Partials parts,
+                                                      const int32_t *__restrict__ filt = nullptr, int32_t flo = 0,
+                                                      int32_t fhi = 0) {
     extern __shared__ unsigned char s_raw[];
     LTable<C> &L = *reinterpret_cast<LTable<C> *>(s_raw);
     __shared__ uint32_t s_dom, s_dom2, s_heavy;
@@ -410,7 +536,8 @@ __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__
     if (s_heavy) body(std::true_type{});
     else body(std::false_type{});
     __syncthreads();
-    ltable_flush<C>(L, gt, gmask, overflow);
+    if (parts.ent) ltable_partials<C, NT>(L, parts);
+    else ltable_flush<C>(L, gt, gmask, overflow);
 }
 
 // ---------------------------------------------------------------------------
@@ -927,7 +1054,33 @@ struct GroupbyBufs {
     OnePassBufs op;      // partitioned path, one-pass partition
     uint32_t *cch = nullptr, *cpre = nullptr;
     void *scan_ws = nullptr;
+    Partials parts;      // direct path with a merge launch
 };
+
+// Direct path: one 1024-thread block per 4096 tuples, up to the tuned number per
+// CU, with LDS tables of C slots.  One per CU by default: the blocks' tables are
+// all merged at the end, and what more of them cost there is more than their
+// occupancy buys (2^28 tuples, 1024 groups: 0.41 ms with one, 0.50 with four).
+struct HashPlan {
+    int C = 0;
+    unsigned grid = 0;
+    bool merge = false;
+};
+constexpr int kHashThreads = 1024;
+// Fewer blocks than this merge straight into the global table: the merge launch
+// costs 5 us, the atomics grow with blocks and groups.  They break even (one
+// block per 4096 rows) at 74 blocks with 16 or 100 groups, 32 with 1024, and
+// below 8 with 5000.
+static unsigned merge_min_blocks(size_t groups) { return groups < 1600 ? 76u - (unsigned)(groups * 43 / 1000) : 8u; }
+
+static HashPlan hash_plan(size_t n, size_t groups) {
+    HashPlan h;
+    const TuneParams tp = tune_get(TUNE_GROUPBY, n);
+    h.C = tp.items >= 4096 && (size_t)props().lds_per_block >= sizeof(LTable<4096>) ? 4096 : 2048;
+    h.grid = grid_for(n, kHashThreads * 4, (unsigned)props().cu_count * (unsigned)std::max(1, tp.param));
+    h.merge = h.grid >= merge_min_blocks(groups) && h.grid <= kMergeMaxBlocks && n < 0xFFFFFFFFull;
+    return h;
+}
 
 static GroupbyBufs groupby_carve(const GroupbyPlan &p, const GbPartPlan &pp, size_t group_capacity, size_t n,
                                  Carver &cv) {
@@ -944,6 +1097,9 @@ static GroupbyBufs groupby_carve(const GroupbyPlan &p, const GbPartPlan &pp, siz
         b.cch = cv.take<uint32_t>(nb + 1);
         b.cpre = cv.take<uint32_t>(nb + 1);
         b.scan_ws = cv.take<char>(scan_workspace_bytes(nb + 1));
+    } else if (const HashPlan h = hash_plan(n, group_capacity); n && h.merge) {
+        b.parts.ent = cv.take<GEntry>((size_t)h.grid * h.C);
+        b.parts.start = cv.take<uint32_t>((size_t)h.grid * (kMergeParts + 1));
     }
     return b;
 }
@@ -999,24 +1155,17 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
             reinterpret_cast<unsigned long long *>(counters), group_capacity);
         QO_LAUNCHED();
     } else if (n) {
-        TuneParams tp = tune_get(TUNE_GROUPBY, n);
+        const HashPlan h = hash_plan(n, group_capacity);
         const bool vec = ((uintptr_t)key % 16 == 0) && ((uintptr_t)val % 16 == 0) && ((uintptr_t)filt % 16 == 0);
-        int C = tp.items >= 4096 ? 4096 : 2048;
-        const size_t lds4096 = sizeof(LTable<4096>);
-        if (C == 4096 && (size_t)props().lds_per_block < lds4096) C = 2048;
-        // One 1024-thread block per CU by default: every block merges its whole
-        // LDS table into the global one at the end, and those global atomics
-        // (blocks x groups x 4) cost more than the occupancy of more blocks buys
-        // (2^28 tuples, 1024 groups: 0.68 ms with 3 x 512 threads per CU, 0.43
-        // ms with 1 x 1024).
-        constexpr int block = 1024;
-        const unsigned grid = grid_for(n, block * 4, (unsigned)props().cu_count * (unsigned)std::max(1, tp.param));
+        const int C = h.C;
+        constexpr int block = kHashThreads;
+        const unsigned grid = h.grid;
         // Low cardinality: the LDS table holds every group.  High cardinality:
         // it caches the keys seen first and the rest go straight to global.
         const int probes = group_capacity * 2 <= (size_t)C ? C : 8;
 #define QO_GBH(CC, V, F)                                                                                    \
     k_groupby_hash<CC, V, block, F><<<grid, block, sizeof(LTable<CC>), st>>>(key, val, n, gt, p.gmask, probes,  \
-                                                                             overflow, filt, flo, fhi)
+                                                                             overflow, b.parts, filt, flo, fhi)
         if (C == 4096) {
             if (filt) {
                 if (vec) QO_GBH(4096, true, true);
@@ -1036,6 +1185,10 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
         }
 #undef QO_GBH
         QO_LAUNCHED();
+        if (b.parts.ent) {
+            k_groupby_merge<<<kMergeParts, kMergeThreads, 0, st>>>(b.parts, grid, (uint32_t)C, gt, p.gmask, overflow);
+            QO_LAUNCHED();
+        }
     }
     if (group_capacity > 0 && group_capacity <= kFinishGroups) {
         const uint32_t entries = (uint32_t)p.entries, cap = (uint32_t)group_capacity;

@@ -70,3 +70,15 @@ def test_join_rows_long_runs(qo, orc, m, hot):
     rp = k * np.int32(3) + np.int32(1)
     for g, e in zip(qo.operators.sort_join_rows(k, rp, sp), orc.sort_join_rows(k, rp, sp)):
         assert np.array_equal(g, e)
+
+
+@pytest.mark.parametrize("groups,n", [(16, 300_000), (16, 320_000), (1024, 126_000), (1024, 140_000), (5000, 40_000),
+                                      (2000, 1_000_003), (70_000, 900_000)])
+def test_group_merge_edges(qo, orc, groups, n):
+    """Around the number of blocks from which a launch merges their tables; more groups than one table holds; the
+    empty-marker key."""
+    k = (orc.gen_uniform_u32(n, 9, 0, 0, groups).astype(np.int64) * 2_654_435_761).astype(np.uint32).astype(np.int32)
+    k[k == k[0]] = -1
+    v = orc.gen_uniform_u32(n, 9, 1, 0, 0).astype(np.int32)
+    for g, e in zip(qo.operators.groupby_agg(k, v, groups), orc.groupby_agg(k, v)):
+        assert np.array_equal(g, e)
