@@ -142,11 +142,6 @@ size_t radix_workspace_bytes(size_t n, bool with_vals);
 size_t split_records_ws_bytes(size_t n, uint32_t parts);
 int launch_split_records(const uint64_t *in, size_t n, uint32_t parts, uint64_t *out, uint2 *bound, void *ws,
                          hipStream_t st);
-int launch_radix_sort_u64(uint64_t *keys, uint32_t *vals, size_t n, int lo_bit, int hi_bit, void *ws,
-                          hipStream_t st);
-// Same, reading the element count from device memory (grid sized for `capacity`).
-int launch_radix_sort_u64_dev(uint64_t *keys, uint32_t *vals, const uint64_t *d_n, size_t capacity,
-                              int lo_bit, int hi_bit, void *ws, hipStream_t st);
 
 // Sort of join rows by (key, s_payload) with caller workspace.
 size_t sort_join_rows_ws_bytes(size_t m);

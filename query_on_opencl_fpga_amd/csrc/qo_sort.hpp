@@ -88,6 +88,27 @@ QO_DEV uint64_t match_digit(uint32_t d, bool valid) {
     return m;
 }
 
+// A sort by the high 32 key bits whose passes are picked on the device: a digit
+// in which all keys agree gets no placement.  An odd number of placements would
+// leave the keys in the other buffer, so the pass of the lowest such digit then
+// copies them over (with four digits there is one).  diff: the bits (of key >> 32)
+// in which any key differs from the first.  Returns what the pass at `shift` does
+// (0: nothing) and, in bit 8, whether the keys are in the other buffer before it.
+// Kernels read diff through a __restrict__ argument: as a scalar load it is there
+// in a fraction of the microsecond a vector load takes at the start of every block.
+constexpr uint32_t kPassPlace = 1, kPassCopy = 2;
+QO_DEV uint32_t radix_pass(uint32_t diff, int shift) {
+    uint32_t mask = 0;  // passes that place
+#pragma unroll
+    for (int p = 0; p < 4; ++p) mask |= (((diff >> (8 * p)) & 255u) != 0 ? 1u : 0u) << p;
+    const uint32_t copy = (__popc(mask) & 1) ? ~mask & (mask + 1u) : 0u;  // lowest pass without a placement
+    const uint32_t p = 1u << ((shift - 32) / 8);
+    const uint32_t before = __popc((mask | copy) & (p - 1u));
+    return ((mask & p) ? kPassPlace : (copy & p) ? kPassCopy : 0u) | ((before & 1u) << 8);
+}
+// Sorts `list` by the high 32 bits, n = *d_n (at most `capacity`).
+int launch_radix_sort_list(uint64_t *list, const uint64_t *d_n, size_t capacity, void *ws, hipStream_t st);
+
 // One-block stable radix sort of up to kBlockSortThreads * ITEMS 64-bit keys
 // (and 32-bit values) that lie in LDS.  What bounds it is the chain of passes:
 // a pass reads the block's keys, ranks them with wave ballots, scans 16 x 256

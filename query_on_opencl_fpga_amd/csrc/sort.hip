@@ -59,12 +59,20 @@ constexpr int kHistTiles = 2;             // tiles per block of k_tile_hist
 constexpr uint32_t kRowsBlocks = 512;     // at most this many column-scan blocks
 constexpr uint32_t kRowsMinSpan = 64;     // tiles per column-scan block, at least
 constexpr uint32_t kRowsOneBlock = 256;   // up to this many tiles, one block scans the rows
+constexpr uint32_t kRowsFew = 64;         // up to this many, each placement block does
+static_assert(kRowsFew / kHistTiles <= kWave, "a lane per histogram block");
 
 // Digit counts of one tile (rem keys at src) into 256 LDS counters; `vec`:
-// src is 16-byte aligned, so two keys are read per load.
+// src is 16-byte aligned, so two keys are read per load.  Returns the bits of
+// any key >> 32 that differ from `first`.
 template <bool MOD = false>
-QO_DEV void hist_tile(const uint64_t *__restrict__ src, uint32_t rem, int shift, uint32_t *s_row, bool vec,
-                      uint32_t mod = 0) {
+QO_DEV uint32_t hist_tile(const uint64_t *__restrict__ src, uint32_t rem, int shift, uint32_t *s_row, bool vec,
+                          uint32_t mod, uint32_t first) {
+    uint32_t diff = 0;
+    auto count = [&](uint64_t k) {
+        atomicAdd(&s_row[key_digit<MOD>(k, shift, mod)], 1u);
+        diff |= (uint32_t)(k >> 32) ^ first;
+    };
     if (vec) {
         constexpr int PER = kSortTile / 512;
         uint4 q[PER];
@@ -77,29 +85,38 @@ QO_DEV void hist_tile(const uint64_t *__restrict__ src, uint32_t rem, int shift,
         for (int j = 0; j < PER; ++j) {
             const uint32_t v = j * 256 + threadIdx.x;
             if (2 * v + 2 <= rem) {
-                const uint64_t k0 = ((uint64_t)q[j].y << 32) | q[j].x;
-                const uint64_t k1 = ((uint64_t)q[j].w << 32) | q[j].z;
-                atomicAdd(&s_row[key_digit<MOD>(k0, shift, mod)], 1u);
-                atomicAdd(&s_row[key_digit<MOD>(k1, shift, mod)], 1u);
+                count(((uint64_t)q[j].y << 32) | q[j].x);
+                count(((uint64_t)q[j].w << 32) | q[j].z);
             } else if (2 * v < rem) {
-                atomicAdd(&s_row[key_digit<MOD>(src[2 * v], shift, mod)], 1u);
+                count(src[2 * v]);
             }
         }
     } else {
-        for (uint32_t i = threadIdx.x; i < rem; i += 256) atomicAdd(&s_row[key_digit<MOD>(src[i], shift, mod)], 1u);
+        for (uint32_t i = threadIdx.x; i < rem; i += 256) count(src[i]);
     }
+    return diff;
 }
 
 // rows[t * 256 + d] = keys of global tile t whose digit is d (zero rows for
 // tiles past their segment's element count).  A single array passes its
-// segment as seg0 with segs = null; a batch passes the segment list.
-template <bool MOD = false>
+// segment as seg0 with segs = null; a batch passes the segment list.  diffs
+// (first pass of a sort with the digits found out on the device): one word per
+// block, the bits of key >> 32 in which its keys differ from the array's first.
+template <bool MOD = false, bool DYN = false>
 __global__ __launch_bounds__(256) void k_tile_hist(const uint64_t *__restrict__ keys, RadixSeg seg0,
                                                    const RadixSeg *segs, int nseg, uint32_t ntile, int shift,
                                                    uint32_t *__restrict__ rows, const uint32_t *run_if = nullptr,
-                                                   uint32_t mod = 0) {
+                                                   uint32_t mod = 0, const uint32_t *__restrict__ sel = nullptr,
+                                                   const uint64_t *kalt = nullptr, uint32_t *diffs = nullptr) {
     if (run_if && *run_if == 0) return;  // gated off: runs only when *run_if != 0
+    if (DYN && !diffs) {  // (the first pass finds the digits out and always counts)
+        const uint32_t plan = radix_pass(*sel, shift);
+        if (!(plan & kPassPlace)) return;
+        if (plan >> 8) keys = kalt;
+    }
     __shared__ uint32_t s_h[kHistTiles][256];
+    __shared__ uint32_t s_diff;
+    if (DYN && threadIdx.x == 0) s_diff = 0;
     for (int i = threadIdx.x; i < kHistTiles * 256; i += 256) (&s_h[0][0])[i] = 0;
     __syncthreads();
     const uint32_t t0 = blockIdx.x * kHistTiles;
@@ -112,10 +129,13 @@ __global__ __launch_bounds__(256) void k_tile_hist(const uint64_t *__restrict__ 
         const size_t tb = (size_t)(t - sg.tile0) * kSortTile;
         if (tb >= n) continue;
         const uint64_t *src = keys + sg.base + tb;
-        hist_tile<MOD>(src, (uint32_t)std::min<size_t>(kSortTile, n - tb), shift, s_h[tt],
-                       (reinterpret_cast<uintptr_t>(src) & 15) == 0, mod);
+        const uint32_t d = hist_tile<MOD>(src, (uint32_t)std::min<size_t>(kSortTile, n - tb), shift, s_h[tt],
+                                          (reinterpret_cast<uintptr_t>(src) & 15) == 0, mod,
+                                          DYN && diffs ? (uint32_t)(keys[sg.base] >> 32) : 0u);
+        if (DYN && diffs && d) atomicOr(&s_diff, d);
     }
     __syncthreads();
+    if (DYN && diffs && threadIdx.x == 0) diffs[blockIdx.x] = s_diff;
 #pragma unroll
     for (int tt = 0; tt < kHistTiles; ++tt)
         if (t0 + tt < ntile) rows[(size_t)(t0 + tt) * 256 + threadIdx.x] = s_h[tt][threadIdx.x];
@@ -132,36 +152,68 @@ static RowsPlan rows_plan(uint32_t ntile) {
     return r;
 }
 
+// The three column-scan kernels are chains of loads by few threads, so what
+// bounds them is the loads in flight: 32 per thread instead of 8, with the values
+// kept in registers between summing and writing (1 M keys, one-block scan, four
+// passes: 133 -> 120 us in all).
+constexpr uint32_t kRowsU = 32;
+
+// Sum of column entries [t, t + kRowsU) of `col` (entries 256 words apart) below
+// t1, loaded together.
+QO_DEV uint32_t rows_batch(const uint32_t *col, uint32_t t, uint32_t t1, uint32_t (&v)[kRowsU]) {
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kRowsU; ++u) v[u] = t + u < t1 ? col[(size_t)(t + u) * 256] : 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < kRowsU; ++u) sum += v[u];
+    return sum;
+}
+
+// Entries [t, t + kRowsU) below t1 := run + the entries before each in v.
+QO_DEV uint32_t rows_write(uint32_t *col, uint32_t t, uint32_t t1, const uint32_t (&v)[kRowsU], uint32_t run) {
+#pragma unroll
+    for (uint32_t u = 0; u < kRowsU; ++u) {
+        if (t + u < t1) col[(size_t)(t + u) * 256] = run;
+        run += v[u];
+    }
+    return run;
+}
+
 // bsum[b * 256 + d] = digit-d keys of the tiles of block b.
 __global__ __launch_bounds__(256) void k_rows_reduce(const uint32_t *__restrict__ rows, uint32_t ntile, uint32_t span,
                                                      uint32_t *__restrict__ bsum) {
     const uint32_t t0 = blockIdx.x * span, t1 = std::min(ntile, t0 + span);
-    const uint32_t *col = rows + threadIdx.x;
-    uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // independent sums: loads stay in flight together
-    uint32_t t = t0;
-    for (; t + 8 <= t1; t += 8)
-#pragma unroll
-        for (int u = 0; u < 8; ++u) c[u] += col[(size_t)(t + u) * 256];
-    for (; t < t1; ++t) c[0] += col[(size_t)t * 256];
-    bsum[(size_t)blockIdx.x * 256 + threadIdx.x] = c[0] + c[1] + c[2] + c[3] + c[4] + c[5] + c[6] + c[7];
+    uint32_t sum = 0, v[kRowsU];
+    for (uint32_t t = t0; t < t1; t += kRowsU) sum += rows_batch(rows + threadIdx.x, t, t1, v);
+    bsum[(size_t)blockIdx.x * 256 + threadIdx.x] = sum;
 }
 
 // One block of 1024 threads: bsum[b][d] := start of digit d in the output +
 // digit-d keys of blocks before b (exclusive, in place).  Thread (q, d) with
-// q = threadIdx / 256 handles quarter q of the blocks for digit d.
-__global__ __launch_bounds__(1024) void k_rows_starts(uint32_t *bsum, uint32_t nb) {
+// q = threadIdx / 256 handles quarter q of the blocks for digit d.  First pass
+// of a sort with the digits found out on the device: *diff := the union of the
+// ndiff words at `diffs`.
+__global__ __launch_bounds__(1024) void k_rows_starts(uint32_t *bsum, uint32_t nb, const uint32_t *diffs = nullptr,
+                                                      uint32_t ndiff = 0, uint32_t *diff = nullptr) {
     __shared__ uint32_t s_part[4][256];
     __shared__ uint32_t s_w[16];
+    __shared__ uint32_t s_diff;
+    if (diff) {
+        if (threadIdx.x == 0) s_diff = 0;
+        __syncthreads();
+        uint32_t d = 0;
+        for (uint32_t i = threadIdx.x; i < ndiff; i += 1024) d |= diffs[i];
+        if (d) atomicOr(&s_diff, d);
+        __syncthreads();
+        if (threadIdx.x == 0) *diff = s_diff;
+    }
     const uint32_t d = threadIdx.x & 255u, q = threadIdx.x >> 8;
     const uint32_t per = (nb + 3) / 4, b0 = std::min(nb, q * per), b1 = std::min(nb, b0 + per);
     uint32_t *col = bsum + d;
-    uint32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t b = b0;
-    for (; b + 8 <= b1; b += 8)
-#pragma unroll
-        for (int u = 0; u < 8; ++u) c[u] += col[(size_t)(b + u) * 256];
-    for (; b < b1; ++b) c[0] += col[(size_t)b * 256];
-    s_part[q][d] = c[0] + c[1] + c[2] + c[3] + c[4] + c[5] + c[6] + c[7];
+    uint32_t v[kRowsU], sum = 0;
+    for (uint32_t b = b0 + kRowsU; b < b1; b += kRowsU) sum += rows_batch(col, b, b1, v);
+    sum += rows_batch(col, b0, b1, v);  // the first batch stays in registers
+    s_part[q][d] = sum;
     __syncthreads();
     const uint32_t p0 = s_part[0][d], p1 = s_part[1][d], p2 = s_part[2][d], p3 = s_part[3][d];
     // Threads 0..255 come first in the block, so their exclusive scan is the digit start.
@@ -170,45 +222,23 @@ __global__ __launch_bounds__(1024) void k_rows_starts(uint32_t *bsum, uint32_t n
     if (q == 0) s_part[0][d] = start;
     __syncthreads();
     uint32_t run = s_part[0][d] + (q > 0 ? p0 : 0u) + (q > 1 ? p1 : 0u) + (q > 2 ? p2 : 0u);
-    b = b0;
-    for (; b + 8 <= b1; b += 8) {
-        uint32_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = col[(size_t)(b + u) * 256];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            col[(size_t)(b + u) * 256] = run;
-            run += v[u];
-        }
-    }
-    for (; b < b1; ++b) {
-        const uint32_t v = col[(size_t)b * 256];
-        col[(size_t)b * 256] = run;
-        run += v;
+    run = rows_write(col, b0, b1, v, run);
+    for (uint32_t b = b0 + kRowsU; b < b1; b += kRowsU) {
+        rows_batch(col, b, b1, v);
+        run = rows_write(col, b, b1, v, run);
     }
 }
 
 // rows[t][d] := output offset of the first digit-d key of tile t (in place).
 __global__ __launch_bounds__(256) void k_rows_apply(uint32_t *__restrict__ rows, uint32_t ntile, uint32_t span,
-                                                    const uint32_t *__restrict__ bsum) {
+                                                    const uint32_t *__restrict__ bsum,
+                                                    const uint32_t *__restrict__ sel = nullptr, int shift = 0) {
+    if (sel && !(radix_pass(*sel, shift) & kPassPlace)) return;
     const uint32_t t0 = blockIdx.x * span, t1 = std::min(ntile, t0 + span);
-    uint32_t *col = rows + threadIdx.x;
-    uint32_t run = bsum[(size_t)blockIdx.x * 256 + threadIdx.x];
-    uint32_t t = t0;
-    for (; t + 8 <= t1; t += 8) {
-        uint32_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = col[(size_t)(t + u) * 256];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            col[(size_t)(t + u) * 256] = run;
-            run += v[u];
-        }
-    }
-    for (; t < t1; ++t) {
-        const uint32_t v = col[(size_t)t * 256];
-        col[(size_t)t * 256] = run;
-        run += v;
+    uint32_t run = bsum[(size_t)blockIdx.x * 256 + threadIdx.x], v[kRowsU];
+    for (uint32_t t = t0; t < t1; t += kRowsU) {
+        rows_batch(rows + threadIdx.x, t, t1, v);
+        run = rows_write(rows + threadIdx.x, t, t1, v, run);
     }
 }
 
@@ -302,15 +332,44 @@ __global__ __launch_bounds__(256) void k_rows_apply_seg(uint32_t *__restrict__ r
 // Places global tile xcd_tile(blockIdx.x): ranks its keys by digit (stable),
 // stages them in LDS in digit order and writes each digit's run at the offset
 // from its row (plus, for a batch, the digit's start in the segment's output).
-template <bool HAS_VAL, bool UNPACK = false, bool MOD = false>
-__global__ __launch_bounds__(256) void k_radix_place(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+//
+// Without values four blocks fit a CU's LDS, so the registers are held to 128
+// (two spilled): 2^26 keys 246 -> 226 us per pass.
+//
+// DYN: *sel picks the pass (radix_pass).  FEW: at most kRowsFew tiles,
+// whose offsets the block works out from the counts itself instead of a scan
+// launch (100,000 keys in four passes 84 -> 76 us); the first pass then unites the
+// histogram's `diffs` too.
+template <bool HAS_VAL, bool UNPACK = false, bool MOD = false, bool DYN = false, bool FEW = false>
+__global__ __launch_bounds__(256, HAS_VAL || FEW ? 2 : 4) void k_radix_place(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                      uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
                                                      RadixSeg seg0, const RadixSeg *segs, int nseg, uint32_t ntile,
                                                      int shift, const uint32_t *__restrict__ offs,
                                                      const uint32_t *__restrict__ dstart, uint32_t sstride,
                                                      RowOut out0 = RowOut{}, const RowOut *outs = nullptr,
-                                                     const uint32_t *run_if = nullptr, uint32_t mod = 0) {
+                                                     const uint32_t *run_if = nullptr, uint32_t mod = 0,
+                                                     const uint32_t *__restrict__ sel = nullptr,
+                                                     const uint32_t *diffs = nullptr, uint32_t ndiff = 0,
+                                                     uint32_t *diff = nullptr) {
     if (run_if && *run_if == 0) return;  // gated off: runs only when *run_if != 0
+    uint32_t plan = kPassPlace;
+    if (DYN) {
+        if (FEW && diffs) {  // first pass: ndiff <= 64 words
+            uint32_t d = lane_id() < ndiff ? diffs[lane_id()] : 0u;
+#pragma unroll
+            for (int o = kWave / 2; o > 0; o >>= 1) d |= __shfl_xor(d, o, kWave);
+            if (blockIdx.x == 0 && threadIdx.x == 0) *diff = d;  // for the later passes
+            plan = radix_pass(d, shift);
+        } else {
+            plan = radix_pass(*sel, shift);
+        }
+        if ((plan & 255u) == 0) return;
+        if (plan >> 8) {  // the keys lie in kout: the pass goes the other way
+            const uint64_t *const t = kin;
+            kin = kout;
+            kout = const_cast<uint64_t *>(t);
+        }
+    }
     __shared__ uint32_t s_cnt[4][256];
     __shared__ uint32_t s_dpre[256];
     __shared__ uint32_t s_gofs[256];
@@ -325,6 +384,21 @@ __global__ __launch_bounds__(256) void k_radix_place(const uint64_t *__restrict_
     if (tb >= n) return;
     const uint32_t rem = (uint32_t)std::min<size_t>(kSortTile, n - tb);
     const uint64_t *ks = kin + sg.base + tb;
+    if (DYN && (plan & kPassCopy)) {
+        uint64_t *to = kout + sg.base + tb;
+        uint64_t c[kSortItems];
+#pragma unroll
+        for (int j = 0; j < kSortItems; ++j) {
+            const uint32_t i = (uint32_t)j * 256 + threadIdx.x;
+            c[j] = i < rem ? ks[i] : 0ull;
+        }
+#pragma unroll
+        for (int j = 0; j < kSortItems; ++j) {
+            const uint32_t i = (uint32_t)j * 256 + threadIdx.x;
+            if (i < rem) to[i] = c[j];
+        }
+        return;
+    }
     const uint32_t *vs = HAS_VAL ? vin + sg.base + tb : nullptr;
     for (int i = threadIdx.x; i < 1024; i += 256) (&s_cnt[0][0])[i] = 0;
     __syncthreads();
@@ -356,7 +430,21 @@ __global__ __launch_bounds__(256) void k_radix_place(const uint64_t *__restrict_
     {
         const unsigned d = threadIdx.x;
         const uint32_t c0 = s_cnt[0][d], c1 = s_cnt[1][d], c2 = s_cnt[2][d], c3 = s_cnt[3][d];
-        s_gofs[d] = offs[(size_t)t * 256 + d] + (dstart ? dstart[(size_t)si * sstride + d] : 0u);
+        if (FEW) {
+            // Keys of digit d in the tiles before this one, and in all of them.
+            uint32_t pre = 0, tot = 0;
+#pragma unroll 16
+            for (uint32_t u = 0; u < ntile; ++u) {
+                const uint32_t c = offs[(size_t)u * 256 + d];
+                pre += u < t ? c : 0u;
+                tot += c;
+            }
+            const uint32_t start = block_excl_scan256(tot, s_w);
+            __syncthreads();  // s_w is reused below
+            s_gofs[d] = start + pre;
+        } else {
+            s_gofs[d] = offs[(size_t)t * 256 + d] + (dstart ? dstart[(size_t)si * sstride + d] : 0u);
+        }
         s_dpre[d] = block_excl_scan256(c0 + c1 + c2 + c3, s_w);
         s_cnt[0][d] = 0;
         s_cnt[1][d] = c0;
@@ -402,6 +490,7 @@ __global__ __launch_bounds__(256) void k_radix_place(const uint64_t *__restrict_
 // Workspace of the reduce-then-scan passes over `tiles` tiles.
 struct RowsBufs {
     uint32_t *rows, *bsum;
+    uint32_t *diff = nullptr;  // sorts with the digits found out on the device
 };
 static RowsBufs rows_carve(uint32_t tiles, Carver &cv) {
     RowsBufs b;
@@ -449,6 +538,51 @@ static int launch_radix_rows(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uin
         std::swap(ksrc, kdst);
         std::swap(vsrc, vdst);
         *in_alt = !*in_alt;
+    }
+    return QO_OK;
+}
+
+// Digits in which all keys agree cost a sort by the high 32 bits nothing: 2^26
+// keys below 100 1.88 -> 0.74 ms, below 10,000 1.89 -> 1.00, below 10^6 1.76 ->
+// 1.45; keys over all 32 bits 1.78 -> 1.71.
+//
+// The passes of a sort by the high 32 bits with the digits found out on the
+// device (see radix_pass).  `diff`: a word and one per histogram block.
+static int launch_radix_rows_dyn(uint64_t *keys, uint64_t *kalt, const RadixSeg &sg, const RowsBufs &b, uint32_t *diff,
+                                 hipStream_t st) {
+    if (sg.ntile == 0) return QO_OK;
+    const RowsPlan rp = rows_plan(sg.ntile);
+    const unsigned hblocks = (sg.ntile + kHistTiles - 1) / kHistTiles;
+    uint32_t *diffs = diff + 1;  // one word per histogram block
+    for (int sh = 32; sh < 64; sh += 8) {
+        const bool first = sh == 32;
+        const uint32_t *from = first ? diffs : nullptr;
+        uint32_t *to = first ? diff : nullptr;
+        k_tile_hist<false, true><<<hblocks, 256, 0, st>>>(keys, sg, nullptr, 1, sg.ntile, sh, b.rows, nullptr, 0,
+                                                          diff, kalt, first ? diffs : nullptr);
+        QO_LAUNCHED();
+        if (sg.ntile <= kRowsFew) {
+            k_radix_place<false, false, false, true, true><<<sg.ntile, 256, 0, st>>>(
+                keys, nullptr, kalt, nullptr, sg, nullptr, 1, sg.ntile, sh, b.rows, nullptr, 0, RowOut{}, nullptr, nullptr,
+                0, diff, from, hblocks, to);
+            QO_LAUNCHED();
+            continue;
+        }
+        if (sg.ntile <= kRowsOneBlock) {
+            k_rows_starts<<<1, 1024, 0, st>>>(b.rows, sg.ntile, from, hblocks, to);
+            QO_LAUNCHED();
+        } else {
+            k_rows_reduce<<<rp.nb, 256, 0, st>>>(b.rows, sg.ntile, rp.span, b.bsum);
+            QO_LAUNCHED();
+            k_rows_starts<<<1, 1024, 0, st>>>(b.bsum, rp.nb, from, hblocks, to);
+            QO_LAUNCHED();
+            k_rows_apply<<<rp.nb, 256, 0, st>>>(b.rows, sg.ntile, rp.span, b.bsum, diff, sh);
+            QO_LAUNCHED();
+        }
+        k_radix_place<false, false, false, true><<<sg.ntile, 256, 0, st>>>(keys, nullptr, kalt, nullptr, sg, nullptr, 1,
+                                                                            sg.ntile, sh, b.rows, nullptr, 0, RowOut{},
+                                                                            nullptr, nullptr, 0, diff);
+        QO_LAUNCHED();
     }
     return QO_OK;
 }
@@ -577,6 +711,7 @@ static void radix_carve(size_t n, bool with_vals, Carver &cv, uint64_t **kalt, u
     *kalt = cv.take<uint64_t>(n ? n : 1);
     *valt = with_vals ? cv.take<uint32_t>(n ? n : 1) : nullptr;
     *rb = rows_carve(tiles, cv);
+    rb->diff = cv.take<uint32_t>(1 + (tiles + kHistTiles - 1) / kHistTiles);
     if (with_vals) {
         uint32_t *list = cv.take<uint32_t>(long_runs_cap(n));
         if (runs) *runs = list;
@@ -672,14 +807,16 @@ static int radix_impl(uint64_t *keys, uint32_t *vals, size_t n, const uint64_t *
     return QO_OK;
 }
 
-int launch_radix_sort_u64(uint64_t *keys, uint32_t *vals, size_t n, int lo_bit, int hi_bit, void *ws,
-                          hipStream_t st) {
-    return radix_impl(keys, vals, n, nullptr, lo_bit, hi_bit, ws, st);
-}
-
-int launch_radix_sort_u64_dev(uint64_t *keys, uint32_t *vals, const uint64_t *d_n, size_t capacity, int lo_bit,
-                              int hi_bit, void *ws, hipStream_t st) {
-    return radix_impl(keys, vals, capacity, d_n, lo_bit, hi_bit, ws, st);
+int launch_radix_sort_list(uint64_t *keys, const uint64_t *d_n, size_t n, void *ws, hipStream_t st) {
+    if (n <= kSmallSort) return radix_impl(keys, nullptr, n, d_n, 32, 64, ws, st);
+    QO_REQUIRE(n < 0xFFFFFFFFull, "sort input too large");
+    const uint32_t tiles = radix_tiles(n);
+    Carver cv(ws);
+    uint64_t *kalt = nullptr;
+    uint32_t *valt = nullptr;
+    RowsBufs rb{};
+    radix_carve(n, false, cv, &kalt, &valt, &rb);
+    return launch_radix_rows_dyn(keys, kalt, RadixSeg{0, n, d_n, 0, tiles}, rb, rb.diff, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -1198,7 +1335,7 @@ int qo_sort_records(qo_record *data, size_t n, qo_stream s) {
     void *ws = workspace(st, radix_workspace_bytes(n, false), &status);
     if (!ws) return status;
     // A Record {x, y} read as little-endian uint64 has y in bits 32..63.
-    return launch_radix_sort_u64(reinterpret_cast<uint64_t *>(data), nullptr, n, 32, 64, ws, st);
+    return launch_radix_sort_list(reinterpret_cast<uint64_t *>(data), nullptr, n, ws, st);
 }
 
 int qo_sort_join_rows(int32_t *key, int32_t *rpay, int32_t *spay, size_t m, qo_stream s) {

@@ -82,3 +82,16 @@ def test_group_merge_edges(qo, orc, groups, n):
     v = orc.gen_uniform_u32(n, 9, 1, 0, 0).astype(np.int32)
     for g, e in zip(qo.operators.groupby_agg(k, v, groups), orc.groupby_agg(k, v)):
         assert np.array_equal(g, e)
+
+
+@pytest.mark.parametrize("mask", [0x0, 0xFF, 0xFF00, 0xFFFFF, 0xFF00FF00, 0xFF0000FF, 0xFF000000, 0xFFFFFFFF])
+@pytest.mark.parametrize("n", [8193, 70001, (1 << 20) + 4097])
+def test_sort_records_skips_equal_digits(qo, orc, n, mask):
+    """Keys that vary in some digits only: zero to four passes, ending in either buffer; aligned and not."""
+    y = orc.gen_uniform_u32(n + 1, 10, 2, 0, 0) & np.uint32(mask) | np.uint32(0x01020304 & ~mask)
+    rec = np.stack([np.arange(n + 1, dtype=np.uint32), y], 1)
+    assert np.array_equal(qo.operators.sort_records(rec[:n]), orc.sort_records(rec[:n]))
+    with qo.device.DeviceBuffer.from_numpy(rec) as d:  # records at an 8-byte offset
+        qo._lib.call("qo_sort_records", d.ptr + 8, n, None)
+        got = d.to_numpy(np.uint32, 2 * n + 2).reshape(-1, 2)
+    assert np.array_equal(got[1:], orc.sort_records(rec[1:])) and np.array_equal(got[0], rec[0])
