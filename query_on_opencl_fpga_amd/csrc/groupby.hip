@@ -1351,87 +1351,119 @@ __global__ void k_agg_chunks(const int32_t *startPos, uint32_t G, size_t n, uint
 
 QO_DEV int32_t agg_identity(int op) { return op == QO_REDUCE_MIN ? (1 << 30) : 0; }
 
-// Owner group of every work unit below umax: units [cofs[g], cofs[g] +
-// chunks[g]) belong to group g (one thread per group writes its units).
-__global__ void k_agg_units(const uint32_t *cofs, const uint32_t *chunks, uint32_t G, uint32_t *unit_group,
-                            uint32_t umax) {
-    const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= G) return;
-    for (uint32_t q = 0; q < chunks[g] && cofs[g] + q < umax; ++q) unit_group[cofs[g] + q] = (uint32_t)g;
-}
-
-// Group of work unit w: from the owner table, or, for units past it (start
-// positions that overlap, which only a malformed input produces), the last g
-// with cofs[g] <= w.  An empty group shares its cofs with the following group,
-// so the last such g is the non-empty group that owns unit w.
-QO_DEV uint32_t unit_owner(const uint32_t *unit_group, uint32_t umax, const uint32_t *cofs, uint32_t G, size_t w) {
-    if (w < umax) return unit_group[w];
-    uint32_t lo = 0, hi = G - 1;
-    while (lo < hi) {
-        uint32_t mid = (lo + hi + 1) >> 1;
-        if (cofs[mid] <= w) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// kAggLanes lanes per work unit, kWave / kAggLanes units per wave at once:
-// each lane reduces every kAggLanes-th row of its unit (all its loads issued
-// before any is used), the unit's lanes combine by shuffles, and the first
-// lane stores the result of a group that is one unit or merges a partial
-// with an atomic.  `acc` holds the identity beforehand.  With one wave per
-// 512-row unit, groups of ~64 rows left each wave mostly waiting on its
-// unit's index loads and atomic (0.32 ms per aggregate over 2^26 Records).
+// kAggLanes lanes per work unit, kWave / kAggLanes units per wave at once, each
+// group of lanes walking a contiguous range of units: a lane reduces every
+// kAggLanes-th row of a unit (all its loads issued before any is used) and keeps
+// its partial while the group stays the same; where the group changes the lanes
+// combine by shuffles, and the first lane stores the result of a group that is
+// one unit or merges a partial with an atomic.  What the lanes hold at the end is
+// combined over the wave and the block first where it is one group's.  `acc`
+// holds the identity beforehand.  Bound by the row loads: 2^26 Records in 16
+// groups 98 us (5.5 TB/s).  With a table of every unit's group, written by a thread
+// per group, and one atomic per unit, few groups left the chip to a few threads and
+// the atomics to a few addresses: the chain from copy to sums over 2^26 Records
+// 113 ms with one group, 5.4 ms with 109, 2.24 with 20,000; now 0.86, 1.14 and 1.29.
 __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict__ s, size_t n,
                                                     const int32_t *__restrict__ startPos, uint32_t G,
                                                     const uint32_t *__restrict__ cofs, const uint32_t *__restrict__ chunks,
-                                                    const uint32_t *__restrict__ unit_group, uint32_t umax, int op,
-                                                    int32_t *acc) {
+                                                    int op, int32_t *acc) {
     constexpr int kPerLane = kAggChunk / kAggLanes;
-    constexpr int kUnitsPerWave = kWave / kAggLanes;
+    constexpr uint32_t kUnitsPerWave = kWave / kAggLanes;
+    constexpr uint32_t kNone = ~0u;
+    constexpr int kWaves = 256 / kWave;
+    __shared__ uint32_t s_cur[kWaves];
+    __shared__ int32_t s_val[kWaves];
     const uint32_t total = cofs[G - 1] + chunks[G - 1];
+    if (total == 0) return;  // the whole grid
     const unsigned lane = lane_id(), sub = lane / kAggLanes, sl = lane % kAggLanes;
-    const size_t waves = (size_t)gridDim.x * (blockDim.x / kWave);
-    for (size_t w0 = ((size_t)blockIdx.x * (blockDim.x / kWave) + wave_id()) * kUnitsPerWave; w0 < total;
-         w0 += waves * kUnitsPerWave) {
-        const size_t w = w0 + sub;
-        const bool active = w < total;
-        uint32_t g = 0;
+    const size_t subs = (size_t)gridDim.x * kWaves * kUnitsPerWave;
+    const size_t per = (total + subs - 1) / subs;
+    const size_t w0 = (((size_t)blockIdx.x * kWaves + wave_id()) * kUnitsPerWave + sub) * per;
+    auto merge = [&](int32_t a, int32_t b) {
+        if (op == QO_REDUCE_MAX) return a > b ? a : b;
+        if (op == QO_REDUCE_MIN) return a < b ? a : b;
+        return (int32_t)((uint32_t)a + (uint32_t)b);
+    };
+    auto emit = [&](uint32_t g, int32_t l) {
+        if (chunks[g] == 1) acc[g] = l;  // the group's only unit: its result is final
+        else if (op == QO_REDUCE_MAX) atomicMax(&acc[g], l);
+        else if (op == QO_REDUCE_MIN) atomicMin(&acc[g], l);
+        else atomicAdd(reinterpret_cast<uint32_t *>(&acc[g]), (uint32_t)l);
+    };
+    // The group of the first unit is the last one with cofs <= w0 (it has units:
+    // cofs of a group without is the next one's), found kAggLanes probes at a time.
+    uint32_t next = 0;
+    {
+        const uint32_t w = w0 < total ? (uint32_t)w0 : total - 1;
+        uint32_t len = G;
+        while (ballot(len > 1)) {
+            const uint32_t step = (len + kAggLanes - 1) / kAggLanes, at = sl * step;
+            const uint64_t le = ballot(at < len && (sl == 0 || cofs[next + at] <= w));
+            const uint32_t k = __popcll((le >> (sub * kAggLanes)) & ((1u << kAggLanes) - 1)) - 1;
+            next += k * step;
+            len = min(step, len - k * step);
+        }
+    }
+    uint32_t cur = kNone;
+    int32_t local = agg_identity(op);
+    size_t gw = 0, gend = 0;    // units of the group in hand
+    int64_t gs = 0, ge = 0;     // its rows
+    uint32_t g = kNone;
+    for (size_t i = 0; i < per; ++i) {
+        const size_t w = w0 + i;
         int64_t a = 0, b = 0;
-        if (active) {
-            g = unit_owner(unit_group, umax, cofs, G, w);
-            int64_t gs, ge;
-            group_range(startPos, g, G, n, gs, ge);
-            a = gs + (int64_t)(w - cofs[g]) * kAggChunk;
+        if (w < total) {
+            while (w >= gend && next < G) {
+                g = next++;
+                gw = cofs[g];
+                gend = gw + chunks[g];
+                group_range(startPos, g, G, n, gs, ge);
+            }
+            a = gs + (int64_t)(w - gw) * kAggChunk;
             b = a + kAggChunk < ge ? a + kAggChunk : ge;
         }
         int32_t v[kPerLane];
 #pragma unroll
         for (int k = 0; k < kPerLane; ++k) {
-            const int64_t i = a + sl + (int64_t)k * kAggLanes;
-            v[k] = i < b ? (int32_t)s[i].x : agg_identity(op);
+            const int64_t r = a + sl + (int64_t)k * kAggLanes;
+            v[k] = r < b ? (int32_t)s[r].x : agg_identity(op);
         }
-        int32_t local = agg_identity(op);
-        uint32_t usum = 0;
+        const bool change = cur != kNone && g != cur;
+        if (ballot(change)) {
+            int32_t l = local;
+            // Xor offsets below kAggLanes stay inside the unit's lanes.
 #pragma unroll
-        for (int k = 0; k < kPerLane; ++k) {
-            if (op == QO_REDUCE_MAX) local = v[k] > local ? v[k] : local;
-            else if (op == QO_REDUCE_MIN) local = v[k] < local ? v[k] : local;
-            else usum += (uint32_t)v[k];
+            for (int o = kAggLanes / 2; o > 0; o >>= 1) l = merge(l, __shfl_xor(l, o, kWave));
+            if (change) {
+                if (sl == 0) emit(cur, l);
+                local = agg_identity(op);
+            }
         }
-        // Combine the unit's lanes (xor offsets below kAggLanes stay inside the unit).
+        cur = g;
 #pragma unroll
-        for (int o = kAggLanes / 2; o > 0; o >>= 1) {
-            if (op == QO_REDUCE_MAX) local = max(local, __shfl_xor(local, o, kWave));
-            else if (op == QO_REDUCE_MIN) local = min(local, __shfl_xor(local, o, kWave));
-            else usum += __shfl_xor(usum, o, kWave);
+        for (int k = 0; k < kPerLane; ++k) local = merge(local, v[k]);
+    }
+#pragma unroll
+    for (int o = kAggLanes / 2; o > 0; o >>= 1) local = merge(local, __shfl_xor(local, o, kWave));
+    const uint32_t c0 = __shfl(cur, 0, kWave);
+    const bool one = ballot(cur != c0) == 0;  // the wave's lanes all hold group c0 (or nothing)
+    if (one) {
+#pragma unroll
+        for (int o = kAggLanes; o < kWave; o <<= 1) local = merge(local, __shfl_xor(local, o, kWave));
+    } else if (sl == 0 && cur != kNone) {
+        emit(cur, local);
+    }
+    if (lane == 0) {
+        s_cur[wave_id()] = one ? c0 : kNone;
+        s_val[wave_id()] = local;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 0; k < kWaves; ++k) {
+            if (s_cur[k] == kNone) continue;
+            if (k + 1 < kWaves && s_cur[k + 1] == s_cur[k]) s_val[k + 1] = merge(s_val[k], s_val[k + 1]);
+            else emit(s_cur[k], s_val[k]);
         }
-        if (!active || sl != 0) continue;
-        if (op != QO_REDUCE_MAX && op != QO_REDUCE_MIN) local = (int32_t)usum;
-        if (chunks[g] == 1) acc[g] = local;  // the group's only unit: its result is final
-        else if (op == QO_REDUCE_MAX) atomicMax(&acc[g], local);
-        else if (op == QO_REDUCE_MIN) atomicMin(&acc[g], local);
-        else atomicAdd(reinterpret_cast<uint32_t *>(&acc[g]), usum);
     }
 }
 
@@ -1445,11 +1477,8 @@ __global__ void k_agg_average(const int32_t *startPos, uint32_t G, size_t n, con
     out[g] = cnt > 0 ? sum[g] / cnt : 0;
 }
 
-// Work units: at most one partial 512-row chunk per group beyond n / 512 full ones.
-static size_t agg_units_max(size_t n, size_t G) { return n / kAggChunk + G + 1; }
-
-size_t aggregate_ws_bytes(size_t G, size_t n) {
-    return G * 12 + agg_units_max(n, G) * 4 + scan_workspace_bytes(G) + 2048;
+size_t aggregate_ws_bytes(size_t G) {
+    return G * 12 + scan_workspace_bytes(G) + 2048;
 }
 
 int launch_aggregate_groups(const qo_record *s, size_t n, const int32_t *startPos, size_t G, int op, int32_t *out,
@@ -1459,7 +1488,6 @@ int launch_aggregate_groups(const qo_record *s, size_t n, const int32_t *startPo
     uint32_t *chunks = cv.take<uint32_t>(G);
     uint32_t *cofs = cv.take<uint32_t>(G);
     int32_t *sum = cv.take<int32_t>(G);
-    uint32_t *unit_group = cv.take<uint32_t>(agg_units_max(n, G));
     void *sws = cv.take<char>(scan_workspace_bytes(G));
     int32_t *acc = op == QO_REDUCE_AVERAGE ? sum : out;
     QO_TRY(launch_fill_u32(acc, op == QO_REDUCE_MIN ? (1u << 30) : 0u, G, st));
@@ -1467,12 +1495,8 @@ int launch_aggregate_groups(const qo_record *s, size_t n, const int32_t *startPo
     k_agg_chunks<<<gb, 256, 0, st>>>(startPos, (uint32_t)G, n, chunks);
     QO_LAUNCHED();
     QO_TRY(launch_scan_excl_u32(chunks, cofs, G, sws, st));
-    const size_t umax = std::min<size_t>(agg_units_max(n, G), 0xFFFFFFFFull);
-    k_agg_units<<<gb, 256, 0, st>>>(cofs, chunks, (uint32_t)G, unit_group, (uint32_t)umax);
-    QO_LAUNCHED();
     const unsigned grid = grid_for((size_t)n / kAggChunk + G, 4 * (kWave / kAggLanes), (unsigned)props().cu_count * 16);
-    k_agg_groups<<<grid, 256, 0, st>>>(s, n, startPos, (uint32_t)G, cofs, chunks, unit_group, (uint32_t)umax, op,
-                                       acc);
+    k_agg_groups<<<grid, 256, 0, st>>>(s, n, startPos, (uint32_t)G, cofs, chunks, op, acc);
     QO_LAUNCHED();
     if (op == QO_REDUCE_AVERAGE) {
         k_agg_average<<<gb, 256, 0, st>>>(startPos, (uint32_t)G, n, sum, out);
@@ -1552,7 +1576,7 @@ int qo_aggregate_groups(const qo_record *sorted, size_t n, const int32_t *startP
     QO_REQUIRE(sorted && startPos && out && numGroups < 0xFFFFFFFFull, "bad aggregate arguments");
     hipStream_t st = stream_of(s);
     int status = QO_OK;
-    void *ws = workspace(st, aggregate_ws_bytes(numGroups, n), &status);
+    void *ws = workspace(st, aggregate_ws_bytes(numGroups), &status);
     if (!ws) return status;
     return launch_aggregate_groups(sorted, n, startPos, numGroups, op, out, ws, st);
 }
