@@ -1285,26 +1285,34 @@ __global__ __launch_bounds__(NT) void k_group_startpos(const qo_record *__restri
     const size_t ebase = (size_t)tile * kTile;
     const qo_record *src = s + ebase;
     const uint32_t rem = (uint32_t)min((size_t)kTile, n - ebase);
-    uint32_t fl[J], c[J], ex[J];
+    uint32_t fl[J], c[J], ex[J], y[J][V], edge[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
         const uint32_t e0 = ((uint32_t)j * NT + threadIdx.x) * V;
-        uint32_t y[V];
-        uint32_t prev = 0;
-        fl[j] = 0;
+        edge[j] = 0;
+#pragma unroll
+        for (int k = 0; k < V; ++k) y[j][k] = 0;
         if (e0 < rem) {
             if (VEC && e0 + 2 <= rem) {
                 const uint4 q = ld_stream(reinterpret_cast<const uint4 *>(src) + (e0 >> 1));
-                y[0] = q.y;
-                y[V - 1] = q.w;
+                y[j][0] = q.y;
+                y[j][V - 1] = q.w;
             } else {
 #pragma unroll
-                for (int k = 0; k < V; ++k) y[k] = e0 + k < rem ? src[e0 + k].y : 0u;
+                for (int k = 0; k < V; ++k) y[j][k] = e0 + k < rem ? src[e0 + k].y : 0u;
             }
-            const bool first = ebase + e0 == 0;
-            if (!first) prev = src[(int64_t)e0 - 1].y;
-            fl[j] = (first || y[0] != prev) ? 1u : 0u;
-            if (V == 2 && e0 + 1 < rem && y[V - 1] != y[0]) fl[j] |= 2u;
+            if (lane_id() == 0 && ebase + e0 != 0) edge[j] = src[(int64_t)e0 - 1].y;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const uint32_t e0 = ((uint32_t)j * NT + threadIdx.x) * V;
+        const uint32_t up = __shfl_up(y[j][V - 1], 1, kWave);
+        const uint32_t prev = lane_id() == 0 ? edge[j] : up;
+        fl[j] = 0;
+        if (e0 < rem) {
+            fl[j] = (ebase + e0 == 0 || y[j][0] != prev) ? 1u : 0u;
+            if (V == 2 && e0 + 1 < rem && y[j][V - 1] != y[j][0]) fl[j] |= 2u;
         }
         c[j] = __popc(fl[j]);
     }
