@@ -147,6 +147,53 @@ QO_DEV T tile_offsets(const T (&c)[J], T (&excl)[J], T *s_tot) {
     return s_tot[K];
 }
 
+// tile_offsets of the set bits of fl (bit k: element k of the lane's V), counted
+// by ballots: the exclusive in-tile rank of each lane's first element.
+template <int J, int NW, int V>
+QO_DEV uint32_t flag_offsets(const uint32_t (&fl)[J], uint32_t (&excl)[J], uint32_t *s_tot) {
+    constexpr int K = J * NW;
+    constexpr int P = (K + kWave - 1) / kWave;
+    const unsigned w = wave_id();
+    const unsigned lane = lane_id();
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        uint32_t tot = 0;
+        excl[j] = 0;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            const uint64_t m = ballot((fl[j] >> k) & 1u);
+            excl[j] += __popcll(m & below);
+            tot += __popcll(m);
+        }
+        if (lane == 0) s_tot[j * NW + w] = tot;
+    }
+    __syncthreads();
+    if (w == 0) {
+        uint32_t v[P];
+        uint32_t sum = 0;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const unsigned idx = lane * P + p;
+            v[p] = idx < (unsigned)K ? s_tot[idx] : 0u;
+            sum += v[p];
+        }
+        const uint32_t inc = wave_incl_scan(sum);
+        uint32_t run = inc - sum;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const unsigned idx = lane * P + p;
+            if (idx < (unsigned)K) s_tot[idx] = run;
+            run += v[p];
+        }
+        if (lane == kWave - 1) s_tot[K] = inc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < J; ++j) excl[j] += s_tot[j * NW + w];
+    return s_tot[K];
+}
+
 // Decoupled look-back status word: [63:62] flag (0 empty, 1 aggregate,
 // 2 inclusive prefix), [61:0] value.
 constexpr uint64_t kFlagAgg = uint64_t(1) << 62;
