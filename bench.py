@@ -430,7 +430,7 @@ def run_ops(args, qo, lib) -> dict:
     ms_copy = _time_op(st, args.steps, args.warmup,
                        lambda: qo._lib.call("qo_copy", work.ptr, src.ptr, ns * 8, st.handle))
     ms = _time_op(st, args.steps, args.warmup, sort_once) - ms_copy
-    row("sort_records (LSD radix on .y, 4 passes; the copy restoring the input is subtracted)", ns, ms,
+    row("sort_records (LSD radix on .y, at most 4 passes; the copy restoring the input is subtracted)", ns, ms,
         16 * ns, "8*N read + 8*N written")
     sp = DeviceBuffer(ns * 4)
     num = DeviceBuffer(8)

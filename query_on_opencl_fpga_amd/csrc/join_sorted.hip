@@ -24,7 +24,8 @@
 // Whole calls, generic path -> this one: 2^28 S rows, half selected, 2^24 dense
 // build keys 5.64 -> 2.40 ms (split 0.96, second split 0.55, finish 0.64, build
 // 0.2); 12,000,008 S rows, half selected, 1,500,001 spread 31-bit keys 684 ->
-// 352 us; 16384 S rows, half selected, 4096 spread keys 204 -> 125 us.
+// 370 us; 16384 S rows, half selected, 4096 spread keys 204 -> 125 us (88 with the
+// table built by one work-group).
 #include <algorithm>
 #include <cmath>
 
