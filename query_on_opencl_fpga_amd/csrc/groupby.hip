@@ -198,6 +198,60 @@ QO_DEV void ltable_add(LTable<C> &L, int32_t k, int32_t v, int probes, GEntry *g
     }
 }
 
+// k_groupby_hash's table: a tuple adds to COUNT and SUM with one LDS atomic on
+// pack = COUNT << 48 | sum of (value + 2^31), since two that queue on few groups'
+// addresses bound the kernel (2^28 tuples, 16 groups 536 -> 457 us; 1024 with Zipf
+// sizes 527 -> 467; 1024 even 387 -> 370; 100 groups 423 -> 429).  Every add returns
+// the word it found: a thread that found COUNT >= 2^15 empties the word into cnt
+// and sum before its next add, so at most one add per thread of the block comes on
+// top, and neither field overflows.  The small table, whose inputs are small, does
+// without (100 K tuples: 21.8 us, 22.5 with the word), and so does k_groupby_chunks,
+// whose keys are many (no gain).
+template <int C>
+struct PackTable {
+    static constexpr bool kPacked = C > 2048;
+    LTable<C> t;
+    unsigned long long pack[kPacked ? C : 1];
+};
+
+// The thread's last add: the upper half of the word it found, and its slot.
+struct PackSeen {
+    uint32_t hi = 0;
+    int slot = 0;
+};
+
+template <int C>
+QO_DEV void pack_empty(PackTable<C> &L, int s, unsigned long long w) {
+    const uint32_t c = (uint32_t)(w >> 48);
+    atomicAdd(&L.t.cnt[s], c);
+    atomicAdd(&L.t.sum[s], (w & ((1ull << 48) - 1)) - ((unsigned long long)c << 31));
+}
+
+template <int C>
+QO_DEV void pack_add(PackTable<C> &L, int32_t k, int32_t v, int probes, GEntry *gt, uint64_t gmask,
+                     uint32_t *overflow, PackSeen &seen) {
+    if constexpr (!PackTable<C>::kPacked) {
+        ltable_add<C>(L.t, k, v, probes, gt, gmask, overflow);
+        return;
+    }
+    if (seen.hi >= 1u << 31) {
+        pack_empty(L, seen.slot, atomicExch(&L.pack[seen.slot], 0ull));
+        seen.hi = 0;
+    }
+    const int s = (uint32_t)k == kEmptyKey ? -1 : l_slot<C>(L.t.key, (uint32_t)k, probes, 0);
+    if (s >= 0) {
+        const int32_t lo = L.t.mn[s], hi = L.t.mx[s];  // read first, as in ltable_add
+        const unsigned long long old =
+            atomicAdd(&L.pack[s], (1ull << 48) + (unsigned long long)((uint32_t)v ^ 0x80000000u));
+        seen.hi = (uint32_t)(old >> 32);
+        seen.slot = s;
+        if (v < lo) atomicMin(&L.t.mn[s], v);
+        if (v > hi) atomicMax(&L.t.mx[s], v);
+    } else {
+        g_update(gt, gmask, (uint32_t)k, 1, (uint64_t)(int64_t)v, v, v, overflow);
+    }
+}
+
 // Merges the block's LDS partials into the global table (after a barrier).
 // Block b walks its slots starting at (97 b) mod C, so blocks that finish
 // together update different global entries instead of queueing on the same
@@ -461,7 +515,8 @@ __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__
                                                       const int32_t *__restrict__ filt = nullptr, int32_t flo = 0,
                                                       int32_t fhi = 0) {
     extern __shared__ unsigned char s_raw[];
-    LTable<C> &L = *reinterpret_cast<LTable<C> *>(s_raw);
+    PackTable<C> &P = *reinterpret_cast<PackTable<C> *>(s_raw);
+    LTable<C> &L = P.t;
     __shared__ uint32_t s_dom, s_dom2, s_heavy;
     if (threadIdx.x < kWave) {
         unsigned bc, bc2;
@@ -475,15 +530,18 @@ __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__
         }
     }
     ltable_init<C>(L);
+    if constexpr (PackTable<C>::kPacked)
+        for (int i = threadIdx.x; i < C; i += NT) P.pack[i] = 0;
     __syncthreads();
     const uint32_t dom = s_dom, dom2 = s_dom2;
+    PackSeen seen;
     auto body = [&](auto heavy_tag) {
         constexpr bool kHeavy = decltype(heavy_tag)::value;
         DomAcc acc, acc2;
         auto add_one = [&](int32_t k, int32_t v) {
             if (kHeavy && (uint32_t)k == dom) acc.add(v);
             else if (kHeavy && (uint32_t)k == dom2) acc2.add(v);
-            else ltable_add<C>(L, k, v, probes, gt, gmask, overflow);
+            else pack_add<C>(P, k, v, probes, gt, gmask, overflow, seen);
         };
         auto add = [&](int32_t k, int32_t v, int32_t f) {
             if (!FILT || (f >= flo && f <= fhi)) add_one(k, v);
@@ -537,6 +595,11 @@ __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__
     if (s_heavy) body(std::true_type{});
     else body(std::false_type{});
     __syncthreads();
+    if constexpr (PackTable<C>::kPacked) {
+        for (int i = threadIdx.x; i < C; i += NT)
+            if (P.pack[i]) pack_empty(P, i, P.pack[i]);
+        __syncthreads();
+    }
     if (parts.ent) ltable_partials<C, NT>(L, parts);
     else ltable_flush<C>(L, gt, gmask, overflow);
 }
@@ -1078,7 +1141,10 @@ static GbPartPlan groupby_part_plan(size_t group_capacity, size_t n, bool filter
     GbPartPlan p;
     const TuneParams tp = tune_get(TUNE_GROUPBY_PART, n);
     if (tp.param == PART_NEVER || n == 0 || n >= 0xFFFFFFFFull || group_capacity < 2) return p;
-    if (tp.param != PART_ALWAYS && (group_capacity <= 1024 || n < (size_t(1) << 20))) return p;
+    // Up to kGroupbyDirect groups one LDS table of 4096 slots holds them all and no
+    // tuple moves: 2^28 tuples, 2000 groups 2247 -> 382 us, 3000 groups 1911 -> 759;
+    // 2^20 tuples, 2000 groups 268 -> 56.
+    if (tp.param != PART_ALWAYS && (group_capacity <= kGroupbyDirect || n < (size_t(1) << 20))) return p;
     const size_t target = (size_t)std::max(16, tp.items);
     const int lmax = filtered ? __builtin_ctz(kOnePassParts) : 2 * kMaxSplitBits;
     int L = 1;
@@ -1120,7 +1186,8 @@ static unsigned merge_min_blocks(size_t groups) { return groups < 1600 ? 76u - (
 static HashPlan hash_plan(size_t n, size_t groups) {
     HashPlan h;
     const TuneParams tp = tune_get(TUNE_GROUPBY, n);
-    h.C = tp.items >= 4096 && (size_t)props().lds_per_block >= sizeof(LTable<4096>) ? 4096 : 2048;
+    const bool large = tp.items >= 4096 || (groups > 1024 && groups <= kGroupbyDirect && n >= (size_t(1) << 20));
+    h.C = large && (size_t)props().lds_per_block >= sizeof(PackTable<4096>) + 8192 ? 4096 : 2048;
     h.grid = grid_for(n, kHashThreads * 4, (unsigned)props().cu_count * (unsigned)std::max(1, tp.param));
     h.merge = h.grid >= merge_min_blocks(groups) && h.grid <= kMergeMaxBlocks && n < 0xFFFFFFFFull;
     return h;
@@ -1206,9 +1273,9 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
         const unsigned grid = h.grid;
         // Low cardinality: the LDS table holds every group.  High cardinality:
         // it caches the keys seen first and the rest go straight to global.
-        const int probes = group_capacity * 2 <= (size_t)C ? C : 8;
+        const int probes = group_capacity * 4 <= (size_t)C * 3 ? C : 8;
 #define QO_GBH(CC, V, F)                                                                                    \
-    k_groupby_hash<CC, V, block, F><<<grid, block, sizeof(LTable<CC>), st>>>(key, val, n, gt, p.gmask, probes,  \
+    k_groupby_hash<CC, V, block, F><<<grid, block, sizeof(PackTable<CC>), st>>>(key, val, n, gt, p.gmask, probes, \
                                                                              overflow, b.parts, filt, flo, fhi)
         if (C == 4096) {
             if (filt) {

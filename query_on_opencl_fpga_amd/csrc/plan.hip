@@ -134,7 +134,7 @@ static int tune_op_of(int impl, const qo_query &q, double m) {
         case QO_IMPL_SORT_GROUP_AGG: return TUNE_SORT;
         case QO_IMPL_HASH_GROUP_AGG:
         case QO_IMPL_FILTER_HASH_GROUP_AGG:
-            return std::min(q.groups, std::max(m, 1.0)) <= 1024.0 ? TUNE_GROUPBY : TUNE_GROUPBY_PART;
+            return std::min(q.groups, std::max(m, 1.0)) <= (double)kGroupbyDirect ? TUNE_GROUPBY : TUNE_GROUPBY_PART;
         default: return -1;
     }
 }
