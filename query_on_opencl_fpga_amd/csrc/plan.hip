@@ -46,10 +46,10 @@ static PrimCost g_cost[QO_COST_NUM] = {
     {12.0, 3300.0},  // QO_COST_STARTPOS: group start positions, 8 B per row
     {28.0, 850.0},   // QO_COST_AGG: one per-group aggregate, 8 B per row (1024 groups)
     {6.0, 5000.0},   // QO_COST_UNPACK: Records -> columns (or a Record copy), 16 B per row
-    {81.0, 3400.0},  // QO_COST_HASH_SMALL: hash group-by, at most 1024 groups, 8 B per row
+    {81.0, 3400.0},  // QO_COST_HASH_SMALL: hash group-by, direct (at most kGroupbyDirect groups), 8 B per row
     {245.0, 1260.0}, // QO_COST_HASH_LARGE: hash group-by, more groups (partitioned), 8 B per row
     {10.0, 6300.0},  // QO_COST_REDUCE: no-group reduce, 8 B per row
-    {75.0, 3960.0},  // QO_COST_FHASH_SMALL: filtered hash group-by (half selected), <= 1024 groups
+    {75.0, 3960.0},  // QO_COST_FHASH_SMALL: filtered hash group-by (half selected), direct
     {222.0, 1300.0}, // QO_COST_FHASH_LARGE: filtered hash group-by (half selected), more groups
 };
 static std::mutex g_cost_mu;
@@ -102,7 +102,7 @@ static int covers(int impl, const Chain &c, int first) {
 // the caller's Records (copied before an in-place sort).
 static double impl_ms(int impl, const qo_query &q, double m, bool owns_input) {
     const double G = std::max(1.0, std::min(q.groups, std::max(m, 1.0)));
-    const int hash = G <= 1024.0 ? QO_COST_HASH_SMALL : QO_COST_HASH_LARGE;
+    const int hash = G <= (double)kGroupbyDirect ? QO_COST_HASH_SMALL : QO_COST_HASH_LARGE;
     switch (impl) {
         case QO_IMPL_FILTER: return prim_ms(QO_COST_FILTER, 8 * m + 8 * m * q.selectivity);
         case QO_IMPL_SORT_GROUP_AGG: {
@@ -117,7 +117,7 @@ static double impl_ms(int impl, const qo_query &q, double m, bool owns_input) {
             // selected ones only: time taken as linear in the selectivity s
             // between the measured filtered group-by (s = 1/2) and the plain
             // one (s = 1), and never below the filtered one's fixed cost.
-            const int fhash = G <= 1024.0 ? QO_COST_FHASH_SMALL : QO_COST_FHASH_LARGE;
+            const int fhash = G <= (double)kGroupbyDirect ? QO_COST_FHASH_SMALL : QO_COST_FHASH_LARGE;
             const double t1 = prim_ms(hash, 8 * m + 64 * G), th = prim_ms(fhash, 8 * m + 64 * G);
             const double t = std::max(g_cost[fhash].fixed_us * 1e-3, t1 + 2.0 * (1.0 - q.selectivity) * (th - t1));
             return prim_ms(QO_COST_UNPACK, 16 * m) + t;
