@@ -181,7 +181,9 @@ QO_DEV uint32_t rows_write(uint32_t *col, uint32_t t, uint32_t t1, const uint32_
 
 // bsum[b * 256 + d] = digit-d keys of the tiles of block b.
 __global__ __launch_bounds__(256) void k_rows_reduce(const uint32_t *__restrict__ rows, uint32_t ntile, uint32_t span,
-                                                     uint32_t *__restrict__ bsum) {
+                                                     uint32_t *__restrict__ bsum,
+                                                     const uint32_t *__restrict__ sel = nullptr, int shift = 0) {
+    if (sel && !(radix_pass(*sel, shift) & kPassPlace)) return;
     const uint32_t t0 = blockIdx.x * span, t1 = std::min(ntile, t0 + span);
     uint32_t sum = 0, v[kRowsU];
     for (uint32_t t = t0; t < t1; t += kRowsU) sum += rows_batch(rows + threadIdx.x, t, t1, v);
@@ -194,7 +196,9 @@ __global__ __launch_bounds__(256) void k_rows_reduce(const uint32_t *__restrict_
 // of a sort with the digits found out on the device: *diff := the union of the
 // ndiff words at `diffs`.
 __global__ __launch_bounds__(1024) void k_rows_starts(uint32_t *bsum, uint32_t nb, const uint32_t *diffs = nullptr,
-                                                      uint32_t ndiff = 0, uint32_t *diff = nullptr) {
+                                                      uint32_t ndiff = 0, uint32_t *diff = nullptr,
+                                                      const uint32_t *__restrict__ sel = nullptr, int shift = 0) {
+    if (sel && !(radix_pass(*sel, shift) & kPassPlace)) return;
     __shared__ uint32_t s_part[4][256];
     __shared__ uint32_t s_w[16];
     __shared__ uint32_t s_diff;
@@ -543,8 +547,8 @@ static int launch_radix_rows(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uin
 }
 
 // Digits in which all keys agree cost a sort by the high 32 bits nothing: 2^26
-// keys below 100 1.88 -> 0.74 ms, below 10,000 1.89 -> 1.00, below 10^6 1.76 ->
-// 1.45; keys over all 32 bits 1.78 -> 1.71.
+// keys below 100 1.88 -> 0.72 ms, below 10,000 1.89 -> 0.98, below 10^6 1.76 ->
+// 1.44; keys over all 32 bits 1.78 -> 1.71.
 //
 // The passes of a sort by the high 32 bits with the digits found out on the
 // device (see radix_pass).  `diff`: a word and one per histogram block.
@@ -558,6 +562,7 @@ static int launch_radix_rows_dyn(uint64_t *keys, uint64_t *kalt, const RadixSeg 
         const bool first = sh == 32;
         const uint32_t *from = first ? diffs : nullptr;
         uint32_t *to = first ? diff : nullptr;
+        const uint32_t *sel = first ? nullptr : diff;  // later column scans are skipped with their pass
         k_tile_hist<false, true><<<hblocks, 256, 0, st>>>(keys, sg, nullptr, 1, sg.ntile, sh, b.rows, nullptr, 0,
                                                           diff, kalt, first ? diffs : nullptr);
         QO_LAUNCHED();
@@ -569,12 +574,12 @@ static int launch_radix_rows_dyn(uint64_t *keys, uint64_t *kalt, const RadixSeg 
             continue;
         }
         if (sg.ntile <= kRowsOneBlock) {
-            k_rows_starts<<<1, 1024, 0, st>>>(b.rows, sg.ntile, from, hblocks, to);
+            k_rows_starts<<<1, 1024, 0, st>>>(b.rows, sg.ntile, from, hblocks, to, sel, sh);
             QO_LAUNCHED();
         } else {
-            k_rows_reduce<<<rp.nb, 256, 0, st>>>(b.rows, sg.ntile, rp.span, b.bsum);
+            k_rows_reduce<<<rp.nb, 256, 0, st>>>(b.rows, sg.ntile, rp.span, b.bsum, sel, sh);
             QO_LAUNCHED();
-            k_rows_starts<<<1, 1024, 0, st>>>(b.bsum, rp.nb, from, hblocks, to);
+            k_rows_starts<<<1, 1024, 0, st>>>(b.bsum, rp.nb, from, hblocks, to, sel, sh);
             QO_LAUNCHED();
             k_rows_apply<<<rp.nb, 256, 0, st>>>(b.rows, sg.ntile, rp.span, b.bsum, diff, sh);
             QO_LAUNCHED();
