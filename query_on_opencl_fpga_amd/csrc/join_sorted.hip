@@ -8,8 +8,7 @@
 // rows move twice (one split, or two) before they are written once.
 //
 //  * k_sj_sample: 16384 S tuples give the host the expected number of rows, how
-//    evenly their keys spread over the build range, the hottest key and whether
-//    every tuple finds a match.
+//    evenly their keys spread over the build range and the hottest key.
 //  * k_sj_split1 / k_sj_split2: S (filter fused; keys outside the build range
 //    dropped) into up to 256 buckets, each again into up to 256.
 //  * k_sj_finish: per bucket, looks every tuple up, counts the matches per
@@ -20,6 +19,11 @@
 // the build tuples are split the same way and ordered in LDS by bins of the
 // bucket's key interval.  A bucket that overflows (skew that the sample did not
 // show) sets a flag; nothing is written then and the generic path runs.
+//
+// Only rows of the result are written: where a bucket's rows start is known
+// beforehand when every tuple in the build range must have a match (the build
+// keys are the whole range), and comes from a look-back over the buckets'
+// matches otherwise.  More rows than the outputs hold: none is written.
 //
 // Whole calls, generic path -> this one: 2^28 S rows, half selected, 2^24 dense
 // build keys 5.64 -> 2.40 ms (split 0.96, second split 0.55, finish 0.64, build
@@ -43,8 +47,8 @@ constexpr int kSjHotBits = 16;
 struct SjInfo {
     uint32_t mode, dups;   // dups: repeated keys or (-1, -1) build tuples
     int32_t rmin, rmax;
-    uint32_t pass, match;  // sampled tuples that pass the filter inside the build range; those with a match
-    uint32_t hot, pad;     // most samples with one key (to the collisions of kSjHotBits hash bits)
+    uint32_t pass;         // sampled tuples that pass the filter inside the build range
+    uint32_t hot;          // most samples with one key (to the collisions of kSjHotBits hash bits)
     uint32_t pmin, pmax;   // ~smallest and largest sampled s_payload, both as value ^ 2^31
     uint32_t bin[kSjBins];
 };
@@ -60,9 +64,9 @@ __global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader
                                                    const int32_t *__restrict__ sfilt, size_t ns, int32_t flo,
                                                    int32_t fhi, SjInfo *info, uint32_t *keys) {
     __shared__ uint32_t s_bin[kSjBins];
-    __shared__ uint32_t s_pass, s_match, s_hot, s_pmin, s_pmax;
+    __shared__ uint32_t s_pass, s_hot, s_pmin, s_pmax;
     if (threadIdx.x < kSjBins) s_bin[threadIdx.x] = 0;
-    if (threadIdx.x == 0) s_pass = s_match = s_hot = s_pmin = s_pmax = 0;
+    if (threadIdx.x == 0) s_pass = s_hot = s_pmin = s_pmax = 0;
     const uint32_t i = blockIdx.x * kSjSampleThreads + threadIdx.x;
     const uint64_t cell = ns >= kSjSamples ? ns / kSjSamples : 1;
     const uint64_t at = ns >= kSjSamples ? (uint64_t)i * cell + hash32(i) % cell : i;
@@ -76,20 +80,15 @@ __global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader
     in = in && span(key, d) && (!HAS_FILTER || (filt >= flo && filt <= fhi));
     __syncthreads();
     uint32_t hot = 0;
-    bool match = false;
     if (in) {
         atomicAdd(&s_bin[(d >> span_bin_shift(last)) & (kSjBins - 1)], 1u);
         hot = 1 + atomicAdd(&keys[hash32((uint32_t)key) >> (32 - kSjHotBits)], 1u);
-        // A repeated build key makes chains long, and the join generic: no walk then.
-        if (hdr->has_dups == 0)
-            match = join_count(reinterpret_cast<const uint64_t *>(hdr + 1), hdr->cap, JoinHash::of(hdr), 0, key) != 0;
     }
-    const uint64_t m = ballot(in), mm = ballot(match);
+    const uint64_t m = ballot(in);
     hot = wave_max(hot);
     const uint32_t pmin = wave_max(in ? ~pay : 0u), pmax = wave_max(in ? pay : 0u);
     if (lane_id() == 0 && m) {
         atomicAdd(&s_pass, popc(m));
-        atomicAdd(&s_match, popc(mm));
         atomicMax(&s_hot, hot);
         atomicMax(&s_pmin, pmin);
         atomicMax(&s_pmax, pmax);
@@ -98,7 +97,6 @@ __global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader
     if (threadIdx.x < kSjBins && s_bin[threadIdx.x]) atomicAdd(&info->bin[threadIdx.x], s_bin[threadIdx.x]);
     if (threadIdx.x == 0 && s_pass) {
         atomicAdd(&info->pass, s_pass);
-        atomicAdd(&info->match, s_match);
         atomicMax(&info->hot, s_hot);
         atomicMax(&info->pmin, s_pmin);
         atomicMax(&info->pmax, s_pmax);
@@ -111,6 +109,9 @@ __global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader
     }
 }
 
+// *flag of a sorted join (a split's overflowing bucket stores kSjOverflow): not
+// zero, and the finish writes nothing.
+constexpr uint32_t kSjOverflow = 1u, kSjFull = 2u;
 constexpr int kSjPartBits = 8;
 using SjSplitLds = SplitLdsT<1u << kSjPartBits>;
 
@@ -163,11 +164,12 @@ __global__ __launch_bounds__(kSplitThreads) void k_sj_split2(const uint64_t *__r
 }
 
 // off[f]: where the rows of bucket f start when every S tuple of a bucket has
-// a match (off[nb]: their number, also in *d_count).  Block b scans the 2^b2
-// buckets of first-split bucket b behind the totals of the first-split buckets
-// before it (A: nsub regions each).
+// a match (off[nb]: their number, also in *d_count; more than `cap` sets kSjFull).
+// Block b scans the 2^b2 buckets of first-split bucket b behind the totals of the
+// first-split buckets before it (A: nsub regions each).
 __global__ __launch_bounds__(256) void k_sj_offsets(SjBuckets A, uint32_t nsub, SjBuckets S, uint32_t nb, int b2,
-                                                    uint32_t *__restrict__ off, uint64_t *d_count) {
+                                                    uint32_t *__restrict__ off, uint64_t *d_count, uint64_t cap,
+                                                    uint32_t *flag) {
     __shared__ uint32_t s_w[4];
     __shared__ uint32_t s_before;
     if (threadIdx.x == 0) s_before = 0;
@@ -187,21 +189,17 @@ __global__ __launch_bounds__(256) void k_sj_offsets(SjBuckets A, uint32_t nsub, 
         if (f == nb - 1) {
             off[nb] = s_before + ex + c;
             *d_count = s_before + ex + c;
+            if (s_before + ex + c > cap) atomicOr(flag, kSjFull);
         }
     }
 }
 
-// Where a bucket's rows go.  Known: at off[f], when every tuple matches; one that
-// does not sets kSjMiss in *flag.  Chained: behind the rows of the buckets before
-// it, by a look-back in ticket order.
-constexpr uint32_t kSjOverflow = 1u, kSjMiss = 2u;
+// Where a bucket's rows go.  Known: at off[f], when every tuple has a match.
+// Chained: behind the rows of the buckets before it, by a look-back in ticket
+// order.
 struct SjKnown {
-    uint32_t at, n;
-    uint32_t *flag;
-    QO_DEV bool begin(uint32_t total) const {
-        if (total != n && threadIdx.x == 0) atomicOr(flag, kSjMiss);
-        return total == n;
-    }
+    uint32_t at;
+    QO_DEV void begin(uint32_t) const {}
     QO_DEV uint64_t position(uint32_t) const { return at; }
     QO_DEV void repeated() const {}  // the table build saw to that
 };
@@ -210,10 +208,9 @@ struct SjChained {
     uint32_t f, nb;
     uint64_t *d_count;
     DevCtl *ctl;
-    QO_DEV bool begin(uint32_t total) const {
+    QO_DEV void begin(uint32_t total) const {
         // Successors need not wait for the placement.
         if (f > 0 && threadIdx.x == 0) st_agent(&status[f], kFlagAgg | total);
-        return true;
     }
     QO_DEV uint64_t position(uint32_t total) const {
         const uint64_t e = lookback(status, f, total, ctl);
@@ -231,7 +228,7 @@ struct SjChained {
 template <bool DENSE, int NT, bool ALL>
 __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, uint32_t nb, int sh, KeySpan span,
                                                      PayloadBins pbins, const uint64_t *__restrict__ slots,
-                                                     SoaEmit emit, uint32_t *flag, const uint32_t *__restrict__ off,
+                                                     SoaEmit emit, const uint32_t *flag, const uint32_t *__restrict__ off,
                                                      uint64_t *status, uint32_t *ticket, uint64_t *d_count,
                                                      DevCtl *ctl) {
     __shared__ SjLds<DENSE, NT> s;
@@ -239,7 +236,7 @@ __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, u
     // flight together, and the tuples' loads wait for them only.
     const uint32_t fl = *flag;
     const uint32_t o0 = ALL ? off[blockIdx.x] : 0u, o1 = ALL ? off[blockIdx.x + 1] : 0u;
-    if (fl & kSjOverflow) return;  // the generic path runs
+    if (fl) return;  // the whole grid
     if (!ALL && threadIdx.x == 0) s.tile = atomicAdd(ticket, 1u);
     sj_clear(s);
     __syncthreads();
@@ -251,7 +248,7 @@ __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, u
     const uint64_t *rsrc = DENSE ? nullptr : R.bucket + (size_t)f * R.cap;
     const uint64_t *slice = DENSE ? slots + base_d : nullptr;
     if (ALL)
-        sj_bucket(s, src, n, rsrc, nr, slice, span.kmin + base_d, sh, pbins, emit, SjKnown{o0, n, flag});
+        sj_bucket(s, src, n, rsrc, nr, slice, span.kmin + base_d, sh, pbins, emit, SjKnown{o0});
     else
         sj_bucket(s, src, n, rsrc, nr, slice, span.kmin + base_d, sh, pbins, emit,
                   SjChained{status, f, nb, d_count, ctl});
@@ -265,7 +262,8 @@ struct SjSide {            // one input's buckets
     uint64_t capB = 0;     // pairs per fine bucket
 };
 struct SjPlan {
-    bool on = false, dense = false, all = false;
+    bool on = false, dense = false;
+    bool all = false;      // every S tuple in the build range has a match
     int nt = 0;            // threads of the finishing work-groups
     KeySpan span{};
     PayloadBins pay{};
@@ -299,6 +297,7 @@ struct SjSpread {
         const uint32_t top = *std::max_element(in.bin, in.bin + kSjBins);
         even = top <= 1.5 * mean + 6.0 * std::sqrt(mean) + 4.0;
     }
+    double expected() const { return per * info.pass; }
     double most(int shift) const {
         const double part = std::min(1.0, std::ldexp(1.0, shift) / span);
         if (even) return rows * part + hot;
@@ -358,13 +357,16 @@ static bool sj_buckets(SjPlan &p, int nt, const SjSpread &s, size_t nr) {
     return true;
 }
 
-static SjPlan sj_plan(const SjInfo &info, size_t nr, size_t ns) {
+static SjPlan sj_plan(const SjInfo &info, size_t nr, size_t ns, size_t out_capacity) {
     SjPlan p;
     if (info.dups || info.rmin > info.rmax || info.pass == 0) return p;
     const uint32_t last = (uint32_t)info.rmax - (uint32_t)info.rmin;
     const SjSpread s(info, last, ns);
     p.dense = info.mode == kJoinKeyRange;
-    p.all = info.match == info.pass;
+    p.all = p.dense && (uint64_t)last + 1 == nr;  // distinct keys that fill their range
+    // Outputs without room for every tuple in range may still hold the rows: only
+    // the generic path counts them before any is written.
+    if (!p.all && s.expected() > (double)out_capacity) return p;
     p.span = KeySpan{(uint32_t)info.rmin, last};
     p.pay = PayloadBins{~info.pmin, 32 - __builtin_clz((info.pmax - ~info.pmin) | 1u)};
     p.on = sj_buckets(p, 512, s, nr) || sj_buckets(p, 1024, s, nr);
@@ -456,7 +458,7 @@ int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, 
     QO_LAUNCHED();
     QO_HIP(hipMemcpyAsync(&info, d_info, sizeof(info), hipMemcpyDeviceToHost, st));
     QO_HIP(hipStreamSynchronize(st));
-    const SjPlan p = sj_plan(info, nr, ns);
+    const SjPlan p = sj_plan(info, nr, ns, out_capacity);
     if (!p.on) return QO_OK;
     Carver size(nullptr);
     sj_carve(p, size);
@@ -475,42 +477,32 @@ int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, 
     const SoaEmit out{okey, orpay, ospay, out_capacity};
     const SjBuckets sb{b.s.b, p.s.capB, b.s.ctrB}, rb{b.r.b, p.r.capB, b.r.ctrB};
     const uint64_t *slots = reinterpret_cast<const uint64_t *>(hdr + 1);
-    uint64_t res[2];
-    for (bool all = p.all;; all = false) {
-        if (all) {
-            k_sj_offsets<<<p.b2 ? p.nb1 : 1u, 256, 0, st>>>(SjBuckets{nullptr, p.s.capA, b.s.ctrA}, kXcdRegions, sb,
-                                                            p.nb, p.b2, b.off, b.res);
-            QO_LAUNCHED();
-        }
+    if (p.all || ns > out_capacity) {
+        k_sj_offsets<<<p.b2 ? p.nb1 : 1u, 256, 0, st>>>(SjBuckets{nullptr, p.s.capA, b.s.ctrA}, kXcdRegions, sb, p.nb,
+                                                        p.b2, b.off, b.res, out_capacity, flag);
+        QO_LAUNCHED();
+    }
 #define QO_SJ_FINISH(D, T, A)                                                                                       \
     k_sj_finish<D, T, A><<<p.nb, T, 0, st>>>(sb, rb, p.nb, p.sh, p.span, p.pay, slots, out, flag, b.off, b.status, b.ticket, \
                                              b.res, dev_ctl())
-        if (p.dense) {
-            if (p.nt == 512) {
-                if (all) QO_SJ_FINISH(true, 512, true);
-                else QO_SJ_FINISH(true, 512, false);
-            } else {
-                if (all) QO_SJ_FINISH(true, 1024, true);
-                else QO_SJ_FINISH(true, 1024, false);
-            }
-        } else {
-            if (p.nt == 512) {
-                if (all) QO_SJ_FINISH(false, 512, true);
-                else QO_SJ_FINISH(false, 512, false);
-            } else {
-                if (all) QO_SJ_FINISH(false, 1024, true);
-                else QO_SJ_FINISH(false, 1024, false);
-            }
-        }
-#undef QO_SJ_FINISH
-        QO_LAUNCHED();
-        QO_HIP(hipMemcpyAsync(res, b.res, sizeof(res), hipMemcpyDeviceToHost, st));
-        QO_HIP(hipStreamSynchronize(st));
-        const uint32_t f = (uint32_t)res[1];
-        if (f & kSjOverflow) return QO_OK;  // nothing was written
-        // An unmatched tuple: the rows start elsewhere, so they are all written again.
-        if (!(all && (f & kSjMiss))) break;
+    if (p.all) {
+        if (p.nt == 512) QO_SJ_FINISH(true, 512, true);
+        else QO_SJ_FINISH(true, 1024, true);
+    } else if (p.dense) {
+        if (p.nt == 512) QO_SJ_FINISH(true, 512, false);
+        else QO_SJ_FINISH(true, 1024, false);
+    } else {
+        if (p.nt == 512) QO_SJ_FINISH(false, 512, false);
+        else QO_SJ_FINISH(false, 1024, false);
     }
+#undef QO_SJ_FINISH
+    QO_LAUNCHED();
+    uint64_t res[2];
+    QO_HIP(hipMemcpyAsync(res, b.res, sizeof(res), hipMemcpyDeviceToHost, st));
+    QO_HIP(hipStreamSynchronize(st));
+    // Nothing was written then.  kSjFull: the rows are too many if every tuple counted has a match.
+    const uint32_t f = (uint32_t)res[1];
+    if ((f & kSjOverflow) || (f && !p.all)) return QO_OK;
     *rows = res[0];
     *done = true;
     return QO_OK;

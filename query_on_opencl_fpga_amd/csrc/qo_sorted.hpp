@@ -168,10 +168,9 @@ QO_DEV void sj_clear(SjLds<DENSE, NT> &s) {
 // Joins and writes one bucket: n tuples at src, keys in [kbase, kbase + 2^sh).
 // DENSE: `slots` is the bucket's slice of the key-range table (2^sh <= 2 NT
 // slots); else nr <= 2 NT build tuples at rsrc.  `start` says where the rows go:
-// begin(total) (every thread; false: the rows are not written), position(total)
-// (first wave only; the first row's output position) and, for build tuples,
-// repeated() when two have one key.  Called by all NT threads after sj_clear and
-// a barrier.
+// begin(total) (every thread), position(total) (first wave only; the first row's
+// output position) and, for build tuples, repeated() when two have one key.
+// Called by all NT threads after sj_clear and a barrier.
 template <bool DENSE, int NT, class Start>
 QO_DEV void sj_bucket(SjLds<DENSE, NT> &s, const uint64_t *__restrict__ src, uint32_t n,
                       const uint64_t *__restrict__ rsrc, uint32_t nr, const uint64_t *__restrict__ slots, uint32_t kbase,
@@ -271,7 +270,7 @@ QO_DEV void sj_bucket(SjLds<DENSE, NT> &s, const uint64_t *__restrict__ src, uin
         }
     }
     const uint32_t total = sj_scan<NT, Lds::kPer>(s.cnt, s.w);
-    if (!start.begin(total)) return;  // block-uniform
+    start.begin(total);
 #pragma unroll
     for (int j = 0; j < IT; ++j) {
         if (pk[j] == kMiss) continue;
