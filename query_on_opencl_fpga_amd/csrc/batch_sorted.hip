@@ -9,13 +9,12 @@
 //  * k_bj_scan: build key range per query; 1024 sampled S tuples per query;
 //  * k_bj_plan: bucket width per query;
 //  * k_bj_split: S (filter fused) and R tiles of all queries to their buckets;
-//  * k_bj_list: the buckets in use and where their rows start if every tuple
-//    matches;
-//  * k_bj_finish: one work-group per bucket (sj_bucket); a second launch, with a
-//    look-back inside the query, writes the queries that have unmatched tuples;
+//  * k_bj_list: the buckets in use;
+//  * k_bj_finish: one work-group per bucket (sj_bucket), whose rows go behind those
+//    of the query's buckets before it, by a look-back;
 //  * k_bj_end: queries that a bucket overflowed or that repeat a build key are
 //    left to the generic stages of the batch, which otherwise return at once.
-// 512 queries of 4K to 64K build rows (99 M S tuples): 0.92 ms, 3.96 ms with the
+// 512 queries of 4K to 64K build rows (99 M S tuples): 1.07 ms, 3.96 ms with the
 // generic stages alone.
 #include <algorithm>
 #include <cmath>
@@ -160,24 +159,15 @@ __global__ __launch_bounds__(256) void k_bj_plan(const SjBQuery *__restrict__ qs
     if (q < nq) state[q].from = s_base + ex;
 }
 
-// Lists the buckets of query blockIdx.x with their sizes, and the rows before
-// each when every tuple matches.
+// Lists the buckets of query blockIdx.x with their sizes.
 static_assert(kBjMaxBuckets == 512, "one bucket per thread");
-__global__ __launch_bounds__(512) void k_bj_list(const SjBQuery *__restrict__ qs, SjBState *state, const uint32_t *sctr,
-                                                 const uint32_t *rctr, SjBucket *list) {
-    __shared__ uint32_t s_w[512 / kWave];
+__global__ __launch_bounds__(512) void k_bj_list(const SjBQuery *__restrict__ qs, const SjBState *state,
+                                                 const uint32_t *sctr, const uint32_t *rctr, SjBucket *list) {
     const uint32_t q = blockIdx.x, f = threadIdx.x;
-    SjBState &st = state[q];
-    const bool in = f < st.nb;
-    uint32_t n = 0, nr = 0;
-    if (in) {
-        const size_t c = (size_t)(qs[q].bucket0 + f) * kCtrStride;
-        n = min(sctr[c], kBjRows);
-        nr = min(rctr[c], kBjKeys);
-    }
-    const uint32_t ex = block_excl_scan<512 / kWave>(n, s_w);
-    if (in) list[st.from + f] = SjBucket{q, f, n, nr, ex, {0, 0, 0}};
-    if (f == 511) st.rows = ex + n;
+    const SjBState &st = state[q];
+    if (f >= st.nb) return;
+    const size_t c = (size_t)(qs[q].bucket0 + f) * kCtrStride;
+    list[st.from + f] = SjBucket{q, f, min(sctr[c], kBjRows), min(rctr[c], kBjKeys)};
 }
 
 // Blocks [0, nst): S tiles; from nst on: build tiles.
@@ -216,76 +206,93 @@ __global__ __launch_bounds__(kSplitThreads) void k_bj_split(const SjBQuery *__re
                          FixedLayout{build ? kBjKeys : kBjRows}, build ? rctr : sctr, sh, FlagOverflow{&st.overflow});
 }
 
-// Where a bucket's rows go: at its place in the list when every tuple of the
-// query matches, or (the launch for the queries where one did not) behind the
-// rows of the query's buckets before it, by a look-back.
-struct BjKnown {
-    SjBState *st;
-    uint32_t at, n;
-    uint32_t *any_missed;
-    QO_DEV bool begin(uint32_t total) const {
-        if (total != n && threadIdx.x == 0) *any_missed = st->missed = 1u;
-        return total == n;
+// lookback over at most kBjMaxBuckets tiles, with the words of all predecessors
+// in flight together: a query's buckets run at the same time, so hardly one finds
+// an inclusive prefix near it, and a load per 64 predecessors is a chain of up to
+// eight.
+QO_DEV uint64_t bj_lookback(uint64_t *status, uint32_t f, uint32_t aggregate, DevCtl *ctl) {
+    constexpr int kWords = kBjMaxBuckets / kWave;
+    const unsigned lane = lane_id();
+    uint64_t excl = 0;
+    if (f > 0) {
+        const uint32_t limit = ctl->spin_limit;
+        for (uint32_t sleeps = 0;;) {  // wave-uniform: the branches depend on ballots only
+            uint64_t w[kWords];
+#pragma unroll
+            for (int k = 0; k < kWords; ++k) {
+                const int idx = (int)f - 1 - k * kWave - (int)lane;
+                w[k] = idx >= 0 ? ld_agent(&status[idx]) : kFlagInc;
+            }
+            uint64_t sum = 0;
+            bool done = false, empty = false;
+#pragma unroll
+            for (int k = 0; k < kWords; ++k) {
+                if (done || empty) continue;
+                const uint64_t inc = ballot(w[k] >> 62 == 2);
+                const unsigned first = inc ? (unsigned)__builtin_ctzll(inc) : 64u;
+                const uint64_t relevant = first >= 63 ? ~uint64_t(0) : ((uint64_t(2) << first) - 1);
+                empty = (ballot(w[k] >> 62 == 0) & relevant) != 0;
+                if (lane <= first) sum += w[k] & kValMask;
+                done = inc != 0;
+            }
+            if (!empty) {
+                excl = wave_sum(sum);
+                break;
+            }
+            if (++sleeps > limit) {
+                if (lane == 0) atomicOr(&ctl->error, kDevErrLookback);
+                return 0;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
     }
-    QO_DEV uint64_t position(uint32_t) const { return at; }
-    QO_DEV void repeated() const { st->repeated = 1u; }
-};
+    if (lane == 0) st_agent(&status[f], kFlagInc | (excl + aggregate));
+    return excl;
+}
+
+// A bucket's rows go behind the rows of the query's buckets before it.
 struct BjChained {
     SjBState *st;
     uint64_t *status;  // of the query's buckets
     uint32_t f;
     DevCtl *ctl;
-    QO_DEV bool begin(uint32_t total) const {
-        if (f > 0 && threadIdx.x == 0) st_agent(&status[f], kFlagAgg | total);
-        return true;
+    QO_DEV void begin(uint32_t total) const {
+        // Successors need not wait for the placement.
+        if (threadIdx.x == 0) st_agent(&status[f], (f ? kFlagAgg : kFlagInc) | total);
     }
     QO_DEV uint64_t position(uint32_t total) const {
-        const uint64_t e = lookback(status, f, total, ctl);
+        const uint64_t e = bj_lookback(status, f, total, ctl);
         if (f == st->nb - 1 && lane_id() == 0) st->rows = e + total;
         return e;
     }
-    QO_DEV void repeated() const {}
+    QO_DEV void repeated() const { st->repeated = 1u; }
 };
 
-// Each list entry is one bucket's work, or (CHAINED, for the queries with
-// unmatched tuples) that of a bucket of the entry's query taken by ticket, so that
-// every predecessor in the look-back is already running or done.
-template <bool CHAINED>
+// One listed bucket, taken by ticket: a query's buckets are listed in order, so
+// every predecessor in the look-back is already running or done.  Of its 513 us
+// for 512 queries 113 are the look-back and 37 the tickets (a ticket counter per
+// query, read after the list, 30 more; a load per 64 predecessors 25 more).  Rows
+// at positions that assume every tuple matches took 363, and left rows behind the
+// result where one did not.
 __global__ __launch_bounds__(kBjThreads, 8) void k_bj_finish(const SjBQuery *__restrict__ qs, SjBState *state,
-                                                             const SjBucket *__restrict__ list, uint32_t *words,
+                                                             const SjBucket *__restrict__ list,
+                                                             uint32_t *words,
                                                              const uint64_t *sbuckets, const uint64_t *rbuckets,
                                                              uint64_t *status, DevCtl *ctl) {
     __shared__ BjLds s;
-    const uint32_t used = words[0];
-    if (CHAINED && words[1] == 0) return;
-    for (uint32_t i = blockIdx.x; i < used; i += gridDim.x) {  // one round without CHAINED
-        SjBucket e = list[i];
-        const SjBQuery &Q = qs[e.q];
-        SjBState &st = state[e.q];
-        if (st.overflow) {  // block-uniform: neither launch sets it
-            if (!CHAINED) return;
-            continue;
-        }
-        if (CHAINED) {
-            if (!st.missed) continue;  // set by the launch before
-            if (threadIdx.x == 0) s.tile = atomicAdd(&st.ticket, 1u);
-        }
-        sj_clear(s);
-        __syncthreads();
-        if (CHAINED) e = list[st.from + s.tile];
-        const size_t b = Q.bucket0 + e.f;
-        const PayloadBins pbins{~st.pmin_inv, (int)st.pay_bits};
-        const SoaEmit emit{Q.okey, Q.orpay, Q.ospay, Q.out_cap};
-        const uint32_t kbase = st.kmin + (e.f << st.sh);
-        const uint64_t *src = sbuckets + b * kBjRows, *rsrc = rbuckets + b * kBjKeys, *none = nullptr;
-        if constexpr (CHAINED)
-            sj_bucket(s, src, e.n, rsrc, e.nr, none, kbase, (int)st.sh, pbins, emit,
-                      BjChained{&st, status + Q.bucket0, e.f, ctl});
-        else
-            sj_bucket(s, src, e.n, rsrc, e.nr, none, kbase, (int)st.sh, pbins, emit, BjKnown{&st, e.at, e.n, words + 1});
-        if (!CHAINED) return;
-        __syncthreads();  // s is reused
-    }
+    if (blockIdx.x >= words[0]) return;
+    if (threadIdx.x == 0) s.tile = atomicAdd(&words[1], 1u);
+    sj_clear(s);
+    __syncthreads();
+    const SjBucket e = list[s.tile];
+    const SjBQuery &Q = qs[e.q];
+    SjBState &st = state[e.q];
+    if (st.overflow) return;  // block-uniform: this launch does not set it
+    const size_t b = Q.bucket0 + e.f;
+    const PayloadBins pbins{~st.pmin_inv, (int)st.pay_bits};
+    const SoaEmit emit{Q.okey, Q.orpay, Q.ospay, Q.out_cap};
+    sj_bucket(s, sbuckets + b * kBjRows, e.n, rbuckets + b * kBjKeys, e.nr, static_cast<const uint64_t *>(nullptr),
+              st.kmin + (e.f << st.sh), (int)st.sh, pbins, emit, BjChained{&st, status + Q.bucket0, e.f, ctl});
 }
 
 // Queries that the generic stages still have to run: skip[q] = 0, *any = 1.
@@ -381,15 +388,10 @@ int bj_plan_launch(const SjBatchPlan &p, uint32_t *any, hipStream_t st) {
         QO_LAUNCHED();
         k_bj_list<<<(unsigned)nq, 512, 0, st>>>(p.d_q, p.state, p.sctr, p.rctr, p.list);
         QO_LAUNCHED();
-        // One block per bucket a query may use (two to four times those in use;
-        // 366 us for 512 queries, 408 with 2048 blocks that walk the list), few for
-        // the launch that usually finds nothing to do.
-        const unsigned fg = std::min<unsigned>(p.buckets, (unsigned)props().cu_count * 8);
-        k_bj_finish<false><<<p.buckets, kBjThreads, 0, st>>>(p.d_q, p.state, p.list, p.words, p.sbuckets, p.rbuckets,
-                                                             p.status, dev_ctl());
-        QO_LAUNCHED();
-        k_bj_finish<true><<<fg, kBjThreads, 0, st>>>(p.d_q, p.state, p.list, p.words, p.sbuckets, p.rbuckets,
-                                                            p.status, dev_ctl());
+        // One block per bucket a query may use (two to four times those in use; 2048
+        // blocks that walk the list took a tenth longer).
+        k_bj_finish<<<p.buckets, kBjThreads, 0, st>>>(p.d_q, p.state, p.list, p.words, p.sbuckets, p.rbuckets,
+                                                      p.status, dev_ctl());
         QO_LAUNCHED();
     }
     k_bj_end<<<qg, 256, 0, st>>>(p.d_q, p.state, nq, p.skip, any);

@@ -210,7 +210,7 @@ struct SjChained {
     DevCtl *ctl;
     QO_DEV void begin(uint32_t total) const {
         // Successors need not wait for the placement.
-        if (f > 0 && threadIdx.x == 0) st_agent(&status[f], kFlagAgg | total);
+        if (threadIdx.x == 0) st_agent(&status[f], (f ? kFlagAgg : kFlagInc) | total);
     }
     QO_DEV uint64_t position(uint32_t total) const {
         const uint64_t e = lookback(status, f, total, ctl);

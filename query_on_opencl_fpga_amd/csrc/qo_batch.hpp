@@ -48,11 +48,11 @@ struct SjBState {             // zero before a launch
     uint32_t pmin_inv, pmax;  // ~smallest and largest sampled s_payload, biased
     uint32_t kmin, last, sh, nb, pay_bits;
     uint32_t from;            // first of its buckets in the list of those in use
-    uint32_t overflow, repeated, missed, ticket;
+    uint32_t overflow, repeated;
     uint64_t rows;            // matches
 };
-struct SjBucket {             // a bucket in use: S and build tuples, rows before it if every tuple matches
-    uint32_t q, f, n, nr, at, pad[3];
+struct SjBucket {             // a bucket in use: its S and build tuples
+    uint32_t q, f, n, nr;
 };
 struct SjBatchPlan {
     std::vector<SjBQuery> q;
@@ -62,7 +62,7 @@ struct SjBatchPlan {
     SjBQuery *d_q = nullptr;
     uint2 *d_stiles = nullptr, *d_rtiles = nullptr;
     SjBucket *list = nullptr;     // the buckets in use, words[0] of them
-    uint32_t *skip = nullptr, *words = nullptr;  // words[1]: some query has unmatched tuples
+    uint32_t *skip = nullptr, *words = nullptr;  // words[1]: tickets of the list
     SjBState *state = nullptr;
     uint32_t *sctr = nullptr, *rctr = nullptr;
     uint64_t *status = nullptr, *sbuckets = nullptr, *rbuckets = nullptr;
