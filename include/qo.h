@@ -242,7 +242,10 @@ int qo_hash_probe(const void *table, size_t table_bytes, const int32_t *skey, co
 int qo_join_table_info(const void *table, int *mode, uint64_t *slots_used, int *has_dups, qo_stream s);
 /* Filter S, build on R, probe, sort output by (key, s_payload).  Synchronous:
  * *h_count receives the match count.  Rows equal in (key, s_payload), which
- * only duplicate R keys produce, come in no specified order. */
+ * only duplicate R keys produce, come in no specified order.  Output rows past
+ * the match count keep what they held; more matches than out_capacity give
+ * QO_ERR_CAPACITY with no row written, and a bounded device-side wait that ran
+ * out QO_ERR_DEVICE_WAIT. */
 int qo_hj_filter_sort(void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay,
                       size_t nr, const int32_t *skey, const int32_t *spay, const int32_t *sfilt,
                       size_t ns, int32_t flo, int32_t fhi, int32_t *okey, int32_t *orpay,
@@ -280,7 +283,8 @@ typedef struct qo_batch qo_batch;
 int qo_batch_create(const qo_join_query *queries, int nq, qo_batch **out);
 /* Launch the whole batch (one graph launch) on stream s. */
 int qo_batch_launch(qo_batch *b, qo_stream s);
-/* After completion: per-query match counts (host array of nq). */
+/* Waits for the device, then reads the per-query match counts (host array of
+ * nq); QO_ERR_DEVICE_WAIT as for qo_stream_sync. */
 int qo_batch_counts(qo_batch *b, uint64_t *h_counts);
 int qo_batch_destroy(qo_batch *b);
 

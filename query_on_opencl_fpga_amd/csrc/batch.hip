@@ -430,7 +430,7 @@ int qo_batch_counts(qo_batch *b, uint64_t *h_counts) {
     QO_REQUIRE(b && h_counts, "null argument");
     QO_HIP(hipDeviceSynchronize());
     QO_HIP(hipMemcpy(h_counts, b->plan.counts, 8 * (size_t)b->plan.nq, hipMemcpyDeviceToHost));
-    return QO_OK;
+    return check_device_error();
 }
 
 int qo_batch_destroy(qo_batch *b) {

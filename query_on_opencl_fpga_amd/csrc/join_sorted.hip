@@ -109,9 +109,10 @@ __global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader
     }
 }
 
-// *flag of a sorted join (a split's overflowing bucket stores kSjOverflow): not
-// zero, and the finish writes nothing.
-constexpr uint32_t kSjOverflow = 1u, kSjFull = 2u;
+// *flag of a sorted join (a split's overflowing bucket stores kSjOverflow): with
+// one of the first two the finish writes nothing; the finish sets kSjWait when its
+// look-back gave up.
+constexpr uint32_t kSjOverflow = 1u, kSjFull = 2u, kSjWait = 4u;
 constexpr int kSjPartBits = 8;
 using SjSplitLds = SplitLdsT<1u << kSjPartBits>;
 
@@ -208,12 +209,13 @@ struct SjChained {
     uint32_t f, nb;
     uint64_t *d_count;
     DevCtl *ctl;
+    uint32_t *flag;
     QO_DEV void begin(uint32_t total) const {
         // Successors need not wait for the placement.
         if (threadIdx.x == 0) st_agent(&status[f], (f ? kFlagAgg : kFlagInc) | total);
     }
     QO_DEV uint64_t position(uint32_t total) const {
-        const uint64_t e = lookback(status, f, total, ctl);
+        const uint64_t e = lookback(status, f, total, ctl, flag, kSjWait);
         if (f == nb - 1 && lane_id() == 0) *d_count = e + total;
         return e;
     }
@@ -228,7 +230,7 @@ struct SjChained {
 template <bool DENSE, int NT, bool ALL>
 __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, uint32_t nb, int sh, KeySpan span,
                                                      PayloadBins pbins, const uint64_t *__restrict__ slots,
-                                                     SoaEmit emit, const uint32_t *flag, const uint32_t *__restrict__ off,
+                                                     SoaEmit emit, uint32_t *flag, const uint32_t *__restrict__ off,
                                                      uint64_t *status, uint32_t *ticket, uint64_t *d_count,
                                                      DevCtl *ctl) {
     __shared__ SjLds<DENSE, NT> s;
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, u
     // flight together, and the tuples' loads wait for them only.
     const uint32_t fl = *flag;
     const uint32_t o0 = ALL ? off[blockIdx.x] : 0u, o1 = ALL ? off[blockIdx.x + 1] : 0u;
-    if (fl) return;  // the whole grid
+    if (fl & (kSjOverflow | kSjFull)) return;  // the whole grid
     if (!ALL && threadIdx.x == 0) s.tile = atomicAdd(ticket, 1u);
     sj_clear(s);
     __syncthreads();
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, u
         sj_bucket(s, src, n, rsrc, nr, slice, span.kmin + base_d, sh, pbins, emit, SjKnown{o0});
     else
         sj_bucket(s, src, n, rsrc, nr, slice, span.kmin + base_d, sh, pbins, emit,
-                  SjChained{status, f, nb, d_count, ctl});
+                  SjChained{status, f, nb, d_count, ctl, flag});
 }
 
 // ---------------------------------------------------------------------------
@@ -502,6 +504,10 @@ int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, 
     QO_HIP(hipStreamSynchronize(st));
     // Nothing was written then.  kSjFull: the rows are too many if every tuple counted has a match.
     const uint32_t f = (uint32_t)res[1];
+    if (f & kSjWait) {
+        QO_TRY(check_device_error());
+        return set_error(QO_ERR_DEVICE_WAIT, "a device-side wait of the join ran out of its bound");
+    }
     if ((f & kSjOverflow) || (f && !p.all)) return QO_OK;
     *rows = res[0];
     *done = true;

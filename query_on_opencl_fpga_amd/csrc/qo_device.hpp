@@ -217,8 +217,10 @@ constexpr uint32_t kDefaultSpinLimit = 1u << 22;  // s_sleep(1) rounds: about a 
 // Tiles must be numbered by a ticket counter, so every predecessor is already
 // resident and the wait ends; it is bounded all the same: after
 // ctl->spin_limit sleeps the wave sets kDevErrLookback in ctl->error and
-// returns 0 (the call's results are then undefined, and the kernel ends).
-QO_DEV uint64_t lookback(uint64_t *status, uint64_t tile, uint64_t aggregate, DevCtl *ctl) {
+// returns 0 (the call's results are then undefined, and the kernel ends); with
+// `word` it sets `bit` there too, for a call that looks at its own words.
+QO_DEV uint64_t lookback(uint64_t *status, uint64_t tile, uint64_t aggregate, DevCtl *ctl, uint32_t *word = nullptr,
+                         uint32_t bit = 0) {
     const unsigned lane = lane_id();
     if (tile == 0) {
         if (lane == 0) st_agent(&status[0], kFlagInc | (aggregate & kValMask));
@@ -240,6 +242,7 @@ QO_DEV uint64_t lookback(uint64_t *status, uint64_t tile, uint64_t aggregate, De
         if (empty_mask & relevant) {
             if (++sleeps > limit) {
                 if (lane == 0) atomicOr(&ctl->error, kDevErrLookback);
+                if (lane == 0 && word) atomicOr(word, bit);
                 return 0;
             }
             __builtin_amdgcn_s_sleep(1);
