@@ -143,8 +143,8 @@ int qo_sort_records(qo_record *data, size_t n, qo_stream s);
 /* Sort join rows ascending by (key, s_payload) as signed int32, stable, in place.
  * Synchronizes stream s once: the rows are sorted on the key first and each
  * key's run by s_payload after; a key with more than 64 rows is sorted by a
- * work-group of its own, and only very long or very many such keys (read back
- * from the device) send all rows through the full-width sort. */
+ * work-group of its own, and only long (more than 6144 rows) or many such keys
+ * (read back from the device) send all rows through the full-width sort. */
 int qo_sort_join_rows(int32_t *key, int32_t *rpay, int32_t *spay, size_t m, qo_stream s);
 
 /* ---- sort-based group-by (reference pipeline) ------------------------------ */

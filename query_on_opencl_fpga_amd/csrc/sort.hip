@@ -704,11 +704,13 @@ int launch_radix_rows_segments(uint64_t *keys, uint32_t *vals, uint64_t *kalt, u
     return QO_OK;
 }
 
-// Long runs the list holds: enough that listing every one and sorting each in a
-// work-group stays cheaper than the eight full-width passes.
-static uint32_t long_runs_cap(size_t m) { return (uint32_t)(4096 + m / 1024); }
-// Longest run that one work-group sorts on its own (4.9 ns per row).
-static uint64_t long_run_limit(size_t m) { return (1u << 14) + m / 256; }
+// Long runs that are sorted by work-groups; more send all rows through the
+// full-width sort.  A run takes its work-group 35 to 40 us whatever its length and
+// two fit a CU, so 512 run at once; the full width costs 75 us (10,000 to 100,000
+// rows), 100 (1 M) or 330 (10 M).  By work-groups, full width, in us: 100,000 rows
+// with 500 long runs 185, 231, with 1428 252, 227; 1 M with 1000 272, 286, with
+// 5000 569, 286; 10 M with 1667 882, 879, with 10,000 1400, 876.
+static uint32_t long_runs_cap(size_t m) { return (uint32_t)(1024 + m / 16384); }
 
 static void radix_carve(size_t n, bool with_vals, Carver &cv, uint64_t **kalt, uint32_t **valt, RowsBufs *rb,
                         uint32_t **runs = nullptr) {
@@ -956,6 +958,9 @@ constexpr uint32_t kFixThreads = 512;  // four blocks per CU (34 KB LDS each), 8
 constexpr uint32_t kFixRounds = (kFixWin + kFixThreads - 1) / kFixThreads;
 constexpr uint32_t kFixChunks = kFixWin / kWave + 2;  // marks of the window's chunks and one past it
 
+constexpr int kLongItems = 6;
+constexpr uint32_t kLongLds = kLongItems * kBlockSortThreads;  // longest run sorted in LDS
+
 // Where the run pass leaves the runs longer than kFixRun.
 struct LongRuns {
     uint32_t *flag;            // set: the rows need the full-width sort
@@ -965,6 +970,7 @@ struct LongRuns {
     SegPos *seg_list = nullptr;  // in place of `list` for a batch: (segment, start), never full
     uint32_t seg = 0;
 };
+constexpr uint32_t kFixLongMax = kFixTile / (kFixRun + 1) + 1;  // long runs that start in a tile
 
 // Block work of the run pass: positions [t0, t0 + kFixTile) of m rows (k, v).
 QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__restrict__ v, size_t m, size_t t0,
@@ -973,6 +979,8 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
     __shared__ uint32_t s_hi[kFixWin];
     __shared__ uint32_t s_lo[kFixWin + 4];  // 4 words of slack for the unrolled rank loop
     __shared__ uint64_t s_mark[kFixChunks];
+    __shared__ uint32_t s_long[kFixLongMax], s_nlong, s_at;
+    if (threadIdx.x == 0) s_nlong = 0;
     const uint32_t own = (uint32_t)(m - t0 < kFixTile ? m - t0 : kFixTile);
     const uint32_t len = (uint32_t)(m - t0 < kFixWin ? m - t0 : kFixWin);
     const bool data_end = t0 + len == m;  // the window reaches the last row
@@ -1003,11 +1011,9 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
     bool long_run = false;
     auto is_long = [&](uint32_t i, uint32_t s) {
         long_run = true;
-        if ((lr.list || lr.seg_list) && i == s) {  // the run's first row lists it
-            const uint32_t at = atomicAdd(lr.n, 1u);
-            if (lr.seg_list) lr.seg_list[at] = SegPos{lr.seg, (uint32_t)(t0 + s)};
-            else if (at < lr.cap) lr.list[at] = (uint32_t)(t0 + s);
-        }
+        if (i != s) return;
+        s_long[atomicAdd(&s_nlong, 1u)] = s;  // the run's first row lists it
+        if (lr.list && t0 + s + kLongLds < m && (uint32_t)(k[t0 + s + kLongLds] >> 32) == s_hi[s]) *lr.flag = 1u;
     };
     for (uint32_t i = threadIdx.x; i < len; i += kFixThreads) {
         const uint32_t c = i / kWave;  // uniform across the wave
@@ -1054,7 +1060,21 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
         out.spay[dst] = join_sort_key_spay(x);
         out.rpay[dst] = (int32_t)v[t0 + i];
     }
-    if (long_run && !lr.list && !lr.seg_list) atomicOr(lr.flag, 1u);
+    if (!lr.list && !lr.seg_list) {
+        if (long_run) atomicOr(lr.flag, 1u);
+        return;
+    }
+    // One reservation per block: one per run, from every wave of the chip to one
+    // address, took 1 ms for 140,000 runs.
+    __syncthreads();
+    if (s_nlong == 0) return;
+    if (threadIdx.x == 0) s_at = atomicAdd(lr.n, s_nlong);
+    __syncthreads();
+    if (threadIdx.x < s_nlong) {
+        const uint32_t at = s_at + threadIdx.x, s = (uint32_t)t0 + s_long[threadIdx.x];
+        if (lr.seg_list) lr.seg_list[at] = SegPos{lr.seg, s};
+        else if (at < lr.cap) lr.list[at] = s;
+    }
 }
 
 __global__ __launch_bounds__(kFixThreads) void k_fix_runs(const uint64_t *__restrict__ k, const uint32_t *__restrict__ v,
@@ -1062,42 +1082,33 @@ __global__ __launch_bounds__(kFixThreads) void k_fix_runs(const uint64_t *__rest
     fix_runs_tile(k, v, m, (size_t)blockIdx.x * kFixTile, out, lr);
 }
 
-// The long runs of k_fix_runs, one work-group each in turn.  A run of up to
-// kLongLds rows is sorted by s_payload in LDS; a longer one, up to `longest`
-// rows, by four digit passes of this work-group between its places in (k, v)
-// and (kalt, valt), which no other run uses; a run longer still, or more runs
-// than the list holds, sets the flag (the full-width sort reads (k, v), where
-// every run is complete in some order at any time).  Bound by the passes' chain
-// of dependent LDS steps, with one work-group per run.  Before it, one key of
-// more than 64 rows sent all rows through eight more passes: 3,000,045 S rows
-// with 200,003 unevenly referenced dense keys (hottest key ~4000 rows) 557 ->
-// 376 us for the whole join, 60,000,045 with 4,000,003 3.94 -> 3.40 ms.
-constexpr int kLongItems = 6;
-constexpr uint32_t kLongLds = kLongItems * kBlockSortThreads;
+// The long runs of k_fix_runs, one work-group each in turn, sorted by s_payload
+// in LDS.  A run longer than kLongLds rows, or more runs than the list holds,
+// sets the flag before any is sorted (the full-width sort then takes all rows).
+// Bound by the passes' chain of dependent LDS steps: 40 us for a run of 6000
+// rows, where the full-width sort of 10,000 to 100,000 rows costs 75.  Runs past
+// LDS, by digit passes of one work-group through memory, took 79 us at 7000 rows,
+// 171 at 20,000 and 735 at 100,000, so from there on the full width is the
+// cheaper one (10 M rows in runs of 20,000: 1.06 ms and 0.88).
 
-// End of the run of equal key that starts at s; `longest` rows at most are
-// looked at (s + longest + 1 is returned for a longer run).
-QO_DEV uint64_t run_end(const uint64_t *k, size_t m, uint64_t s, uint64_t longest, uint32_t *s_min) {
+// End of the run of equal key that starts at s, looked for up to `hi` (returned
+// when the run goes on there), by the whole work-group: 1024 probes a round.
+QO_DEV uint64_t run_end(const uint64_t *k, uint64_t s, uint64_t hi, uint32_t *s_min) {
     const uint32_t key = (uint32_t)(k[s] >> 32);
-    auto differs = [&](uint64_t p) { return p >= m || (uint32_t)(k[p] >> 32) != key; };
-    for (uint64_t from = s; from <= s + longest; from += (uint64_t)kBlockSortThreads * kWave) {
-        if (threadIdx.x == 0) *s_min = ~0u;
+    uint64_t lo = s;  // the run's; the end lies in (lo, hi]
+    while (hi - lo > 1) {
+        const uint64_t step = (hi - lo + kBlockSortThreads - 1) / kBlockSortThreads;
+        const uint32_t probes = (uint32_t)((hi - lo - 1) / step);  // below hi; at most 1023
+        if (threadIdx.x == 0) *s_min = probes;
         __syncthreads();
-        if (differs(from + (uint64_t)(threadIdx.x + 1) * kWave)) atomicMin(s_min, threadIdx.x);
+        if (threadIdx.x < probes && (uint32_t)(k[lo + (threadIdx.x + 1) * step] >> 32) != key) atomicMin(s_min, threadIdx.x);
         __syncthreads();
-        const uint32_t c = *s_min;
+        const uint32_t c = *s_min;  // probes inside the run: the end lies in (probe c - 1, probe c] or up to hi
         __syncthreads();
-        if (c == ~0u) continue;  // block-uniform
-        const uint64_t p0 = from + (uint64_t)c * kWave;  // the end lies in (p0, p0 + 64]
-        if (threadIdx.x == 0) *s_min = kWave;
-        __syncthreads();
-        if (threadIdx.x < kWave && differs(p0 + threadIdx.x + 1)) atomicMin(s_min, threadIdx.x + 1);
-        __syncthreads();
-        const uint64_t e = p0 + *s_min;
-        __syncthreads();
-        return e;
+        lo += c * step;
+        hi = lo + step < hi ? lo + step : hi;
     }
-    return s + longest + 1;
+    return hi;
 }
 
 struct LongLds {
@@ -1106,30 +1117,29 @@ struct LongLds {
     uint32_t min;
 };
 
-// The run that starts at s, by the whole work-group; false when it is longer
-// than `longest` (not written).  Ends with a barrier.
-QO_DEV bool fix_long_run(LongLds &L, uint64_t *k, uint32_t *v, uint64_t *kalt, uint32_t *valt, size_t m, uint64_t s,
-                         uint64_t longest, const RowOut &out) {
-    const unsigned w = wave_id(), lane = lane_id();
-    const uint64_t e = run_end(k, m, s, longest, &L.min);
-    const uint64_t len = e - s;
+// The run [s, s + len) of one key, by the whole work-group; len <= kLongLds.
+// Ends with a barrier.
+QO_DEV void fix_run_lds(LongLds &L, const uint64_t *k, const uint32_t *v, uint64_t s, uint32_t len, const RowOut &out) {
     const int32_t key = join_sort_key_key(k[s]);
-    if (len > longest) return false;
-    if (len <= kLongLds) {
-        // Sorted as s_payload (order-preserving) << 32 | r_payload.
-        for (uint32_t i = threadIdx.x; i < (uint32_t)len; i += kBlockSortThreads)
-            L.S.key[i] = (k[s + i] << 32) | v[s + i];
-        __syncthreads();
-        block_sort<kLongItems, false>(L.S, (uint32_t)len, 32, 64);
-        for (uint32_t i = threadIdx.x; i < (uint32_t)len; i += kBlockSortThreads) {
-            const uint64_t x = L.S.key[i];
-            out.key[s + i] = key;
-            out.spay[s + i] = (int32_t)((uint32_t)(x >> 32) ^ 0x80000000u);
-            out.rpay[s + i] = (int32_t)(uint32_t)x;
-        }
-        __syncthreads();  // S is reused
-        return true;
+    // Sorted as s_payload (order-preserving) << 32 | r_payload.
+    for (uint32_t i = threadIdx.x; i < len; i += kBlockSortThreads) L.S.key[i] = (k[s + i] << 32) | v[s + i];
+    __syncthreads();
+    block_sort<kLongItems, false>(L.S, len, 32, 64);
+    for (uint32_t i = threadIdx.x; i < len; i += kBlockSortThreads) {
+        const uint64_t x = L.S.key[i];
+        out.key[s + i] = key;
+        out.spay[s + i] = (int32_t)((uint32_t)(x >> 32) ^ 0x80000000u);
+        out.rpay[s + i] = (int32_t)(uint32_t)x;
     }
+    __syncthreads();  // S is reused
+}
+
+// A longer run, by four digit passes of the work-group between its places in
+// (k, v) and (kalt, valt).  Ends with a barrier.
+QO_DEV void fix_run_passes(LongLds &L, uint64_t *k, uint32_t *v, uint64_t *kalt, uint32_t *valt, uint64_t s,
+                           uint64_t len, const RowOut &out) {
+    const unsigned w = wave_id(), lane = lane_id();
+    const int32_t key = join_sort_key_key(k[s]);
     // Digit counts of the four passes, then per pass the tiles in order.
     for (uint32_t i = threadIdx.x; i < 1024; i += kBlockSortThreads) (&L.hist[0][0])[i] = 0;
     __syncthreads();
@@ -1196,8 +1206,7 @@ QO_DEV bool fix_long_run(LongLds &L, uint64_t *k, uint32_t *v, uint64_t *kalt, u
             }
             __syncthreads();  // the counts are reused by the next tile
         }
-        __threadfence();  // the next pass reads what other waves wrote
-        __syncthreads();
+        __syncthreads();  // the next pass reads what other waves of the work-group wrote
         uint64_t *const kt = ks;
         ks = kd;
         kd = kt;
@@ -1211,20 +1220,22 @@ QO_DEV bool fix_long_run(LongLds &L, uint64_t *k, uint32_t *v, uint64_t *kalt, u
         out.rpay[s + i] = (int32_t)vs[i];
     }
     __syncthreads();
-    return true;
 }
 
-__global__ __launch_bounds__(kBlockSortThreads) void k_fix_long(uint64_t *k, uint32_t *v, uint64_t *kalt,
-                                                                uint32_t *valt, size_t m, uint64_t longest, RowOut out,
+__global__ __launch_bounds__(kBlockSortThreads) void k_fix_long(const uint64_t *k, const uint32_t *v, size_t m, RowOut out,
                                                                 LongRuns lr) {
     __shared__ LongLds L;
     const uint32_t n = *lr.n;
+    if (n == 0 || *lr.flag) return;  // whole block
     if (n > lr.cap) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) *lr.flag = 1u;
-        return;  // whole block
+        if (threadIdx.x == 0) *lr.flag = 1u;
+        return;  // every block
     }
-    for (uint32_t r = blockIdx.x; r < n; r += gridDim.x)
-        if (!fix_long_run(L, k, v, kalt, valt, m, lr.list[r], longest, out) && threadIdx.x == 0) *lr.flag = 1u;
+    for (uint32_t r = blockIdx.x; r < n; r += gridDim.x) {
+        const uint64_t s = lr.list[r];
+        const uint64_t e = run_end(k, s, std::min<uint64_t>(m, s + kLongLds), &L.min);
+        fix_run_lds(L, k, v, s, (uint32_t)(e - s), out);
+    }
 }
 
 // Segmented form: block b is global tile b of the segments (kSortTile rows per
@@ -1255,7 +1266,9 @@ __global__ __launch_bounds__(kBlockSortThreads) void k_fix_long_seg(uint64_t *k,
         const SegPos p = list[r];
         const RadixSeg sg = segs[p.seg];
         const size_t m = seg_count(sg);
-        fix_long_run(L, k + sg.base, v + sg.base, kalt + sg.base, valt + sg.base, m, p.start, m, outs[p.seg]);
+        const uint64_t len = run_end(k + sg.base, p.start, m, &L.min) - p.start;
+        if (len <= kLongLds) fix_run_lds(L, k + sg.base, v + sg.base, p.start, (uint32_t)len, outs[p.seg]);
+        else fix_run_passes(L, k + sg.base, v + sg.base, kalt + sg.base, valt + sg.base, p.start, len, outs[p.seg]);
     }
 }
 
@@ -1305,12 +1318,11 @@ int sort_packed_join_rows(uint64_t *k64, uint32_t *v32, size_t m, void *rws, int
     QO_TRY(launch_fill_u32(flag, 0, 2, st));
     const size_t blocks = (m + kFixTile - 1) / kFixTile;
     const LongRuns lr{flag, flag + 1, runs, long_runs_cap(m)};
-    uint64_t *ks = in_alt ? kalt : k64, *kd = in_alt ? k64 : kalt;
-    uint32_t *vs = in_alt ? valt : v32, *vd = in_alt ? v32 : valt;
+    const uint64_t *ks = in_alt ? kalt : k64;
+    const uint32_t *vs = in_alt ? valt : v32;
     k_fix_runs<<<(unsigned)blocks, kFixThreads, 0, st>>>(ks, vs, m, out, lr);
     QO_LAUNCHED();
-    k_fix_long<<<(unsigned)props().cu_count * 2, kBlockSortThreads, 0, st>>>(ks, vs, kd, vd, m, long_run_limit(m), out,
-                                                                           lr);
+    k_fix_long<<<(unsigned)props().cu_count * 2, kBlockSortThreads, 0, st>>>(ks, vs, m, out, lr);
     QO_LAUNCHED();
     uint32_t long_run = 0;
     QO_HIP(hipMemcpyAsync(&long_run, flag, 4, hipMemcpyDeviceToHost, st));
