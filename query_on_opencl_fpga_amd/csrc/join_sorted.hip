@@ -42,6 +42,7 @@ namespace qo {
 constexpr uint32_t kSjSamples = 16384;
 constexpr uint32_t kSjBins = 256;
 constexpr int kSjHotBits = 16;
+constexpr int kSjHotRounds = 8;
 
 // What the host plans from: the table's state and the sample's counts.
 struct SjInfo {
@@ -79,12 +80,23 @@ __global__ __launch_bounds__(kSjSampleThreads) void k_sj_sample(const JoinHeader
     uint32_t d = 0;
     in = in && span(key, d) && (!HAS_FILTER || (filt >= flo && filt <= fhi));
     __syncthreads();
-    uint32_t hot = 0;
-    if (in) {
-        atomicAdd(&s_bin[(d >> span_bin_shift(last)) & (kSjBins - 1)], 1u);
-        hot = 1 + atomicAdd(&keys[hash32((uint32_t)key) >> (32 - kSjHotBits)], 1u);
-    }
     const uint64_t m = ballot(in);
+    // Samples of one key meet at one address, where 16384 take 0.2 ms: a few keys
+    // of the wave are counted there once, which a hot one is unlikely to escape.
+    uint32_t hot = in ? 1u : 0u;  // samples this lane counts
+    uint64_t open = m;
+#pragma unroll
+    for (int r = 0; r < kSjHotRounds; ++r) {
+        // Another part of the wave each time: hot keys may come in any pattern.
+        const uint64_t from = open >> (r * (kWave / kSjHotRounds)) << (r * (kWave / kSjHotRounds));
+        if (from == 0) continue;
+        const int leader = __builtin_ctzll(from);
+        const uint64_t same = ballot(key == __shfl(key, leader, kWave)) & open;
+        if ((same >> lane_id()) & 1u) hot = (int)lane_id() == leader ? popc(same) : 0u;
+        open &= ~same;
+    }
+    if (hot) hot += atomicAdd(&keys[hash32((uint32_t)key) >> (32 - kSjHotBits)], hot);
+    if (in) atomicAdd(&s_bin[(d >> span_bin_shift(last)) & (kSjBins - 1)], 1u);
     hot = wave_max(hot);
     const uint32_t pmin = wave_max(in ? ~pay : 0u), pmax = wave_max(in ? pay : 0u);
     if (lane_id() == 0 && m) {
