@@ -328,12 +328,13 @@ struct SjSpread {
     }
 };
 
-// A fine bucket has room for all the rows a work-group takes, whatever the
-// expected number: a hot key of some thousand rows still fits.  `most`: rows
-// expected in the fullest bucket of the first split.
-static SjSide sj_side(const SjPlan &p, double most, uint32_t limit) {
+// A fine bucket has room for all the rows a work-group takes, so that a hot key of
+// some thousand rows still fits; where fewer than 256 are expected in one (then S
+// is small, and its sample shows such a key), for eight times those and 1024.
+// `most`: rows expected in the fullest bucket of the first split.
+static SjSide sj_side(const SjPlan &p, double most, double mean, uint32_t limit) {
     SjSide o;
-    o.capB = limit;
+    o.capB = std::min<uint64_t>(limit, ((uint64_t)(8.0 * mean) + 1024 + 31) / 32 * 32);
     if (p.b2) o.capA = ((uint64_t)(most / kXcdRegions * 1.25 + 8.0 * std::sqrt(most)) + kSplitTile + 31) / 32 * 32;
     return o;
 }
@@ -355,7 +356,13 @@ static bool sj_buckets(SjPlan &p, int nt, const SjSpread &s, size_t nr) {
     }
     const uint64_t nb = ((uint64_t)p.span.last >> p.sh) + 1;
     // Of uneven keys no more buckets than a few per 1000 rows: most would be empty.
+    // Even ones can need many for the build keys alone: a slice of the table each, or
+    // (spread keys) their share of R, which is split as well.  Half of S selected,
+    // this path and the generic one in us: 2^24 dense keys with 2^18 S rows 408, 396,
+    // 2^20 418, 487; 2^20 spread keys with 2^14 rows 305, 333, 2^22 401, 366; 2^24
+    // spread with 2^22 rows 876, 829, with 2^24 969, 1131.
     if (nb > kSjMaxBuckets || s.most(p.sh) > 0.9 * limit || (!s.even && nb > 1024 + s.rows / 256)) return false;
+    if (p.dense ? (double)nb > 8192.0 + s.rows / 16.0 : (double)nr > 1048576.0 + 4.0 * s.rows) return false;
     p.nb = (uint32_t)nb;
     int bits = 0;
     while ((1u << bits) < p.nb) ++bits;
@@ -363,10 +370,10 @@ static bool sj_buckets(SjPlan &p, int nt, const SjSpread &s, size_t nr) {
     p.nb1 = ((p.nb - 1) >> p.b2) + 1;
     p.parts1 = 1;
     while (p.parts1 < p.nb1) p.parts1 *= 2;
-    p.s = sj_side(p, s.most(p.sh + p.b2), (uint32_t)limit);
+    p.s = sj_side(p, s.most(p.sh + p.b2), s.rows / p.nb, (uint32_t)limit);
     if (!p.dense) {
         const double even = (double)nr * std::min(1.0, std::ldexp(1.0, p.sh + p.b2) / s.span);
-        p.r = sj_side(p, s.even ? even : std::min((double)nr, 4.0 * even), 2u * (uint32_t)nt);
+        p.r = sj_side(p, s.even ? even : std::min((double)nr, 4.0 * even), (double)nr / p.nb, 2u * (uint32_t)nt);
     }
     return true;
 }

@@ -73,3 +73,30 @@ def test_hot_key_costs_no_serial_count(qo, kind, nr, ns, hot):
     sk = rk[rng.integers(0, nr, ns)]
     sk[: int(hot * ns)] = rk[3]
     compare(qo, rk, rng.permutation(sk), 1.3)
+
+
+@pytest.mark.parametrize("kind", ["dense", "spread"])
+@pytest.mark.parametrize("nr,ns", [(1 << 22, 1 << 14), (1 << 24, 1 << 14), (1 << 24, 1 << 18)])
+def test_small_probe_of_a_large_build_side(qo, kind, nr, ns):
+    """Few S tuples and many build keys: no bucket per slice of the build side for them."""
+    rng = np.random.default_rng(nr + ns)
+    rk = keys(kind, nr, rng)
+    compare(qo, rk, rk[rng.integers(0, nr, ns)], 1.2)
+
+
+@pytest.mark.parametrize("kind", ["dense", "spread"])
+def test_small_probe_keeps_a_small_workspace(qo, kind):
+    """The device memory that a join of 2^16 rows with 2^24 build keys leaves reserved beside its tables."""
+    import torch
+    rng = np.random.default_rng(5)
+    nr, ns = 1 << 24, 1 << 16
+    rk = keys(kind, nr, rng)
+    j = Join(qo, rk, rk[rng.integers(0, nr, ns)])
+    used = []
+    for route in (L2, AUTO):
+        j.route(route)
+        qo._lib.call("qo_release_workspaces")
+        free = torch.cuda.mem_get_info()[0]
+        j.run()
+        used.append(free - torch.cuda.mem_get_info()[0])
+    assert used[1] < 1.5 * used[0] + (64 << 20), used
