@@ -329,11 +329,17 @@ size_t join_build_ws_bytes(size_t table_bytes, size_t nr) { return join_part_ws_
 // sequence is asynchronous and the same for every input.
 int launch_join_build(void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
                       void *ws, hipStream_t st) {
+    JoinBuild b;
+    QO_TRY(launch_join_build_begin(table, table_bytes, rkey, rpay, nr, b, st));
+    return b.done ? QO_OK : launch_join_build_rest(table, table_bytes, rkey, rpay, nr, b, ws, st);
+}
+
+int launch_join_build_begin(void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
+                            JoinBuild &b, hipStream_t st) {
     const size_t cap = join_table_slots(table_bytes);
     QO_REQUIRE(cap >= 2 && cap <= 0xFFFFFFFFull, "join table of %zu bytes has an unsupported size", table_bytes);
     QO_REQUIRE(nr < cap, "join table with %zu slots cannot hold %zu rows", cap, nr);
     JoinHeader *hdr = static_cast<JoinHeader *>(table);
-    uint64_t *slots = reinterpret_cast<uint64_t *>(hdr + 1);
     const TuneParams tr = tune_get(TUNE_JOIN_RANGE, nr);
     const int part = tune_get(TUNE_JOIN_PART, nr).param;
     if (cap <= kSmallBuildSlots && cap * 8 + 1024 <= (size_t)props().lds_per_block &&
@@ -341,17 +347,28 @@ int launch_join_build(void *table, size_t table_bytes, const int32_t *rkey, cons
         k_build_small<<<1, kSmallBuildThreads, cap * 8, st>>>(rkey, rpay, (uint32_t)nr, hdr, (uint32_t)cap,
                                                               tr.param != PART_NEVER);
         QO_LAUNCHED();
+        b.done = true;
         return QO_OK;
     }
     k_join_init<<<1, 64, 0, st>>>(hdr, cap, nr);
     QO_LAUNCHED();
+    b.range = nr && tr.param != PART_NEVER;
+    if (!b.range) return QO_OK;
+    k_key_range<<<(unsigned)props().cu_count, 256, 0, st>>>(rkey, nr, hdr);
+    QO_LAUNCHED();
+    k_range_decide<<<1, 64, 0, st>>>(hdr, (uint64_t)std::max(1, tr.items) << 20);
+    QO_LAUNCHED();
+    return QO_OK;
+}
+
+int launch_join_build_rest(void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
+                           const JoinBuild &b, void *ws, hipStream_t st) {
+    const size_t cap = join_table_slots(table_bytes);
+    JoinHeader *hdr = static_cast<JoinHeader *>(table);
+    uint64_t *slots = reinterpret_cast<uint64_t *>(hdr + 1);
     const unsigned cus = (unsigned)props().cu_count;
     const unsigned fill_grid = grid_for(cap / 2 + 1, 256, cus * 8);
-    if (nr && tr.param != PART_NEVER) {
-        k_key_range<<<cus, 256, 0, st>>>(rkey, nr, hdr);
-        QO_LAUNCHED();
-        k_range_decide<<<1, 64, 0, st>>>(hdr, (uint64_t)std::max(1, tr.items) << 20);
-        QO_LAUNCHED();
+    if (b.range) {
         // Large tables: slices assembled in LDS and written whole.  Else every
         // tuple stored at its slot, which leaves partial lines to merge.
         bool sliced = false;
@@ -587,12 +604,22 @@ int qo_hj_filter_sort(void *table, size_t table_bytes, const int32_t *rkey, cons
     QO_REQUIRE(table && h_count, "null pointer");
     hipStream_t st = stream_of(s);
     int status = QO_OK;
-    void *ws = workspace(st, join_build_ws_bytes(table_bytes, nr), &status);
+    SortedJoin sorted{table, rkey, rpay, nr, skey, spay, sfilt, ns, flo, fhi, okey, orpay, ospay, out_capacity, st, {}};
+    const bool wanted = sorted.wanted();
+    void *ws = workspace(st, std::max(join_build_ws_bytes(table_bytes, nr), wanted ? SortedJoin::sample_ws_bytes() : 0),
+                         &status);
     if (!ws) return status;
-    QO_TRY(launch_join_build(table, table_bytes, rkey, rpay, nr, ws, st));
+    // The sample needs the key range only: its counts reach the host while the
+    // table is built, so the device does not wait for what the host decides.
+    JoinBuild build;
+    QO_TRY(launch_join_build_begin(table, table_bytes, rkey, rpay, nr, build, st));
+    if (wanted) QO_TRY(sorted.sample(ws));
+    if (!build.done) {
+        QO_TRY(launch_join_build_rest(table, table_bytes, rkey, rpay, nr, build, ws, st));
+        if (wanted) QO_TRY(sorted.built());
+    }
     bool done = false;
-    QO_TRY(sorted_join_try(table, table_bytes, rkey, rpay, nr, skey, spay, sfilt, ns, flo, fhi, okey, orpay, ospay,
-                           out_capacity, h_count, st, &done));
+    if (wanted) QO_TRY(sorted.run(build.done, h_count, &done));
     if (done) {
         if (*h_count > out_capacity) return set_error(QO_ERR_CAPACITY, "join produced %llu rows, capacity %zu",
                                                       (unsigned long long)*h_count, out_capacity);
@@ -618,12 +645,19 @@ int qo_hj_filter_sort(void *table, size_t table_bytes, const int32_t *rkey, cons
     out.k64 = k64;
     out.v32 = v32;
     QO_TRY(launch_join_probe(table, table_bytes, skey, spay, sfilt, ns, flo, fhi, out, d_count, sws, st));
-    uint64_t m = 0;
-    int32_t range[2] = {INT32_MAX, INT32_MIN};  // build key range, when the build measured it
+    // The match count and the build key range, when the build measured it.
+    if (!sorted.host.ptr) QO_TRY(host_words(st, &sorted.host));
+    struct Found {
+        uint64_t m;
+        int32_t range[2];
+    };
+    const Found &found = *static_cast<const Found *>(sorted.host.ptr);
     JoinHeader *hdr = static_cast<JoinHeader *>(table);
-    QO_HIP(hipMemcpyAsync(&m, d_count, 8, hipMemcpyDeviceToHost, st));
-    QO_HIP(hipMemcpyAsync(range, &hdr->rmin, sizeof(range), hipMemcpyDeviceToHost, st));
+    QO_HIP(hipMemcpyAsync(sorted.host.ptr, d_count, 8, hipMemcpyDeviceToHost, st));
+    QO_HIP(hipMemcpyAsync(static_cast<char *>(sorted.host.ptr) + 8, &hdr->rmin, 8, hipMemcpyDeviceToHost, st));
     QO_HIP(hipStreamSynchronize(st));
+    const uint64_t m = found.m;
+    const int32_t range[2] = {found.range[0], found.range[1]};
     *h_count = m;
     if (m > out_capacity) return set_error(QO_ERR_CAPACITY, "join produced %llu rows, capacity %zu",
                                            (unsigned long long)m, out_capacity);

@@ -32,6 +32,8 @@
 // table built by one work-group).
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
+#include <cstring>
 
 #include "qo_internal.hpp"
 #include "qo_join.hpp"
@@ -129,14 +131,25 @@ constexpr int kSjPartBits = 8;
 using SjSplitLds = SplitLdsT<1u << kSjPartBits>;
 
 // Columns -> `parts` buckets of (key - kmin) >> shift.
+// The table the plan counts on, which was not built yet when it was made: off with
+// repeated keys, (-1, -1) build tuples or a table of the other kind.
+struct SjGate {
+    const JoinHeader *hdr;
+    uint32_t mode;
+    QO_DEV bool off() const {
+        return (hdr->has_dups | hdr->sentinel_count | hdr->overflow) != 0 || hdr->mode != mode;
+    }
+};
+
 template <bool HAS_FILTER, class Layout>
 __global__ __launch_bounds__(kSplitThreads) void k_sj_split1(const int32_t *__restrict__ kcol,
                                                              const int32_t *__restrict__ pcol,
                                                              const int32_t *__restrict__ fcol, size_t n, int32_t flo,
                                                              int32_t fhi, bool vec, KeySpan span, int shift,
                                                              uint32_t parts, uint64_t *__restrict__ bucket, Layout out,
-                                                             uint32_t *ctr, FlagOverflow overflow) {
+                                                             uint32_t *ctr, FlagOverflow overflow, SjGate gate) {
     __shared__ SjSplitLds sh;
+    if (gate.off()) return;  // the whole grid
     int32_t key[kSplitJ][4], pay[kSplitJ][4];
     uint32_t pass[kSplitJ];
     load_s_tile<kSplitJ, HAS_FILTER, kSplitThreads>(kcol, pcol, fcol, n, flo, fhi, vec, blockIdx.x, key, pay, pass);
@@ -158,8 +171,9 @@ __global__ __launch_bounds__(kSplitThreads) void k_sj_split2(const uint64_t *__r
                                                              const uint32_t *inctr, uint32_t nb1, uint32_t tpr,
                                                              KeySpan span, int shift, int b2,
                                                              uint64_t *__restrict__ bucket, FixedLayout out,
-                                                             uint32_t *ctr, FlagOverflow overflow) {
+                                                             uint32_t *ctr, FlagOverflow overflow, SjGate gate) {
     __shared__ SjSplitLds sh;
+    if (gate.off()) return;  // the whole grid
     const uint32_t x = blockIdx.x & 7u, q = blockIdx.x >> 3;
     const uint32_t per = kXcdRegions * tpr;
     const uint32_t b = (q / per) * 8u + x, rem = q % per;
@@ -244,13 +258,13 @@ __global__ __launch_bounds__(NT, 8) void k_sj_finish(SjBuckets S, SjBuckets R, u
                                                      PayloadBins pbins, const uint64_t *__restrict__ slots,
                                                      SoaEmit emit, uint32_t *flag, const uint32_t *__restrict__ off,
                                                      uint64_t *status, uint32_t *ticket, uint64_t *d_count,
-                                                     DevCtl *ctl) {
+                                                     DevCtl *ctl, SjGate gate) {
     __shared__ SjLds<DENSE, NT> s;
     // In the ALL form the flag and the bucket's place are three scalar loads in
     // flight together, and the tuples' loads wait for them only.
     const uint32_t fl = *flag;
     const uint32_t o0 = ALL ? off[blockIdx.x] : 0u, o1 = ALL ? off[blockIdx.x + 1] : 0u;
-    if (fl & (kSjOverflow | kSjFull)) return;  // the whole grid
+    if ((fl & (kSjOverflow | kSjFull)) || gate.off()) return;  // the whole grid
     if (!ALL && threadIdx.x == 0) s.tile = atomicAdd(ticket, 1u);
     sj_clear(s);
     __syncthreads();
@@ -300,7 +314,7 @@ struct SjSpread {
     bool even;
     SjSpread(const SjInfo &in, uint32_t last, size_t ns) : info(in) {
         per = (double)ns / (double)std::min<size_t>(ns, kSjSamples);
-        rows = std::min((double)ns, std::max(1.0, per * (in.pass + 4.0 * std::sqrt((double)in.pass))));
+        rows = std::min((double)ns, per * (in.pass + 4.0 * std::sqrt((double)in.pass)));
         // A key seen up to 6 times in the sample may be chance (or a collision); the
         // largest of many counts lies above its own mean.
         hot = in.hot <= 6 ? 0.0 : per * (in.hot - std::sqrt((double)in.hot));
@@ -432,58 +446,79 @@ static SjBufs sj_carve(const SjPlan &p, Carver &cv) {
 
 template <bool HAS_FILTER>
 static int sj_split(const SjPlan &p, const SjSide &side, const SjSideBufs &b, uint32_t *flag, const int32_t *key,
-                    const int32_t *pay, const int32_t *filt, size_t n, int32_t flo, int32_t fhi, hipStream_t st) {
+                    const int32_t *pay, const int32_t *filt, size_t n, int32_t flo, int32_t fhi, const SjGate &gate,
+                    hipStream_t st) {
     const bool vec = (((uintptr_t)key | (uintptr_t)pay | (HAS_FILTER ? (uintptr_t)filt : 0)) & 15u) == 0;
     const size_t tiles = (n + kSplitTile - 1) / kSplitTile;
     QO_REQUIRE(tiles < 0x7FFFFFFFull, "join input too large");
     const FlagOverflow ovf{flag};
     if (!p.b2) {
         k_sj_split1<HAS_FILTER><<<(unsigned)tiles, kSplitThreads, 0, st>>>(
-            key, pay, filt, n, flo, fhi, vec, p.span, p.sh, p.parts1, b.b, FixedLayout{side.capB}, b.ctrB, ovf);
+            key, pay, filt, n, flo, fhi, vec, p.span, p.sh, p.parts1, b.b, FixedLayout{side.capB}, b.ctrB, ovf,
+            gate);
         QO_LAUNCHED();
         return QO_OK;
     }
     k_sj_split1<HAS_FILTER><<<(unsigned)tiles, kSplitThreads, 0, st>>>(key, pay, filt, n, flo, fhi, vec, p.span,
                                                                       p.sh + p.b2, p.parts1, b.a, XcdLayout{side.capA},
-                                                                      b.ctrA, ovf);
+                                                                      b.ctrA, ovf, gate);
     QO_LAUNCHED();
     const uint32_t tpr = (uint32_t)((side.capA + kSplitTile - 1) / kSplitTile);
     const uint64_t grid = (uint64_t)((p.nb1 + 7) / 8) * 8 * kXcdRegions * tpr;
     QO_REQUIRE(grid < 0x7FFFFFFFull, "join input too large");
     k_sj_split2<<<(unsigned)grid, kSplitThreads, 0, st>>>(b.a, side.capA, b.ctrA, p.nb1, tpr, p.span, p.sh, p.b2, b.b,
-                                                          FixedLayout{side.capB}, b.ctrB, ovf);
+                                                          FixedLayout{side.capB}, b.ctrB, ovf, gate);
     QO_LAUNCHED();
     return QO_OK;
 }
 
-int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
-                    const int32_t *skey, const int32_t *spay, const int32_t *sfilt, size_t ns, int32_t flo,
-                    int32_t fhi, int32_t *okey, int32_t *orpay, int32_t *ospay, size_t out_capacity, uint64_t *rows,
-                    hipStream_t st, bool *done) {
-    *done = false;
-    if (nr == 0 || ns < kSjMinRows || ns >= 0xFFFFFFFFull || tune_get(TUNE_JOIN_PART, ns).param != PART_AUTO)
-        return QO_OK;
+constexpr size_t kSjSampleWords = sizeof(SjInfo) / 4 + (size_t(1) << kSjHotBits);
+// The stream's host words: the sample's counts, then the first words of the
+// built table's header, then the result.
+constexpr size_t kSjHostHeader = 2048, kSjHostResult = 3072;
+static_assert(sizeof(SjInfo) <= kSjHostHeader && kSjHostResult + 16 <= kHostWordsBytes, "host words");
+constexpr size_t kSjHeaderBytes = offsetof(JoinHeader, nr);
+
+bool SortedJoin::wanted() const {
+    return nr != 0 && ns >= kSjMinRows && ns < 0xFFFFFFFFull && tune_get(TUNE_JOIN_PART, ns).param == PART_AUTO;
+}
+
+size_t SortedJoin::sample_ws_bytes() { return kSjSampleWords * 4; }
+
+int SortedJoin::sample(void *ws) {
+    QO_TRY(host_words(st, &host));
     const JoinHeader *hdr = static_cast<const JoinHeader *>(table);
-    int status = QO_OK;
-    constexpr size_t kWords = sizeof(SjInfo) / 4 + (size_t(1) << kSjHotBits);
-    void *ws = workspace(st, kWords * 4 + 256, &status);
-    if (!ws) return status;
     SjInfo *d_info = static_cast<SjInfo *>(ws);
     uint32_t *d_keys = reinterpret_cast<uint32_t *>(d_info + 1);
-    SjInfo info;
-    QO_TRY(launch_fill_u32(d_info, 0, kWords, st));
-    if (sfilt)
-        k_sj_sample<true><<<kSjSamples / kSjSampleThreads, kSjSampleThreads, 0, st>>>(hdr, skey, spay, sfilt, ns, flo, fhi, d_info, d_keys);
-    else
-        k_sj_sample<false><<<kSjSamples / kSjSampleThreads, kSjSampleThreads, 0, st>>>(hdr, skey, spay, sfilt, ns, flo, fhi, d_info, d_keys);
+    QO_TRY(launch_fill_u32(d_info, 0, kSjSampleWords, st));
+    constexpr unsigned grid = kSjSamples / kSjSampleThreads;
+    if (sfilt) k_sj_sample<true><<<grid, kSjSampleThreads, 0, st>>>(hdr, skey, spay, sfilt, ns, flo, fhi, d_info, d_keys);
+    else k_sj_sample<false><<<grid, kSjSampleThreads, 0, st>>>(hdr, skey, spay, sfilt, ns, flo, fhi, d_info, d_keys);
     QO_LAUNCHED();
-    QO_HIP(hipMemcpyAsync(&info, d_info, sizeof(info), hipMemcpyDeviceToHost, st));
-    QO_HIP(hipStreamSynchronize(st));
+    QO_HIP(hipMemcpyAsync(host.ptr, d_info, sizeof(SjInfo), hipMemcpyDeviceToHost, st));
+    QO_HIP(hipEventRecord(host.ev[0], st));
+    return QO_OK;
+}
+
+int SortedJoin::built() {
+    QO_HIP(hipMemcpyAsync(static_cast<char *>(host.ptr) + kSjHostHeader, table, kSjHeaderBytes, hipMemcpyDeviceToHost, st));
+    QO_HIP(hipEventRecord(host.ev[1], st));
+    return QO_OK;
+}
+
+int SortedJoin::run(bool table_known, uint64_t *rows, bool *done) {
+    *done = false;
+    QO_HIP(hipEventSynchronize(host.ev[0]));
+    SjInfo info;
+    memcpy(&info, host.ptr, sizeof(info));
     const SjPlan p = sj_plan(info, nr, ns, out_capacity);
     if (!p.on) return QO_OK;
+    const JoinHeader *hdr = static_cast<const JoinHeader *>(table);
+    const SjGate gate{hdr, info.mode};
+    int status = QO_OK;
     Carver size(nullptr);
     sj_carve(p, size);
-    ws = workspace(st, size.off + 256, &status);
+    void *ws = workspace(st, size.off + 256, &status);
     if (!ws) {  // no room for the buckets: the generic path may need less
         (void)hipGetLastError();
         return QO_OK;
@@ -492,9 +527,9 @@ int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, 
     const SjBufs b = sj_carve(p, cv);
     uint32_t *flag = reinterpret_cast<uint32_t *>(b.res + 1);
     QO_TRY(launch_fill_u32(b.res, 0, b.clear_words, st));
-    if (sfilt) QO_TRY(sj_split<true>(p, p.s, b.s, flag, skey, spay, sfilt, ns, flo, fhi, st));
-    else QO_TRY(sj_split<false>(p, p.s, b.s, flag, skey, spay, nullptr, ns, 0, 0, st));
-    if (!p.dense) QO_TRY(sj_split<false>(p, p.r, b.r, flag, rkey, rpay, nullptr, nr, 0, 0, st));
+    if (sfilt) QO_TRY(sj_split<true>(p, p.s, b.s, flag, skey, spay, sfilt, ns, flo, fhi, gate, st));
+    else QO_TRY(sj_split<false>(p, p.s, b.s, flag, skey, spay, nullptr, ns, 0, 0, gate, st));
+    if (!p.dense) QO_TRY(sj_split<false>(p, p.r, b.r, flag, rkey, rpay, nullptr, nr, 0, 0, gate, st));
     const SoaEmit out{okey, orpay, ospay, out_capacity};
     const SjBuckets sb{b.s.b, p.s.capB, b.s.ctrB}, rb{b.r.b, p.r.capB, b.r.ctrB};
     const uint64_t *slots = reinterpret_cast<const uint64_t *>(hdr + 1);
@@ -505,7 +540,7 @@ int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, 
     }
 #define QO_SJ_FINISH(D, T, A)                                                                                       \
     k_sj_finish<D, T, A><<<p.nb, T, 0, st>>>(sb, rb, p.nb, p.sh, p.span, p.pay, slots, out, flag, b.off, b.status, b.ticket, \
-                                             b.res, dev_ctl())
+                                             b.res, dev_ctl(), gate)
     if (p.all) {
         if (p.nt == 512) QO_SJ_FINISH(true, 512, true);
         else QO_SJ_FINISH(true, 1024, true);
@@ -518,8 +553,15 @@ int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, 
     }
 #undef QO_SJ_FINISH
     QO_LAUNCHED();
-    uint64_t res[2];
-    QO_HIP(hipMemcpyAsync(res, b.res, sizeof(res), hipMemcpyDeviceToHost, st));
+    const uint64_t *res = reinterpret_cast<const uint64_t *>(static_cast<const char *>(host.ptr) + kSjHostResult);
+    QO_HIP(hipMemcpyAsync(const_cast<uint64_t *>(res), b.res, 16, hipMemcpyDeviceToHost, st));
+    if (!table_known) {
+        // Off on the device too then, and the caller's probe is queued without a gap.
+        QO_HIP(hipEventSynchronize(host.ev[1]));
+        JoinHeader h;
+        memcpy(&h, static_cast<const char *>(host.ptr) + kSjHostHeader, kSjHeaderBytes);
+        if ((h.has_dups | h.sentinel_count | h.overflow) || h.mode != info.mode) return QO_OK;
+    }
     QO_HIP(hipStreamSynchronize(st));
     // Nothing was written then.  kSjFull: the rows are too many if every tuple counted has a match.
     const uint32_t f = (uint32_t)res[1];

@@ -60,6 +60,14 @@ void *workspace(hipStream_t s, size_t bytes, int *status);
 // whose own temporaries must outlive the operators it calls, which take slot 0
 // (qo_plan_execute).
 constexpr int kWorkspaceSlots = 2;
+// Pinned host memory and events of a stream, for words a call reads back while the
+// device goes on.  Given back with the stream's workspaces.
+constexpr size_t kHostWordsBytes = 4096;
+struct HostWords {
+    void *ptr = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+};
+int host_words(hipStream_t s, HostWords *out);
 void *workspace_slot(int slot, hipStream_t s, size_t bytes, int *status);
 
 // Carves aligned sub-buffers out of a workspace; a null base only measures.
@@ -206,16 +214,45 @@ int launch_join_probe(const void *table, size_t table_bytes, const int32_t *skey
                       const int32_t *sfilt, size_t ns, int32_t flo, int32_t fhi, const JoinOut &out,
                       uint64_t *d_count, void *ws, hipStream_t st);
 
+// Build of a join table in two calls.  The first finds the key range and the
+// table's kind as far as the range decides it (a small table is built whole:
+// *done), the second the table; both with the parameters of the first.
+struct JoinBuild {
+    bool done = false;   // the table was built whole
+    bool range = false;  // the key range was looked at
+};
+int launch_join_build_begin(void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
+                            JoinBuild &b, hipStream_t st);
+int launch_join_build_rest(void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
+                           const JoinBuild &b, void *ws, hipStream_t st);
+
 // Sorted join against the table built from (rkey, rpay), by a split in key
-// order (join_sorted.hip).  *done = false when its conditions do not hold
-// (repeated build keys, few or unevenly spread S keys, a bucket that
-// overflowed): nothing was written and the probe and sort have to run.  Else
-// *rows is the match count and the first out_capacity rows are written.  Uses
-// the stream's workspace (slot 0) and synchronises the stream.
-int sorted_join_try(const void *table, size_t table_bytes, const int32_t *rkey, const int32_t *rpay, size_t nr,
-                    const int32_t *skey, const int32_t *spay, const int32_t *sfilt, size_t ns, int32_t flo,
-                    int32_t fhi, int32_t *okey, int32_t *orpay, int32_t *ospay, size_t out_capacity, uint64_t *rows,
-                    hipStream_t st, bool *done);
+// order (join_sorted.hip).
+struct SortedJoin {
+    const void *table;
+    const int32_t *rkey, *rpay;
+    size_t nr;
+    const int32_t *skey, *spay, *sfilt;
+    size_t ns;
+    int32_t flo, fhi;
+    int32_t *okey, *orpay, *ospay;
+    size_t out_capacity;
+    hipStream_t st;
+    HostWords host;
+
+    bool wanted() const;                 // the call is one for it, as far as the host can tell
+    static size_t sample_ws_bytes();
+    // Samples S, behind launch_join_build_begin, in `ws`, which the rest of the
+    // build may use again.
+    int sample(void *ws);
+    int built();                         // behind launch_join_build_rest
+    // *done = false when its conditions do not hold (repeated build keys, unevenly
+    // spread S keys, a bucket that overflowed): nothing was written and the probe
+    // and sort have to run.  Else *rows is the match count, and they are written
+    // unless there are more than out_capacity.  table_known: the table was built
+    // whole before the sample.  Uses the stream's workspace (slot 0).
+    int run(bool table_known, uint64_t *rows, bool *done);
+};
 
 }  // namespace qo
 

@@ -33,6 +33,13 @@ struct Ws {
     size_t bytes = 0;
 };
 std::map<std::pair<int, StreamKey>, Ws> g_ws;  // (slot, stream) -> workspace
+std::map<StreamKey, HostWords> g_host;
+
+void free_host_words(const HostWords &h) {
+    if (h.ptr) (void)hipHostFree(h.ptr);
+    for (hipEvent_t e : h.ev)
+        if (e) (void)hipEventDestroy(e);
+}
 void load_tune_file(const char *arch);
 }  // namespace
 
@@ -152,6 +159,16 @@ void *workspace_slot(int slot, hipStream_t s, size_t bytes, int *status) {
     }
     w.bytes = grow;
     return w.ptr;
+}
+
+int host_words(hipStream_t s, HostWords *out) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    HostWords &h = g_host[stream_key_of(s)];
+    if (!h.ptr) QO_HIP(hipHostMalloc(&h.ptr, kHostWordsBytes, hipHostMallocDefault));
+    for (hipEvent_t &e : h.ev)
+        if (!e) QO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    *out = h;
+    return QO_OK;
 }
 
 __global__ void k_fill_u32(uint32_t *dst, uint32_t v, size_t n) {
@@ -400,6 +417,11 @@ int qo_stream_destroy(qo_stream s) {
             if (it->second.ptr) (void)hipFree(it->second.ptr);
             g_ws.erase(it);
         }
+        auto h = g_host.find(stream_key_of(st));
+        if (h != g_host.end()) {
+            free_host_words(h->second);
+            g_host.erase(h);
+        }
     }
     QO_HIP(hipStreamDestroy(st));
     return QO_OK;
@@ -471,6 +493,8 @@ int qo_release_workspaces(void) {
     for (auto &kv : g_ws)
         if (kv.second.ptr) (void)hipFree(kv.second.ptr);
     g_ws.clear();
+    for (auto &kv : g_host) free_host_words(kv.second);
+    g_host.clear();
     return QO_OK;
 }
 

@@ -100,3 +100,25 @@ def test_small_probe_keeps_a_small_workspace(qo, kind):
         j.run()
         used.append(free - torch.cuda.mem_get_info()[0])
     assert used[1] < 1.5 * used[0] + (64 << 20), used
+
+
+def cases(nr, ns, kind):
+    """Joins that leave the sorted join: (name, R keys, S keys)."""
+    rng = np.random.default_rng(nr)
+    rk = keys(kind, nr, rng)
+    sk = rk[rng.integers(0, nr, ns)]
+    dup = rk.copy()
+    dup[:3] = dup[-3:]
+    yield "repeated build keys", dup, sk
+    hot = sk.copy()
+    hot[: ns // 20] = rk[5]                  # more rows than a bucket holds
+    yield "hot key", rk, rng.permutation(hot)
+    yield "few keys referenced", rk, np.sort(rk)[rng.integers(0, 40, ns)]
+
+
+@pytest.mark.parametrize("kind", ["dense", "spread"])
+@pytest.mark.parametrize("nr,ns", [(200_000, 2_000_000), (1_500_000, 6_000_000)])
+def test_joins_that_leave_the_sorted_join(qo, kind, nr, ns):
+    for name, rk, sk in cases(nr, ns, kind):
+        print(name, flush=True)
+        compare(qo, rk, sk, 1.12)
