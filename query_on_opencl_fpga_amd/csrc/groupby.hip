@@ -103,9 +103,10 @@ QO_DEV void g_update(GEntry *t, uint64_t mask, uint32_t key, uint64_t cnt, uint6
 // on, 0.02 % further), so the wave enters the probe loop only when one of its
 // lanes is further out.  `lkey` holds C + 2 words; the two past the end stay
 // kEmptyKey, which no looked-up key equals, so the second read needs no wrap.
-// TWO costs LDS bank cycles where keys do sit at home (a few groups).
+// TWO costs LDS bank cycles where keys do sit at home (a few groups).  With
+// `stop` the probe loop is left out once *stop is set.
 template <int C, bool TWO = false>
-QO_DEV int l_slot(uint32_t *lkey, uint32_t key, int probes, int skip) {
+QO_DEV int l_slot(uint32_t *lkey, uint32_t key, int probes, int skip, const volatile uint32_t *stop = nullptr) {
     static_assert((C & (C - 1)) == 0, "power-of-two table");
     constexpr int kBits = __builtin_ctz(C);
     uint32_t h = ((key * 0x9E3779B9u) << skip) >> (32 - kBits);
@@ -117,6 +118,7 @@ QO_DEV int l_slot(uint32_t *lkey, uint32_t key, int probes, int skip) {
     } else if (lkey[h] == key) {
         return (int)h;
     }
+    if (stop && *stop) return -1;
     for (int p = 0; p < probes; ++p) {
         uint32_t k = lkey[h];
         if (k == key) return (int)h;
@@ -227,9 +229,12 @@ QO_DEV void pack_empty(PackTable<C> &L, int s, unsigned long long w) {
     atomicAdd(&L.t.sum[s], (w & ((1ull << 48) - 1)) - ((unsigned long long)c << 31));
 }
 
-template <int C>
+// `full` (may be null): a tuple that finds no slot sets it and *stop and is left
+// out, as are the block's further ones that are not in their home slot; the caller
+// runs all tuples again in shares (k_groupby_hash).
+template <int C, int SKIP = 0>
 QO_DEV void pack_add(PackTable<C> &L, int32_t k, int32_t v, int probes, GEntry *gt, uint64_t gmask,
-                     uint32_t *overflow, PackSeen &seen) {
+                     uint32_t *overflow, uint32_t *full, uint32_t *stop, PackSeen &seen) {
     if constexpr (!PackTable<C>::kPacked) {
         ltable_add<C>(L.t, k, v, probes, gt, gmask, overflow);
         return;
@@ -238,7 +243,7 @@ QO_DEV void pack_add(PackTable<C> &L, int32_t k, int32_t v, int probes, GEntry *
         pack_empty(L, seen.slot, atomicExch(&L.pack[seen.slot], 0ull));
         seen.hi = 0;
     }
-    const int s = (uint32_t)k == kEmptyKey ? -1 : l_slot<C>(L.t.key, (uint32_t)k, probes, 0);
+    const int s = (uint32_t)k == kEmptyKey ? -1 : l_slot<C>(L.t.key, (uint32_t)k, probes, SKIP, full ? stop : nullptr);
     if (s >= 0) {
         const int32_t lo = L.t.mn[s], hi = L.t.mx[s];  // read first, as in ltable_add
         const unsigned long long old =
@@ -247,6 +252,8 @@ QO_DEV void pack_add(PackTable<C> &L, int32_t k, int32_t v, int probes, GEntry *
         seen.slot = s;
         if (v < lo) atomicMin(&L.t.mn[s], v);
         if (v > hi) atomicMax(&L.t.mx[s], v);
+    } else if (full && (uint32_t)k != kEmptyKey) {
+        if (*stop == 0) *full = *stop = 1u;
     } else {
         g_update(gt, gmask, (uint32_t)k, 1, (uint64_t)(int64_t)v, v, v, overflow);
     }
@@ -463,12 +470,12 @@ struct DomAcc {
     }
 };
 
-// Block totals of the dominant key, added once to its LDS entry (or to the
-// global table when it has none).  All NT threads call it; the caller
-// synchronises before reading the table.
+// Block totals of the dominant key, added once to its LDS entry (or, when it has
+// none, to the global table or to what `full` says is left out, see pack_add).
+// All NT threads call it; the caller synchronises before reading the table.
 template <int C, int NT>
 QO_DEV void dom_merge(LTable<C> &L, const DomAcc &a, uint32_t dom, int probes, int skip, GEntry *gt, uint64_t gmask,
-                      uint32_t *overflow) {
+                      uint32_t *overflow, uint32_t *full = nullptr) {
     __shared__ uint64_t s_ds[NT / kWave];
     __shared__ uint32_t s_dc[NT / kWave];
     __shared__ int32_t s_dmn[NT / kWave], s_dmx[NT / kWave];
@@ -495,6 +502,8 @@ QO_DEV void dom_merge(LTable<C> &L, const DomAcc &a, uint32_t dom, int probes, i
                 atomicAdd(&L.sum[sl], (unsigned long long)ts);
                 atomicMin(&L.mn[sl], tmn);
                 atomicMax(&L.mx[sl], tmx);
+            } else if (full && dom != kEmptyKey) {
+                *full = 1u;
             } else {
                 g_update(gt, gmask, dom, tc, ts, tmn, tmx, overflow);
             }
@@ -509,16 +518,33 @@ QO_DEV void dom_merge(LTable<C> &L, const DomAcc &a, uint32_t dom, int probes, i
 // lanes on one LDS address.
 // FILT: only tuples with lo <= filt[i] <= hi are aggregated (the filter is
 // fused: its column is read beside key and value, no compaction pass).
-template <int C, bool VEC, int NT, bool FILT = false>
+//
+// Tables that hold more than half their slots of groups (`full` given) say so
+// when the keys are more than the capacity promised and do not fit.  Tuple by
+// tuple such keys went to the global table (2^24 tuples, capacity 3000: 3500 keys
+// 0.16 ms, 6000 keys 47).  A second launch (SHARE) then takes every tuple again,
+// a quarter of the keys per block by two bits of their hash, and replaces the
+// blocks' groups.  Keys of the empty-marker pattern were counted by the first.
+constexpr int kShareBits = 2;
+template <int C, bool VEC, int NT, bool FILT = false, bool SHARE = false>
 __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__ key, const int32_t *__restrict__ val,
                                                       size_t n, GEntry *gt, uint64_t gmask, int probes,
-                                                      uint32_t *overflow, Partials parts,
+                                                      uint32_t *overflow, uint32_t *full, Partials parts,
                                                       const int32_t *__restrict__ filt = nullptr, int32_t flo = 0,
                                                       int32_t fhi = 0) {
     extern __shared__ unsigned char s_raw[];
+    if (SHARE) {
+        if (*full == 0) return;  // the whole grid
+        full = nullptr;          // what finds no slot now goes to the global table
+    }
+    constexpr int kSkip = SHARE ? kShareBits : 0;
+    const uint32_t share = blockIdx.x & ((1u << kShareBits) - 1u);
+    // Blocks that walk the input: all of them, or one of each share.
+    const uint32_t walk = SHARE ? blockIdx.x >> kShareBits : blockIdx.x, walks = SHARE ? gridDim.x >> kShareBits : gridDim.x;
     PackTable<C> &P = *reinterpret_cast<PackTable<C> *>(s_raw);
     LTable<C> &L = P.t;
-    __shared__ uint32_t s_dom, s_dom2, s_heavy;
+    __shared__ uint32_t s_dom, s_dom2, s_heavy, s_stop;
+    if (threadIdx.x == 0) s_stop = 0;
     if (threadIdx.x < kWave) {
         unsigned bc, bc2;
         uint32_t d2;
@@ -542,13 +568,15 @@ __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__
         auto add_one = [&](int32_t k, int32_t v) {
             if (kHeavy && (uint32_t)k == dom) acc.add(v);
             else if (kHeavy && (uint32_t)k == dom2) acc2.add(v);
-            else pack_add<C>(P, k, v, probes, gt, gmask, overflow, seen);
+            else pack_add<C, kSkip>(P, k, v, probes, gt, gmask, overflow, full, &s_stop, seen);
         };
         auto add = [&](int32_t k, int32_t v, int32_t f) {
+            if (SHARE && ((uint32_t)k == kEmptyKey || fib_slot((uint32_t)k, kShareBits) != share)) return;
             if (!FILT || (f >= flo && f <= fhi)) add_one(k, v);
         };
-        const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-        const size_t stride = (size_t)gridDim.x * blockDim.x;
+        if (SHARE && walk >= walks) return;  // block-uniform: the grid's last few blocks
+        const size_t tid = (size_t)walk * blockDim.x + threadIdx.x;
+        const size_t stride = (size_t)walks * blockDim.x;
         size_t from = 0;
         if (VEC) {
             const size_t nv = n / 4;
@@ -586,10 +614,10 @@ __global__ __launch_bounds__(NT) void k_groupby_hash(const int32_t *__restrict__
         }
         for (size_t e = from + tid; e < n; e += stride) add(key[e], val[e], FILT ? filt[e] : 0);
         if (kHeavy) {
-            dom_merge<C, NT>(L, acc, dom, probes, 0, gt, gmask, overflow);
+            dom_merge<C, NT>(L, acc, dom, probes, kSkip, gt, gmask, overflow, full);
             if (dom2 != dom) {  // block-uniform
                 __syncthreads();  // dom_merge's staging is reused
-                dom_merge<C, NT>(L, acc2, dom2, probes, 0, gt, gmask, overflow);
+                dom_merge<C, NT>(L, acc2, dom2, probes, kSkip, gt, gmask, overflow, full);
             }
         }
     };
@@ -1176,6 +1204,8 @@ struct HashPlan {
     int C = 0;
     unsigned grid = 0;
     bool merge = false;
+    bool share = false;  // a second launch for keys that do not fit (see k_groupby_hash)
+    int probes = 0;
 };
 constexpr int kHashThreads = 1024;
 // Fewer blocks than this merge straight into the global table: the merge launch
@@ -1196,6 +1226,12 @@ static HashPlan hash_plan(size_t n, size_t groups) {
     h.grid = grid_for(n, kHashThreads * 4, (unsigned)props().cu_count * (unsigned)std::max(1, tp.param));
     h.merge = groups <= kMergeMaxGroups && h.grid >= merge_min_blocks(groups) && h.grid <= kMergeMaxBlocks &&
               n < 0xFFFFFFFFull;
+    // Low cardinality: the LDS table holds every group.  High cardinality: it
+    // caches the keys seen first and the rest go straight to global.  A table past
+    // half full is looked through for 512 slots only: with 3072 keys in 4096 slots
+    // no cluster is that long, and more keys than it holds would each look at all.
+    h.share = h.C == 4096 && groups > 1024 && groups <= kGroupbyDirect && h.merge;
+    h.probes = groups * 4 <= (size_t)h.C * 3 ? (h.share || groups * 2 > (size_t)h.C ? 512 : h.C) : 8;
     return h;
 }
 
@@ -1277,12 +1313,10 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
         const int C = h.C;
         constexpr int block = kHashThreads;
         const unsigned grid = h.grid;
-        // Low cardinality: the LDS table holds every group.  High cardinality:
-        // it caches the keys seen first and the rest go straight to global.
-        const int probes = group_capacity * 4 <= (size_t)C * 3 ? C : 8;
-#define QO_GBH(CC, V, F)                                                                                    \
-    k_groupby_hash<CC, V, block, F><<<grid, block, sizeof(PackTable<CC>), st>>>(key, val, n, gt, p.gmask, probes, \
-                                                                             overflow, b.parts, filt, flo, fhi)
+        uint32_t *full = h.share ? reinterpret_cast<uint32_t *>(counters + 2) : nullptr;
+#define QO_GBH(CC, V, F, ...)                                                                               \
+    k_groupby_hash<CC, V, block, F, ##__VA_ARGS__><<<grid, block, sizeof(PackTable<CC>), st>>>(key, val, n, gt, p.gmask, \
+                                                                             h.probes, overflow, full, b.parts, filt, flo, fhi)
         if (C == 4096) {
             if (filt) {
                 if (vec) QO_GBH(4096, true, true);
@@ -1300,8 +1334,18 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
                 else QO_GBH(2048, false, false);
             }
         }
-#undef QO_GBH
         QO_LAUNCHED();
+        if (h.share) {
+            if (filt) {
+                if (vec) QO_GBH(4096, true, true, true);
+                else QO_GBH(4096, false, true, true);
+            } else {
+                if (vec) QO_GBH(4096, true, false, true);
+                else QO_GBH(4096, false, false, true);
+            }
+            QO_LAUNCHED();
+        }
+#undef QO_GBH
         if (b.parts.ent) {
             k_groupby_merge<<<kMergeParts, kMergeThreads, 0, st>>>(b.parts, grid, (uint32_t)C, gt, p.gmask, overflow);
             QO_LAUNCHED();
