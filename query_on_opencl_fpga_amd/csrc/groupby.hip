@@ -1166,16 +1166,17 @@ struct GbPartPlan {
 // With a filter the partition stays one pass (at most kOnePassParts buckets,
 // whose LDS tables spill to the global table beyond 2^20 groups): the filter is
 // fused into that pass.
-static GbPartPlan groupby_part_plan(size_t group_capacity, size_t n, bool filtered) {
+static GbPartPlan groupby_part_plan(const GroupbyCall &c) {
+    const size_t group_capacity = c.capacity, n = c.n;
     GbPartPlan p;
-    const TuneParams tp = tune_get(TUNE_GROUPBY_PART, n);
+    const TuneParams &tp = c.part;
     if (tp.param == PART_NEVER || n == 0 || n >= 0xFFFFFFFFull || group_capacity < 2) return p;
     // Up to kGroupbyDirect groups one LDS table of 4096 slots holds them all and no
     // tuple moves: 2^28 tuples, 2000 groups 2247 -> 382 us, 3000 groups 1911 -> 759;
     // 2^20 tuples, 2000 groups 268 -> 56.
     if (tp.param != PART_ALWAYS && (group_capacity <= kGroupbyDirect || n < (size_t(1) << 20))) return p;
     const size_t target = (size_t)std::max(16, tp.items);
-    const int lmax = filtered ? __builtin_ctz(kOnePassParts) : 2 * kMaxSplitBits;
+    const int lmax = c.filtered ? __builtin_ctz(kOnePassParts) : 2 * kMaxSplitBits;
     int L = 1;
     while (L < lmax && (group_capacity >> L) > target) ++L;
     p.on = true;
@@ -1218,9 +1219,10 @@ constexpr int kHashThreads = 1024;
 constexpr size_t kMergeMaxGroups = (size_t)kMergeParts * kMergeSlots;
 static unsigned merge_min_blocks(size_t groups) { return groups < 1600 ? 76u - (unsigned)(groups * 43 / 1000) : 8u; }
 
-static HashPlan hash_plan(size_t n, size_t groups) {
+static HashPlan hash_plan(const GroupbyCall &c) {
+    const size_t groups = c.capacity, n = c.n;
     HashPlan h;
-    const TuneParams tp = tune_get(TUNE_GROUPBY, n);
+    const TuneParams &tp = c.direct;
     const bool large = tp.items >= 4096 || (groups > 1024 && groups <= kGroupbyDirect && n >= (size_t(1) << 20));
     h.C = large && (size_t)props().lds_per_block >= sizeof(PackTable<4096>) + 8192 ? 4096 : 2048;
     h.grid = grid_for(n, kHashThreads * 4, (unsigned)props().cu_count * (unsigned)std::max(1, tp.param));
@@ -1235,8 +1237,8 @@ static HashPlan hash_plan(size_t n, size_t groups) {
     return h;
 }
 
-static GroupbyBufs groupby_carve(const GroupbyPlan &p, const GbPartPlan &pp, size_t group_capacity, size_t n,
-                                 Carver &cv) {
+static GroupbyBufs groupby_carve(const GroupbyCall &c, const GroupbyPlan &p, const GbPartPlan &pp, Carver &cv) {
+    const size_t group_capacity = c.capacity, n = c.n;
     GroupbyBufs b;
     b.gt = cv.take<GEntry>(p.entries);
     b.counters = cv.take<uint64_t>(4);
@@ -1250,27 +1252,32 @@ static GroupbyBufs groupby_carve(const GroupbyPlan &p, const GbPartPlan &pp, siz
         b.cch = cv.take<uint32_t>(nb + 1);
         b.cpre = cv.take<uint32_t>(nb + 1);
         b.scan_ws = cv.take<char>(scan_workspace_bytes(nb + 1));
-    } else if (const HashPlan h = hash_plan(n, group_capacity); n && h.merge) {
+    } else if (const HashPlan h = hash_plan(c); n && h.merge) {
         b.parts.ent = cv.take<GEntry>((size_t)h.grid * h.C);
         b.parts.start = cv.take<uint32_t>((size_t)h.grid * (kMergeParts + 1));
     }
     return b;
 }
 
-size_t groupby_ws_bytes(size_t group_capacity, size_t n, bool filtered) {
+GroupbyCall groupby_call(size_t group_capacity, size_t n, bool filtered) {
+    return GroupbyCall{group_capacity, n, filtered, tune_get(TUNE_GROUPBY_PART, n), tune_get(TUNE_GROUPBY, n)};
+}
+
+size_t groupby_ws_bytes(const GroupbyCall &c) {
     Carver cv(nullptr);
-    groupby_carve(groupby_plan(group_capacity), groupby_part_plan(group_capacity, n, filtered), group_capacity, n,
-                  cv);
+    groupby_carve(c, groupby_plan(c.capacity), groupby_part_plan(c), cv);
     return cv.off + 256;
 }
 
-int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t group_capacity, int32_t *okey,
-                   int64_t *ocount, int64_t *osum, int32_t *omin, int32_t *omax, uint64_t *d_num, void *ws,
-                   hipStream_t st, const int32_t *filt, int32_t flo, int32_t fhi) {
-    GroupbyPlan p = groupby_plan(group_capacity);
-    const GbPartPlan pp = groupby_part_plan(group_capacity, n, filt != nullptr);
+int launch_groupby(const GroupbyCall &c, const int32_t *key, const int32_t *val, int32_t *okey, int64_t *ocount,
+                   int64_t *osum, int32_t *omin, int32_t *omax, uint64_t *d_num, void *ws, hipStream_t st,
+                   const int32_t *filt, int32_t flo, int32_t fhi) {
+    QO_REQUIRE(c.filtered == (filt != nullptr), "group-by planned for another filter");
+    const size_t group_capacity = c.capacity, n = c.n;
+    const GroupbyPlan p = groupby_plan(group_capacity);
+    const GbPartPlan pp = groupby_part_plan(c);
     Carver cv(ws);
-    const GroupbyBufs b = groupby_carve(p, pp, group_capacity, n, cv);
+    const GroupbyBufs b = groupby_carve(c, p, pp, cv);
     GEntry *gt = b.gt;
     uint64_t *counters = b.counters;
     uint64_t *list = b.list;
@@ -1308,7 +1315,7 @@ int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t grou
             reinterpret_cast<unsigned long long *>(counters), group_capacity);
         QO_LAUNCHED();
     } else if (n) {
-        const HashPlan h = hash_plan(n, group_capacity);
+        const HashPlan h = hash_plan(c);
         const bool vec = ((uintptr_t)key % 16 == 0) && ((uintptr_t)val % 16 == 0) && ((uintptr_t)filt % 16 == 0);
         const int C = h.C;
         constexpr int block = kHashThreads;
@@ -1677,10 +1684,10 @@ int qo_groupby_agg_filtered(const int32_t *key, const int32_t *val, const int32_
     QO_REQUIRE(group_capacity < (size_t(1) << 31), "group capacity too large");
     hipStream_t st = stream_of(s);
     int status = QO_OK;
-    void *ws = workspace(st, groupby_ws_bytes(group_capacity, n, filt != nullptr), &status);
+    const GroupbyCall c = groupby_call(group_capacity, n, filt != nullptr);
+    void *ws = workspace(st, groupby_ws_bytes(c), &status);
     if (!ws) return status;
-    return launch_groupby(key, val, n, group_capacity, okey, ocount, osum, omin, omax, d_numGroups, ws, st, filt, lo,
-                          hi);
+    return launch_groupby(c, key, val, okey, ocount, osum, omin, omax, d_numGroups, ws, st, filt, lo, hi);
 }
 
 int qo_group_startpos(const qo_record *sorted, size_t n, int32_t *startPos, uint64_t *d_numGroups, qo_stream s) {

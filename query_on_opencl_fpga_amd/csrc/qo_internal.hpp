@@ -160,10 +160,18 @@ int sort_join_rows_ws(int32_t *key, int32_t *rpay, int32_t *spay, size_t m, void
 
 // Hash group-by with caller workspace (groupby.hip); with filt, only tuples
 // with lo <= filt[i] <= hi are aggregated (the filter is fused).
-size_t groupby_ws_bytes(size_t group_capacity, size_t n, bool filtered = false);
-int launch_groupby(const int32_t *key, const int32_t *val, size_t n, size_t group_capacity, int32_t *okey,
-                   int64_t *ocount, int64_t *osum, int32_t *omin, int32_t *omax, uint64_t *d_num, void *ws,
-                   hipStream_t st, const int32_t *filt = nullptr, int32_t flo = 0, int32_t fhi = 0);
+// One call's parameters, read from the tune table once: its workspace and its
+// launches agree whatever another thread sets in between.
+struct GroupbyCall {
+    size_t capacity, n;
+    bool filtered;
+    TuneParams part, direct;
+};
+GroupbyCall groupby_call(size_t group_capacity, size_t n, bool filtered = false);
+size_t groupby_ws_bytes(const GroupbyCall &c);
+int launch_groupby(const GroupbyCall &c, const int32_t *key, const int32_t *val, int32_t *okey, int64_t *ocount,
+                   int64_t *osum, int32_t *omin, int32_t *omax, uint64_t *d_num, void *ws, hipStream_t st,
+                   const int32_t *filt = nullptr, int32_t flo = 0, int32_t fhi = 0);
 
 // Join table helpers (join.hip).
 size_t join_table_slots(size_t table_bytes);

@@ -245,7 +245,7 @@ static size_t request_bytes(qo_server *sv, const qo_request &r) {
     if (r.kind == QO_Q_FILTER) return 4096;
     if (r.kind == QO_Q_GROUPBY) {
         size_t G = A.d.group_capacity ? A.d.group_capacity : 1;
-        return G * 28 + groupby_ws_bytes(G, A.d.n, groupby_filter(A.d, r) != nullptr) + 8192;
+        return G * 28 + groupby_ws_bytes(groupby_call(G, A.d.n, groupby_filter(A.d, r) != nullptr)) + 8192;
     }
     const Table &B = sv->tables[r.table_b];
     qo_join_query q{};
@@ -307,14 +307,14 @@ static int launch_batch(qo_server *sv, Batch &b, hipStream_t st) {
     cv.take<ResSlot>(n);
     cv.take<FQuery>(fi.size() + 1);
     cv.take<uint32_t>(64);
-    std::vector<size_t> gsz;
+    std::vector<GroupbyCall> gcall;
     for (int i : gi) {
         size_t G = sv->tables[live[i]->r.table_a].d.group_capacity;
         cv.take<int32_t>(G); cv.take<int64_t>(G); cv.take<int64_t>(G); cv.take<int32_t>(G); cv.take<int32_t>(G);
         cv.take<uint64_t>(1);
         const qo_table_desc &A = sv->tables[live[i]->r.table_a].d;
-        cv.take<char>(groupby_ws_bytes(G, A.n, groupby_filter(A, live[i]->r) != nullptr));
-        gsz.push_back(G);
+        gcall.push_back(groupby_call(G, A.n, groupby_filter(A, live[i]->r) != nullptr));
+        cv.take<char>(groupby_ws_bytes(gcall.back()));
     }
     for (auto &q : b.jq) {
         cv.take<int32_t>(q.out_capacity); cv.take<int32_t>(q.out_capacity); cv.take<int32_t>(q.out_capacity);
@@ -366,7 +366,7 @@ static int launch_batch(qo_server *sv, Batch &b, hipStream_t st) {
     for (size_t k = 0; k < gi.size(); ++k) {
         const qo_request &r = live[gi[k]]->r;
         const qo_table_desc &A = sv->tables[r.table_a].d;
-        size_t G = gsz[k];
+        const size_t G = gcall[k].capacity;
         int32_t *okey = c2.take<int32_t>(G);
         int64_t *ocnt = c2.take<int64_t>(G);
         int64_t *osum = c2.take<int64_t>(G);
@@ -374,8 +374,8 @@ static int launch_batch(qo_server *sv, Batch &b, hipStream_t st) {
         int32_t *omax = c2.take<int32_t>(G);
         uint64_t *num = c2.take<uint64_t>(1);
         const int32_t *filt = groupby_filter(A, r);
-        void *ws = c2.take<char>(groupby_ws_bytes(G, A.n, filt != nullptr));
-        QO_TRY(launch_groupby(A.grp, A.val, A.n, G, okey, ocnt, osum, omin, omax, num, ws, st, filt, r.lo, r.hi));
+        void *ws = c2.take<char>(groupby_ws_bytes(gcall[k]));
+        QO_TRY(launch_groupby(gcall[k], A.grp, A.val, okey, ocnt, osum, omin, omax, num, ws, st, filt, r.lo, r.hi));
         k_s_checksum_groupby<<<std::min<unsigned>(kGrid, (unsigned)((G + 255) / 256) + 1), 256, 0, st>>>(
             okey, ocnt, osum, omin, omax, num, G, b.d_res + slot_of(live[gi[k]]));
         QO_LAUNCHED();
