@@ -1174,7 +1174,10 @@ static GbPartPlan groupby_part_plan(const GroupbyCall &c) {
     // Up to kGroupbyDirect groups one LDS table of 4096 slots holds them all and no
     // tuple moves: 2^28 tuples, 2000 groups 2247 -> 382 us, 3000 groups 1911 -> 759;
     // 2^20 tuples, 2000 groups 268 -> 56.
-    if (tp.param != PART_ALWAYS && (group_capacity <= kGroupbyDirect || n < (size_t(1) << 20))) return p;
+    // (Without the merge launch blocks x groups global atomics end such a call: 1024 is
+    // the limit then.)
+    const size_t direct = c.merge ? kGroupbyDirect : 1024;
+    if (tp.param != PART_ALWAYS && (group_capacity <= direct || n < (size_t(1) << 20))) return p;
     const size_t target = (size_t)std::max(16, tp.items);
     const int lmax = c.filtered ? __builtin_ctz(kOnePassParts) : 2 * kMaxSplitBits;
     int L = 1;
@@ -1226,7 +1229,7 @@ static HashPlan hash_plan(const GroupbyCall &c) {
     const bool large = tp.items >= 4096 || (groups > 1024 && groups <= kGroupbyDirect && n >= (size_t(1) << 20));
     h.C = large && (size_t)props().lds_per_block >= sizeof(PackTable<4096>) + 8192 ? 4096 : 2048;
     h.grid = grid_for(n, kHashThreads * 4, (unsigned)props().cu_count * (unsigned)std::max(1, tp.param));
-    h.merge = groups <= kMergeMaxGroups && h.grid >= merge_min_blocks(groups) && h.grid <= kMergeMaxBlocks &&
+    h.merge = c.merge && groups <= kMergeMaxGroups && h.grid >= merge_min_blocks(groups) && h.grid <= kMergeMaxBlocks &&
               n < 0xFFFFFFFFull;
     // Low cardinality: the LDS table holds every group.  High cardinality: it
     // caches the keys seen first and the rest go straight to global.  A table past
@@ -1684,8 +1687,13 @@ int qo_groupby_agg_filtered(const int32_t *key, const int32_t *val, const int32_
     QO_REQUIRE(group_capacity < (size_t(1) << 31), "group capacity too large");
     hipStream_t st = stream_of(s);
     int status = QO_OK;
-    const GroupbyCall c = groupby_call(group_capacity, n, filt != nullptr);
+    GroupbyCall c = groupby_call(group_capacity, n, filt != nullptr);
     void *ws = workspace(st, groupby_ws_bytes(c), &status);
+    if (!ws) {
+        (void)hipGetLastError();
+        c.merge = false;
+        ws = workspace(st, groupby_ws_bytes(c), &status);
+    }
     if (!ws) return status;
     return launch_groupby(c, key, val, okey, ocount, osum, omin, omax, d_numGroups, ws, st, filt, lo, hi);
 }

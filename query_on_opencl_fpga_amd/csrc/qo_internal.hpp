@@ -166,6 +166,7 @@ struct GroupbyCall {
     size_t capacity, n;
     bool filtered;
     TuneParams part, direct;
+    bool merge = true;  // false: without the tables that a merge launch needs (up to 32 MB), for little memory
 };
 GroupbyCall groupby_call(size_t group_capacity, size_t n, bool filtered = false);
 size_t groupby_ws_bytes(const GroupbyCall &c);

@@ -245,7 +245,9 @@ static size_t request_bytes(qo_server *sv, const qo_request &r) {
     if (r.kind == QO_Q_FILTER) return 4096;
     if (r.kind == QO_Q_GROUPBY) {
         size_t G = A.d.group_capacity ? A.d.group_capacity : 1;
-        return G * 28 + groupby_ws_bytes(groupby_call(G, A.d.n, groupby_filter(A.d, r) != nullptr)) + 8192;
+        GroupbyCall c = groupby_call(G, A.d.n, groupby_filter(A.d, r) != nullptr);
+        c.merge = false;  // the least it can run in; launch_batch adds the rest where the budget has room
+        return G * 28 + groupby_ws_bytes(c) + 8192;
     }
     const Table &B = sv->tables[r.table_b];
     qo_join_query q{};
@@ -308,13 +310,22 @@ static int launch_batch(qo_server *sv, Batch &b, hipStream_t st) {
     cv.take<FQuery>(fi.size() + 1);
     cv.take<uint32_t>(64);
     std::vector<GroupbyCall> gcall;
+    size_t left = sv->cfg.memory_budget_bytes - std::min<size_t>(b.est, sv->cfg.memory_budget_bytes);
     for (int i : gi) {
         size_t G = sv->tables[live[i]->r.table_a].d.group_capacity;
         cv.take<int32_t>(G); cv.take<int64_t>(G); cv.take<int64_t>(G); cv.take<int32_t>(G); cv.take<int32_t>(G);
         cv.take<uint64_t>(1);
         const qo_table_desc &A = sv->tables[live[i]->r.table_a].d;
         gcall.push_back(groupby_call(G, A.n, groupby_filter(A, live[i]->r) != nullptr));
-        cv.take<char>(groupby_ws_bytes(gcall.back()));
+        GroupbyCall &c = gcall.back();
+        const size_t most = groupby_ws_bytes(c);
+        c.merge = false;
+        const size_t least = groupby_ws_bytes(c), more = most > least ? most - least : 0;
+        if (more <= left) {
+            c.merge = true;
+            left -= more;
+        }
+        cv.take<char>(groupby_ws_bytes(c));
     }
     for (auto &q : b.jq) {
         cv.take<int32_t>(q.out_capacity); cv.take<int32_t>(q.out_capacity); cv.take<int32_t>(q.out_capacity);
