@@ -228,7 +228,6 @@ static void plan_carve(JoinBatchPlan &p, Carver &cv) {
     p.sort_ws = cv.take<char>(radix_rows_seg_bytes(p.mt, p.nq, (uint32_t)p.hchunks.size()));
     p.part_ws = p.part_ws_bytes ? cv.take<char>(p.part_ws_bytes) : nullptr;
     p.counts = cv.take<unsigned long long>(p.nq);
-    p.long_list = p.sj.all_on ? cv.take<SegPos>(p.total_match / 64 + 1) : nullptr;
     bj_plan_carve(p.sj, cv);
 }
 
@@ -319,26 +318,30 @@ int join_plan_launch(const JoinBatchPlan &p, hipStream_t st) {
         QO_REQUIRE(hp, "query %d: the partitioned probe did not take its hash-mixed table", i);
     }
     if (p.mt) {
-        // Radix passes over the key bits only, then one pass that orders every
-        // run of equal key by s_payload and writes the query's output columns.
-        // Runs of more than 64 rows: with the sorted join able to take every
-        // query (so that each has at most a million rows and few come here), a
-        // work-group per run.  Otherwise the full-width sort, whose 42 launches
-        // are gated on a flag, rewrites the outputs.
-        uint32_t *long_words = p.small + 4;
         bool in_alt = false;
-        QO_TRY(launch_radix_rows_segments(p.mkeys, p.mvals, p.kalt, p.valt, p.d_segs, p.nq, p.mt, p.d_chunks,
-                                           (uint32_t)p.hchunks.size(), p.d_chunk0, 32, 64, p.sort_ws, st, &in_alt,
-                                           nullptr, run_if));
-        uint64_t *ks = in_alt ? p.kalt : p.mkeys, *ka = in_alt ? p.mkeys : p.kalt;
-        uint32_t *vs = in_alt ? p.valt : p.mvals, *va = in_alt ? p.mvals : p.valt;
-        QO_TRY(launch_fix_runs_segments(ks, vs, ka, va, p.d_segs, p.nq, p.mt, p.d_outs, long_words, p.long_list, st,
-                                        run_if));
-        if (!p.long_list) {
-            bool alt2 = false;
-            QO_TRY(launch_radix_rows_segments(ks, vs, ka, va, p.d_segs, p.nq, p.mt, p.d_chunks,
-                                               (uint32_t)p.hchunks.size(), p.d_chunk0, 0, 64, p.sort_ws, st, &alt2,
-                                               p.d_outs, long_words));
+        auto sort = [&](uint64_t *k, uint32_t *v, uint64_t *ka, uint32_t *va, int lo_bit, const RowOut *outs,
+                        const uint32_t *only_if) {
+            return launch_radix_rows_segments(k, v, ka, va, p.d_segs, p.nq, p.mt, p.d_chunks, (uint32_t)p.hchunks.size(),
+                                              p.d_chunk0, lo_bit, 64, p.sort_ws, st, &in_alt, outs, only_if);
+        };
+        if (p.sj.all_on) {
+            // The sorted join usually leaves nothing: the fewest launches that sort
+            // whatever it did leave are the eight full-width passes.  (Key bits first
+            // and a work-group per run of more than 64 rows were 20 launches less, but
+            // one run of 900,000 rows took 5.6 ms, and 140,000 runs as long.)
+            QO_TRY(sort(p.mkeys, p.mvals, p.kalt, p.valt, 0, p.d_outs, run_if));
+        } else {
+            // Radix passes over the key bits only, then one pass that orders every
+            // run of equal key by s_payload and writes the query's output columns.
+            // Should some key have more than 64 rows, the full-width sort (its
+            // kernels gated on that flag, so they return at once otherwise)
+            // rewrites the outputs.
+            uint32_t *long_flag = p.small + 4;
+            QO_TRY(sort(p.mkeys, p.mvals, p.kalt, p.valt, 32, nullptr, nullptr));
+            uint64_t *ks = in_alt ? p.kalt : p.mkeys, *ka = in_alt ? p.mkeys : p.kalt;
+            uint32_t *vs = in_alt ? p.valt : p.mvals, *va = in_alt ? p.mvals : p.valt;
+            QO_TRY(launch_fix_runs_segments(ks, vs, p.d_segs, p.nq, p.mt, p.d_outs, long_flag, st));
+            QO_TRY(sort(ks, vs, ka, va, 0, p.d_outs, long_flag));
         }
     }
     return bj_counts_launch(p.sj, p.gcounts, p.nq, p.counts, st);

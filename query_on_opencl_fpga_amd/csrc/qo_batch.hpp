@@ -114,7 +114,6 @@ struct JoinBatchPlan {
     uint32_t *d_chunk0 = nullptr;
     RowOut *d_outs = nullptr;
     void *sort_ws = nullptr;
-    SegPos *long_list = nullptr;  // long runs of the generic sort (all queries small)
     void *part_ws = nullptr;
     unsigned long long *gcounts = nullptr;  // match counters of the generic stages (in `small`)
     unsigned long long *counts = nullptr;   // match count per query

@@ -51,20 +51,12 @@ int launch_radix_rows_segments(uint64_t *keys, uint32_t *vals, uint64_t *kalt, u
                                uint32_t nchunks, const uint32_t *d_chunk0, int lo_bit, int hi_bit, void *ws,
                                hipStream_t st, bool *in_alt, const RowOut *d_outs = nullptr,
                                const uint32_t *run_if = nullptr);
-// Start of a long run of a segment (position in the segment).
-struct SegPos {
-    uint32_t seg, start;
-};
 // After a segmented sort of join rows on their key bits only [32, 64): sorts
 // every run of equal key by s_payload and writes each segment's rows to its
-// RowOut (segment tiles of kSortTile rows).  A run longer than 64 rows is sorted
-// by one work-group between (keys, vals) and (kalt, valt) when long_list is
-// given (room for total rows / 64 entries; long_words[1] counts them); without
-// it such a run sets long_words[0] and is not written.  long_words: two words,
-// zeroed beforehand.
-int launch_fix_runs_segments(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uint32_t *valt, const RadixSeg *d_segs,
-                             int nseg, uint32_t total_tiles, const RowOut *d_outs, uint32_t *long_words,
-                             SegPos *long_list, hipStream_t st, const uint32_t *run_if = nullptr);
+// RowOut (segment tiles of kSortTile rows); a run longer than 64 rows sets
+// *long_flag and is not written.
+int launch_fix_runs_segments(const uint64_t *keys, const uint32_t *vals, const RadixSeg *d_segs, int nseg,
+                             uint32_t total_tiles, const RowOut *d_outs, uint32_t *long_flag, hipStream_t st);
 // Join rows sort ascending by (key, s_payload) as signed int32: flip the sign
 // bits so unsigned 64-bit order is the signed lexicographic order.
 __host__ __device__ __forceinline__ uint64_t join_sort_key(int32_t key, int32_t spay) {

@@ -1002,8 +1002,6 @@ struct LongRuns {
     uint32_t *n = nullptr;     // starts of the long runs (counted past cap too)
     uint32_t *list = nullptr;  // null: a long run sets the flag
     uint32_t cap = 0;
-    SegPos *seg_list = nullptr;  // in place of `list` for a batch: (segment, start), never full
-    uint32_t seg = 0;
 };
 constexpr uint32_t kFixLongMax = kFixTile / (kFixRun + 1) + 1;  // long runs that start in a tile
 
@@ -1095,7 +1093,7 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
         out.spay[dst] = join_sort_key_spay(x);
         out.rpay[dst] = (int32_t)v[t0 + i];
     }
-    if (!lr.list && !lr.seg_list) {
+    if (!lr.list) {
         if (long_run) atomicOr(lr.flag, 1u);
         return;
     }
@@ -1106,9 +1104,8 @@ QO_DEV void fix_runs_tile(const uint64_t *__restrict__ k, const uint32_t *__rest
     if (threadIdx.x == 0) s_at = atomicAdd(lr.n, s_nlong);
     __syncthreads();
     if (threadIdx.x < s_nlong) {
-        const uint32_t at = s_at + threadIdx.x, s = (uint32_t)t0 + s_long[threadIdx.x];
-        if (lr.seg_list) lr.seg_list[at] = SegPos{lr.seg, s};
-        else if (at < lr.cap) lr.list[at] = s;
+        const uint32_t at = s_at + threadIdx.x;
+        if (at < lr.cap) lr.list[at] = (uint32_t)t0 + s_long[threadIdx.x];
     }
 }
 
@@ -1148,7 +1145,6 @@ QO_DEV uint64_t run_end(const uint64_t *k, uint64_t s, uint64_t hi, uint32_t *s_
 
 struct LongLds {
     BlockSort<kLongItems, false> S;
-    uint32_t hist[4][256];
     uint32_t min;
 };
 
@@ -1167,94 +1163,6 @@ QO_DEV void fix_run_lds(LongLds &L, const uint64_t *k, const uint32_t *v, uint64
         out.rpay[s + i] = (int32_t)(uint32_t)x;
     }
     __syncthreads();  // S is reused
-}
-
-// A longer run, by four digit passes of the work-group between its places in
-// (k, v) and (kalt, valt).  Ends with a barrier.
-QO_DEV void fix_run_passes(LongLds &L, uint64_t *k, uint32_t *v, uint64_t *kalt, uint32_t *valt, uint64_t s,
-                           uint64_t len, const RowOut &out) {
-    const unsigned w = wave_id(), lane = lane_id();
-    const int32_t key = join_sort_key_key(k[s]);
-    // Digit counts of the four passes, then per pass the tiles in order.
-    for (uint32_t i = threadIdx.x; i < 1024; i += kBlockSortThreads) (&L.hist[0][0])[i] = 0;
-    __syncthreads();
-    for (uint64_t i = threadIdx.x; i < len; i += kBlockSortThreads) {
-        const uint32_t x = (uint32_t)k[s + i];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) atomicAdd(&L.hist[p][(x >> (8 * p)) & 255u], 1u);
-    }
-    uint64_t *ks = k + s, *kd = kalt + s;
-    uint32_t *vs = v + s, *vd = valt + s;
-    for (int p = 0; p < 4; ++p) {
-        __syncthreads();
-        const uint32_t c = threadIdx.x < 256 ? L.hist[p][threadIdx.x] : 0u;
-        const uint32_t start = block_excl_scan<kBlockSortWaves>(c, L.S.w);
-        if (threadIdx.x < 256) L.S.dpre[threadIdx.x] = start;
-        if (threadIdx.x == 0) L.min = 0;
-        __syncthreads();
-        if (c == (uint32_t)len) L.min = 1u;
-        __syncthreads();
-        if (L.min) continue;  // one digit: nothing moves
-        for (uint64_t t0 = 0; t0 < len; t0 += kLongLds) {
-            for (int i = 0; i < 256 / kWave; ++i) L.S.cnt[w][i * kWave + lane] = 0;
-            __syncthreads();
-            const uint32_t rem = (uint32_t)(len - t0 < kLongLds ? len - t0 : kLongLds);
-            uint64_t x[kLongItems];
-            uint32_t y[kLongItems], rank[kLongItems];
-#pragma unroll
-            for (int j = 0; j < kLongItems; ++j) {
-                const uint32_t i = (w * kLongItems + j) * kWave + lane;
-                x[j] = i < rem ? ks[t0 + i] : 0;
-                y[j] = i < rem ? vs[t0 + i] : 0;
-            }
-#pragma unroll
-            for (int j = 0; j < kLongItems; ++j) {
-                const bool valid = (w * kLongItems + j) * kWave + lane < rem;
-                const uint32_t d = (uint32_t)(x[j] >> (8 * p)) & 255u;
-                const uint64_t mk = match_digit(d, valid);
-                const uint32_t pre = L.S.cnt[w][d];
-                const uint32_t q = popc(mk & lanemask_lt());
-                wave_lockstep();  // every lane has read its digit's count before the leaders advance it
-                if (valid && q == 0) L.S.cnt[w][d] = pre + popc(mk);
-                wave_lockstep();
-                rank[j] = pre + q;
-            }
-            __syncthreads();
-            if (threadIdx.x < 256) {
-                uint32_t run = L.S.dpre[threadIdx.x];
-#pragma unroll
-                for (int i = 0; i < kBlockSortWaves; ++i) {
-                    const uint32_t u = L.S.cnt[i][threadIdx.x];
-                    L.S.cnt[i][threadIdx.x] = run;
-                    run += u;
-                }
-                L.S.dpre[threadIdx.x] = run;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < kLongItems; ++j) {
-                if ((w * kLongItems + j) * kWave + lane >= rem) continue;
-                const uint32_t d = (uint32_t)(x[j] >> (8 * p)) & 255u;
-                const uint32_t at = L.S.cnt[w][d] + rank[j];
-                kd[at] = x[j];
-                vd[at] = y[j];
-            }
-            __syncthreads();  // the counts are reused by the next tile
-        }
-        __syncthreads();  // the next pass reads what other waves of the work-group wrote
-        uint64_t *const kt = ks;
-        ks = kd;
-        kd = kt;
-        uint32_t *const vt = vs;
-        vs = vd;
-        vd = vt;
-    }
-    for (uint64_t i = threadIdx.x; i < len; i += kBlockSortThreads) {
-        out.key[s + i] = key;
-        out.spay[s + i] = join_sort_key_spay(ks[i]);
-        out.rpay[s + i] = (int32_t)vs[i];
-    }
-    __syncthreads();
 }
 
 __global__ __launch_bounds__(kBlockSortThreads) void k_fix_long(const uint64_t *k, const uint32_t *v, size_t m, RowOut out,
@@ -1277,49 +1185,21 @@ __global__ __launch_bounds__(kBlockSortThreads) void k_fix_long(const uint64_t *
 // tile; n = *d_n clamped to cap rows per segment).
 __global__ __launch_bounds__(kFixThreads) void k_fix_runs_seg(const uint64_t *__restrict__ k,
                                                               const uint32_t *__restrict__ v, const RadixSeg *segs,
-                                                              int nseg, const RowOut *outs, LongRuns lr,
-                                                              const uint32_t *run_if) {
-    if (run_if && *run_if == 0) return;  // gated off: runs only when *run_if != 0
+                                                              int nseg, const RowOut *outs, LongRuns lr) {
     const int si = seg_index_of(segs, nseg, blockIdx.x);
     const RadixSeg sg = segs[si];
     uint64_t n = sg.d_n ? *sg.d_n : sg.cap;
     if (n > sg.cap) n = sg.cap;
     const size_t t0 = (size_t)(blockIdx.x - sg.tile0) * kFixTile;
     if (t0 >= n) return;  // whole block
-    lr.seg = (uint32_t)si;
     fix_runs_tile(k + sg.base, v + sg.base, n, t0, outs[si], lr);
 }
 
-// Long runs of the segments (any length: a segment's rows bound it).
-__global__ __launch_bounds__(kBlockSortThreads) void k_fix_long_seg(uint64_t *k, uint32_t *v, uint64_t *kalt,
-                                                                    uint32_t *valt, const RadixSeg *segs,
-                                                                    const RowOut *outs, const uint32_t *n_runs,
-                                                                    const SegPos *list) {
-    __shared__ LongLds L;
-    const uint32_t n = *n_runs;
-    for (uint32_t r = blockIdx.x; r < n; r += gridDim.x) {
-        const SegPos p = list[r];
-        const RadixSeg sg = segs[p.seg];
-        const size_t m = seg_count(sg);
-        const uint64_t len = run_end(k + sg.base, p.start, m, &L.min) - p.start;
-        if (len <= kLongLds) fix_run_lds(L, k + sg.base, v + sg.base, p.start, (uint32_t)len, outs[p.seg]);
-        else fix_run_passes(L, k + sg.base, v + sg.base, kalt + sg.base, valt + sg.base, p.start, len, outs[p.seg]);
-    }
-}
-
-int launch_fix_runs_segments(uint64_t *keys, uint32_t *vals, uint64_t *kalt, uint32_t *valt, const RadixSeg *d_segs,
-                             int nseg, uint32_t total_tiles, const RowOut *d_outs, uint32_t *long_words,
-                             SegPos *long_list, hipStream_t st, const uint32_t *run_if) {
+int launch_fix_runs_segments(const uint64_t *keys, const uint32_t *vals, const RadixSeg *d_segs, int nseg,
+                             uint32_t total_tiles, const RowOut *d_outs, uint32_t *long_flag, hipStream_t st) {
     static_assert(kFixTile == (uint32_t)kSortTile, "run pass tiles are sort tiles");
     if (total_tiles == 0) return QO_OK;
-    LongRuns lr{long_words};
-    lr.n = long_words + 1;
-    lr.seg_list = long_list;
-    k_fix_runs_seg<<<total_tiles, kFixThreads, 0, st>>>(keys, vals, d_segs, nseg, d_outs, lr, run_if);
-    QO_LAUNCHED();
-    if (!long_list) return QO_OK;
-    k_fix_long_seg<<<(unsigned)props().cu_count * 2, kBlockSortThreads, 0, st>>>(keys, vals, kalt, valt, d_segs, d_outs,
-                                                                               lr.n, long_list);
+    k_fix_runs_seg<<<total_tiles, kFixThreads, 0, st>>>(keys, vals, d_segs, nseg, d_outs, LongRuns{long_flag});
     QO_LAUNCHED();
     return QO_OK;
 }
