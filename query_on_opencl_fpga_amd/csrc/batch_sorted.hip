@@ -117,7 +117,8 @@ __global__ __launch_bounds__(kSplitThreads) void k_bj_scan(const SjBQuery *__res
 }
 
 // Bucket width of a query: the widest whose expected rows and build keys fit a
-// work-group with a quarter to spare, in at most the query's buckets.
+// work-group with a quarter to spare, in at most the query's buckets.  A bucket
+// holds no more than all of them, however far its width goes past the keys' span.
 QO_DEV void bj_plan_query(const SjBQuery &Q, SjBState &s) {
     if (!Q.on || Q.nr == 0 || Q.ns == 0) return;  // no buckets, no rows
     const uint32_t kmin = ~s.rmin_inv, last = s.rmax - kmin;
@@ -126,7 +127,7 @@ QO_DEV void bj_plan_query(const SjBQuery &Q, SjBState &s) {
     const float rows = fminf((float)Q.ns, per * (pass + 4.0f * sqrtf(pass) + 4.0f));
     int sh = 0;
     for (; sh < 31; ++sh) {
-        const float w = (float)(uint64_t(2) << sh) / span;
+        const float w = fminf(1.0f, (float)(uint64_t(2) << sh) / span);
         const bool fits = rows * w <= (float)kBjWantRows && (float)Q.nr * w <= (float)kBjWantKeys;
         if ((last >> sh) == 0 || (!fits && (last >> sh) < Q.nbmax)) break;
     }
@@ -135,7 +136,7 @@ QO_DEV void bj_plan_query(const SjBQuery &Q, SjBState &s) {
     s.sh = (uint32_t)sh;
     s.nb = (last >> sh) + 1u;
     s.pay_bits = 32u - (uint32_t)__clz((int)((s.pmax - ~s.pmin_inv) | 1u));
-    const float w = (float)(uint64_t(1) << sh) / span;
+    const float w = fminf(1.0f, (float)(uint64_t(1) << sh) / span);
     if (s.nb > Q.nbmax || rows * w > 0.9f * kBjRows || (float)Q.nr * w > 0.95f * kBjKeys) {
         s.overflow = 1u;  // the generic stages run it
         s.nb = 0;
@@ -325,10 +326,10 @@ void bj_plan_init(const qo_join_query *queries, int nq, const std::vector<char> 
         q.rvec = (((uintptr_t)u.rkey | (uintptr_t)u.rpay) & 15u) == 0;
         q.bucket0 = p.buckets;
         // The power-of-two width leaves a bucket at least half of what it may hold;
-        // a query that fits one bucket gets one.
+        // a query that fits one bucket gets two, for keys that span more than 2^31.
         const uint64_t want = 2 * std::max<uint64_t>({1, (u.ns + kBjWantRows - 1) / kBjWantRows,
                                                        (u.nr + kBjWantKeys - 1) / kBjWantKeys}) + 1;
-        q.nbmax = want == 3 ? 1u : (uint32_t)std::min<uint64_t>(kBjMaxBuckets, want);
+        q.nbmax = want == 3 ? 2u : (uint32_t)std::min<uint64_t>(kBjMaxBuckets, want);
         q.on = !generic[i] && u.ns <= (uint64_t)kBjMaxBuckets * kBjWantRows && u.nr <= (uint64_t)kBjMaxBuckets * kBjWantKeys;
         if (!q.on) {
             q.nbmax = 0;
