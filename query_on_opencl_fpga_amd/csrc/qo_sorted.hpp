@@ -35,8 +35,8 @@ struct PayloadBins {
     int bits;
     QO_DEV uint32_t operator()(uint32_t pay, int sb) const {
         const uint32_t x = pay ^ 0x80000000u;
-        const uint32_t t = x < pmin ? 0u : (x - pmin) >> (bits > sb ? bits - sb : 0);
-        return min(t, (1u << sb) - 1u);
+        if (sb == 0 || x < pmin) return 0u;  // bits - sb < 32 from here on
+        return min((x - pmin) >> (bits > sb ? bits - sb : 0), (1u << sb) - 1u);
     }
 };
 
