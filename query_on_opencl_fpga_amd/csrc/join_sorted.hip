@@ -344,11 +344,12 @@ struct SjSpread {
 
 // A fine bucket has room for all the rows a work-group takes, so that a hot key of
 // some thousand rows still fits; where fewer than 256 are expected in one (then S
-// is small, and its sample shows such a key), for eight times those and 1024.
-// `most`: rows expected in the fullest bucket of the first split.
-static SjSide sj_side(const SjPlan &p, double most, double mean, uint32_t limit) {
+// is small, and its sample shows such a key), for eight times those and 1024 beside
+// the fullest one's (`top`).  `most`: rows expected in the fullest bucket of the
+// first split.
+static SjSide sj_side(const SjPlan &p, double most, double top, double mean, uint32_t limit) {
     SjSide o;
-    o.capB = std::min<uint64_t>(limit, ((uint64_t)(8.0 * mean) + 1024 + 31) / 32 * 32);
+    o.capB = std::min<uint64_t>(limit, ((uint64_t)(top + 8.0 * mean) + 1024 + 31) / 32 * 32);
     if (p.b2) o.capA = ((uint64_t)(most / kXcdRegions * 1.25 + 8.0 * std::sqrt(most)) + kSplitTile + 31) / 32 * 32;
     return o;
 }
@@ -384,10 +385,10 @@ static bool sj_buckets(SjPlan &p, int nt, const SjSpread &s, size_t nr) {
     p.nb1 = ((p.nb - 1) >> p.b2) + 1;
     p.parts1 = 1;
     while (p.parts1 < p.nb1) p.parts1 *= 2;
-    p.s = sj_side(p, s.most(p.sh + p.b2), s.rows / p.nb, (uint32_t)limit);
+    p.s = sj_side(p, s.most(p.sh + p.b2), s.most(p.sh), s.rows / p.nb, (uint32_t)limit);
     if (!p.dense) {
         const double even = (double)nr * std::min(1.0, std::ldexp(1.0, p.sh + p.b2) / s.span);
-        p.r = sj_side(p, s.even ? even : std::min((double)nr, 4.0 * even), (double)nr / p.nb, 2u * (uint32_t)nt);
+        p.r = sj_side(p, s.even ? even : std::min((double)nr, 4.0 * even), 0.0, (double)nr / p.nb, 2u * (uint32_t)nt);
     }
     return true;
 }

@@ -1,6 +1,7 @@
 // CPU build driver, for the sanitizer build: a sorted join whose buckets hold more
 // than 1024 spread build keys each (work-groups of 1024 threads, one s_payload
-// interval per key), with s_payloads over the whole int32 range.
+// interval per key), with s_payloads over the whole int32 range; or, with an
+// argument, one of many buckets of few rows and a key of 4000.
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
@@ -27,12 +28,13 @@ static int32_t *dev(const std::vector<int32_t> &h) {
     return static_cast<int32_t *>(p);
 }
 
-int main() {
+int main(int argc, char **) {
+    const bool hot = argc > 1;
     CK(qo_init(0));
     // One key holds 3000 rows, so buckets need the larger work-groups; 500 rows are
     // spread over 10,000 keys 3355 apart, so a bucket of some 500 rows holds a
     // thousand keys and more.  The rest of S does not pass the filter.
-    const size_t nr = 10000, ns = 20000;
+    const size_t nr = hot ? 6000 : 10000, ns = 20000, hot_rows = hot ? 4000 : 3000, rows = hot ? ns : 3500;
     std::vector<int32_t> rk(nr), rp(nr), sk(ns), sp(ns), sf(ns);
     for (size_t i = 0; i < nr; ++i) {
         rk[i] = (int32_t)(i * 3355) - 15000000;
@@ -42,11 +44,11 @@ int main() {
     auto rnd = [&] { return x = x * 1664525u + 1013904223u; };
     std::vector<std::tuple<int32_t, int32_t, int32_t>> want;
     for (size_t i = 0; i < ns; ++i) {
-        const size_t at = i * 7919 % ns, r = i < 3000 ? 77 : (rnd() >> 8) % nr;
+        const size_t at = i * 7919 % ns, r = i < hot_rows ? 77 : (rnd() >> 8) % nr;
         sk[at] = rk[r];
         sp[at] = i == 0 ? INT32_MIN : i == 1 ? INT32_MAX : (int32_t)rnd();
-        sf[at] = i < 3500 ? 1 : 2;
-        if (i < 3500) want.emplace_back(rk[r], sp[at], rp[r]);
+        sf[at] = i < rows ? 1 : 2;
+        if (i < rows) want.emplace_back(rk[r], sp[at], rp[r]);
     }
     std::sort(want.begin(), want.end());
     const size_t tb = qo_join_table_bytes(nr);

@@ -2,7 +2,8 @@
 and undefined-behaviour sanitizers:
 
 * join_sorted_wide: buckets of more than 1024 spread build keys (one s_payload
-  interval per key) and s_payloads over the whole int32 range.
+  interval per key) and s_payloads over the whole int32 range; many buckets of
+  few rows with one key of 4000, which the sample shows and a bucket has room for.
 """
 import os
 import subprocess
@@ -30,3 +31,8 @@ def run(exe, *args):
 
 def test_one_payload_interval_per_key(cpu_build):
     assert "k_sj_finish<<<8, 1024" in run(cpu_build / "join_sorted_wide")
+
+
+def test_room_for_a_hot_key_among_few_rows(cpu_build):
+    trace = run(cpu_build / "join_sorted_wide", "hot")
+    assert "k_sj_finish" in trace and "k_join_probe" not in trace
