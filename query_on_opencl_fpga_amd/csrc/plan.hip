@@ -41,16 +41,16 @@ struct PrimCost {
     double fixed_us, gbps;
 };
 static PrimCost g_cost[QO_COST_NUM] = {
-    {13.0, 4300.0},  // QO_COST_FILTER: filter compaction, 8 B read + 8 B per selected row written
-    {15.0, 4000.0},  // QO_COST_SORT_PASS: one radix pass, 24 B per row (histogram read, read, write)
-    {12.0, 3300.0},  // QO_COST_STARTPOS: group start positions, 8 B per row
-    {28.0, 850.0},   // QO_COST_AGG: one per-group aggregate, 8 B per row (1024 groups)
-    {6.0, 5000.0},   // QO_COST_UNPACK: Records -> columns (or a Record copy), 16 B per row
-    {81.0, 3400.0},  // QO_COST_HASH_SMALL: hash group-by, direct (at most kGroupbyDirect groups), 8 B per row
-    {245.0, 1260.0}, // QO_COST_HASH_LARGE: hash group-by, more groups (partitioned), 8 B per row
-    {10.0, 6300.0},  // QO_COST_REDUCE: no-group reduce, 8 B per row
-    {75.0, 3960.0},  // QO_COST_FHASH_SMALL: filtered hash group-by (half selected), direct
-    {222.0, 1300.0}, // QO_COST_FHASH_LARGE: filtered hash group-by (half selected), more groups
+    {11.5, 5000.0},  // QO_COST_FILTER: filter compaction, 8 B read + 8 B per selected row written
+    {5.1, 4550.0},   // QO_COST_SORT_PASS: one radix pass, 24 B per row (histogram read, read, write)
+    {11.8, 3750.0},  // QO_COST_STARTPOS: group start positions, 8 B per row
+    {20.6, 5450.0},  // QO_COST_AGG: one per-group aggregate, 8 B per row (1024 groups)
+    {6.2, 5000.0},   // QO_COST_UNPACK: Records -> columns (or a Record copy), 16 B per row
+    {31.1, 5400.0},  // QO_COST_HASH_SMALL: hash group-by, direct (at most kGroupbyDirect groups), 8 B per row
+    {227.0, 1510.0}, // QO_COST_HASH_LARGE: hash group-by, more groups (partitioned), 8 B per row
+    {10.1, 6230.0},  // QO_COST_REDUCE: no-group reduce, 8 B per row
+    {27.0, 5680.0},  // QO_COST_FHASH_SMALL: filtered hash group-by (half selected), direct
+    {206.0, 1610.0}, // QO_COST_FHASH_LARGE: filtered hash group-by (half selected), more groups
 };
 static std::mutex g_cost_mu;
 

@@ -28,3 +28,15 @@ def test_sort_pass_is_no_faster_than_a_copy(qo):
     finally:
         for i, (f, g) in enumerate(saved):
             P.set_cost(i, f, g)
+
+
+def test_built_in_costs_are_this_device(qo):
+    """The table a plan starts from, next to a calibration at the size it was taken at: within a factor of two."""
+    built_in = P.cost_table()
+    try:
+        measured = P.calibrate(26, 5)
+    finally:
+        for i, (f, g) in enumerate(built_in):
+            P.set_cost(i, f, g)
+    for name, (f0, g0), (f1, g1) in zip(P.COST_NAMES, built_in, measured):
+        assert 0.5 < g0 / g1 < 2 and (0.5 < f0 / f1 < 2 or abs(f0 - f1) < 5), (name, f0, g0, f1, g1)
