@@ -1486,18 +1486,24 @@ __global__ void k_agg_chunks(const int32_t *startPos, uint32_t G, size_t n, uint
 
 QO_DEV int32_t agg_identity(int op) { return op == QO_REDUCE_MIN ? (1 << 30) : 0; }
 
-// kAggLanes lanes per work unit, kWave / kAggLanes units per wave at once, each
-// group of lanes walking a contiguous range of units: a lane reduces every
-// kAggLanes-th row of a unit (all its loads issued before any is used) and keeps
-// its partial while the group stays the same; where the group changes the lanes
+// kAggLanes lanes per work unit, a block's 32 units side by side in a contiguous
+// range of units that it walks: a lane reduces every kAggLanes-th row of a unit
+// (all its loads issued before any is used) and keeps its partial while the group
+// stays the same; where the group changes the lanes
 // combine by shuffles, and the first lane stores the result of a group that is
 // one unit or merges a partial with an atomic.  What the lanes hold at the end is
 // combined over the wave and the block first where it is one group's.  `acc`
 // holds the identity beforehand.  Bound by the row loads: 2^26 Records in 16
 // groups 98 us (5.5 TB/s).  With a table of every unit's group, written by a thread
 // per group, and one atomic per unit, few groups left the chip to a few threads and
-// the atomics to a few addresses: the chain from copy to sums over 2^26 Records
-// 113 ms with one group, 5.4 ms with 109, 2.24 with 20,000; now 0.86, 1.14 and 1.29.
+// the atomics to a few addresses: over 2^26 Records (times of a whole call) 1020 us
+// in 671 groups, now 124, 160 in 13,421, now 127, and 128 in 167,772, now 131.
+// A wave holds offset and start of the 64 groups from that of its first unit on, in
+// registers, and loads the next ones before this step's rows: a step waits for its
+// rows alone.  With each unit's group looked up by its own lanes, in three dependent
+// loads, groups of 200 rows took 146 us, now 133; with a range per group of lanes
+// instead of one per block, small groups' rows lay on lines that L1 had lost before
+// their neighbours were read: 2^26 Records in groups of 10 rows 607 us, now 478.
 __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict__ s, size_t n,
                                                     const int32_t *__restrict__ startPos, uint32_t G,
                                                     const uint32_t *__restrict__ cofs, const uint32_t *__restrict__ chunks,
@@ -1511,49 +1517,101 @@ __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict_
     const uint32_t total = cofs[G - 1] + chunks[G - 1];
     if (total == 0) return;  // the whole grid
     const unsigned lane = lane_id(), sub = lane / kAggLanes, sl = lane % kAggLanes;
-    const size_t subs = (size_t)gridDim.x * kWaves * kUnitsPerWave;
-    const size_t per = (total + subs - 1) / subs;
-    const size_t w0 = (((size_t)blockIdx.x * kWaves + wave_id()) * kUnitsPerWave + sub) * per;
+    constexpr uint32_t kStep = kWaves * kUnitsPerWave;  // units of a block at once
+    const size_t all = (total + kStep - 1) / kStep, s0 = blockIdx.x * all / gridDim.x;
+    const size_t steps = (blockIdx.x + 1) * all / gridDim.x - s0;
+    if (steps == 0) return;  // whole block
+    const size_t u0 = s0 * kStep + wave_id() * kUnitsPerWave;  // the wave's first unit
     auto merge = [&](int32_t a, int32_t b) {
         if (op == QO_REDUCE_MAX) return a > b ? a : b;
         if (op == QO_REDUCE_MIN) return a < b ? a : b;
         return (int32_t)((uint32_t)a + (uint32_t)b);
     };
-    auto emit = [&](uint32_t g, int32_t l) {
-        if (chunks[g] == 1) acc[g] = l;  // the group's only unit: its result is final
+    auto emit = [&](uint32_t g, bool whole, int32_t l) {
+        if (whole) acc[g] = l;  // the group's only unit: its result is final
         else if (op == QO_REDUCE_MAX) atomicMax(&acc[g], l);
         else if (op == QO_REDUCE_MIN) atomicMin(&acc[g], l);
         else atomicAdd(reinterpret_cast<uint32_t *>(&acc[g]), (uint32_t)l);
     };
-    // The group of the first unit is the last one with cofs <= w0 (it has units:
-    // cofs of a group without is the next one's), found kAggLanes probes at a time.
-    uint32_t next = 0;
-    {
-        const uint32_t w = w0 < total ? (uint32_t)w0 : total - 1;
-        uint32_t len = G;
-        while (ballot(len > 1)) {
-            const uint32_t step = (len + kAggLanes - 1) / kAggLanes, at = sl * step;
-            const uint64_t le = ballot(at < len && (sl == 0 || cofs[next + at] <= w));
-            const uint32_t k = __popcll((le >> (sub * kAggLanes)) & ((1u << kAggLanes) - 1)) - 1;
-            next += k * step;
+    // A group before or at the last with cofs <= w (which has units: cofs of a group
+    // without is the next one's) by less than half a wave, found kWave probes at a
+    // time among `len` from `from` on; cofs[from] <= w.
+    auto group_near = [&](uint32_t from, uint32_t len, uint32_t w) {
+        while (len > kWave / 2) {
+            const uint32_t step = 1 + (len - 1) / kWave, at = lane * step;
+            const uint32_t k = __popcll(ballot(at < len && (lane == 0 || cofs[from + at] <= w))) - 1;
+            from += k * step;
             len = min(step, len - k * step);
         }
+        return from;
+    };
+    // The wave's lanes hold first unit and first row of the groups from `base` on; the
+    // units of a step are kStep after the last step's, so in one of the next few groups.
+    uint32_t base = 0, first = 0;
+    int32_t row = 0;
+    auto load_groups = [&] {
+        const size_t at = (size_t)base + lane;
+        first = at < G ? cofs[at] : at == G ? total : kNone;
+        row = at < G ? startPos[at] : 0;
+    };
+    if (u0 < total) {
+        const uint32_t w = (uint32_t)u0;
+        if (total == G && cofs[w] == w && chunks[w] == 1) {
+            base = w;  // as many units as groups, and unit w is group w's only one: most likely
+        } else {
+            // Sought from where it is if all groups have as many units, at twice the
+            // distance with each lane.
+            const int64_t d = (int64_t)lane - kWave / 2, c = (int64_t)((uint64_t)w * G / total);
+            const int64_t at = c + (d < 0 ? -((int64_t)1 << (-d - 1)) : d > 0 ? (int64_t)1 << (d - 1) : 0);
+            const int k = __popcll(ballot(at <= 0 || (at < (int64_t)G && cofs[at] <= w)));
+            const int64_t lo = k == 0 ? 0 : max(__shfl(at, k - 1, kWave), (int64_t)0);
+            const int64_t hi = k == kWave ? (int64_t)G : min(__shfl(at, k, kWave), (int64_t)G);
+            base = group_near((uint32_t)lo, (uint32_t)(hi - lo), w);
+        }
     }
+    load_groups();
     uint32_t cur = kNone;
+    bool whole = false;  // cur is one unit
     int32_t local = agg_identity(op);
-    size_t gw = 0, gend = 0;    // units of the group in hand
-    int64_t gs = 0, ge = 0;     // its rows
-    uint32_t g = kNone;
-    for (size_t i = 0; i < per; ++i) {
-        const size_t w = w0 + i;
-        int64_t a = 0, b = 0;
-        if (w < total) {
-            while (w >= gend && next < G) {
-                g = next++;
-                gw = cofs[g];
-                gend = gw + chunks[g];
-                group_range(startPos, g, G, n, gs, ge);
+    for (size_t i = 0; i < steps; ++i) {
+        const size_t w = u0 + i * kStep + sub;
+        uint32_t g = kNone, gw = 0, gend = 0;  // the unit's group, its units
+        int64_t gs = 0, ge = 0;                // and rows
+        for (;;) {
+            uint32_t k = 0;  // groups of those held that begin at unit w or before
+#pragma unroll
+            for (int u = 0; u < (int)kUnitsPerWave; ++u) {
+                const uint32_t c = __popcll(ballot(first <= __shfl((uint32_t)w, u * kAggLanes, kWave)));
+                if ((int)sub == u) k = c;
             }
+            const bool find = w < total && g == kNone, hit = find && k > 0 && k < kWave;
+            const int at = hit ? (int)k - 1 : 0;
+            const uint32_t cw = __shfl(first, at, kWave), ce = __shfl(first, at + 1, kWave);
+            const int32_t rs = __shfl(row, at, kWave), re = __shfl(row, at + 1, kWave);
+            if (hit) {
+                g = base + at;
+                gw = cw;
+                gend = ce;
+                gs = max(rs, 0);
+                ge = g == G - 1 ? (int64_t)n : min((int64_t)re, (int64_t)n);
+            }
+            const uint64_t miss = ballot(find && !hit);
+            if (miss == 0) break;
+            // Past many groups without units: those of the first unit not found.
+            const uint32_t u = __shfl((uint32_t)w, __ffsll((unsigned long long)miss) - 1, kWave);
+            const uint32_t to = group_near(base, G - base, u);
+            if (to == base) break;  // never with offsets that ascend
+            base = to;
+            load_groups();
+        }
+        // For the next step, before this one's rows.
+        const uint32_t g0 = __shfl(g, 0, kWave);
+        if (g0 != kNone) {
+            base = g0;
+            load_groups();
+        }
+        int64_t a = 0, b = 0;
+        if (g != kNone) {
             a = gs + (int64_t)(w - gw) * kAggChunk;
             b = a + kAggChunk < ge ? a + kAggChunk : ge;
         }
@@ -1563,18 +1621,21 @@ __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict_
             const int64_t r = a + sl + (int64_t)k * kAggLanes;
             v[k] = r < b ? (int32_t)s[r].x : agg_identity(op);
         }
-        const bool change = cur != kNone && g != cur;
+        const bool change = cur != kNone && g != kNone && g != cur;
         if (ballot(change)) {
             int32_t l = local;
             // Xor offsets below kAggLanes stay inside the unit's lanes.
 #pragma unroll
             for (int o = kAggLanes / 2; o > 0; o >>= 1) l = merge(l, __shfl_xor(l, o, kWave));
             if (change) {
-                if (sl == 0) emit(cur, l);
+                if (sl == 0) emit(cur, whole, l);
                 local = agg_identity(op);
             }
         }
-        cur = g;
+        if (g != kNone) {
+            cur = g;
+            whole = gend - gw == 1;
+        }
 #pragma unroll
         for (int k = 0; k < kPerLane; ++k) local = merge(local, v[k]);
     }
@@ -1586,7 +1647,7 @@ __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict_
 #pragma unroll
         for (int o = kAggLanes; o < kWave; o <<= 1) local = merge(local, __shfl_xor(local, o, kWave));
     } else if (sl == 0 && cur != kNone) {
-        emit(cur, local);
+        emit(cur, whole, local);
     }
     if (lane == 0) {
         s_cur[wave_id()] = one ? c0 : kNone;
@@ -1597,7 +1658,7 @@ __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict_
         for (int k = 0; k < kWaves; ++k) {
             if (s_cur[k] == kNone) continue;
             if (k + 1 < kWaves && s_cur[k + 1] == s_cur[k]) s_val[k + 1] = merge(s_val[k], s_val[k + 1]);
-            else emit(s_cur[k], s_val[k]);
+            else emit(s_cur[k], chunks[s_cur[k]] == 1, s_val[k]);
         }
     }
 }
