@@ -1392,8 +1392,8 @@ int launch_groupby(const GroupbyCall &c, const int32_t *key, const int32_t *val,
 // ---------------------------------------------------------------------------
 // Group start positions over Records sorted by .y: record i starts a group
 // when i == 0 or its .y differs from record i - 1's.  Tiles of J * NT * 2
-// records (16-byte loads of two records; the record before each pair is read
-// with its own load, an L1 hit), 32-bit in-tile offsets, one ticketed
+// records (16-byte loads of two records; the key before each pair comes from the
+// lane before, for a wave's first lane from a load), 32-bit in-tile offsets, one ticketed
 // decoupled look-back per tile; the starts are written in order.
 template <int J, int NT, bool VEC>
 __global__ __launch_bounds__(NT) void k_group_startpos(const qo_record *__restrict__ s, size_t n, int32_t *startPos,
@@ -1598,7 +1598,7 @@ __global__ __launch_bounds__(256) void k_agg_groups(const qo_record *__restrict_
             const uint64_t miss = ballot(find && !hit);
             if (miss == 0) break;
             // Past many groups without units: those of the first unit not found.
-            const uint32_t u = __shfl((uint32_t)w, __ffsll((unsigned long long)miss) - 1, kWave);
+            const uint32_t u = __shfl((uint32_t)w, __builtin_ctzll(miss), kWave);
             const uint32_t to = group_near(base, G - base, u);
             if (to == base) break;  // never with offsets that ascend
             base = to;
