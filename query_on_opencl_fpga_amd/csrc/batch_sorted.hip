@@ -143,32 +143,42 @@ QO_DEV void bj_plan_query(const SjBQuery &Q, SjBState &s) {
     }
 }
 
-// words[0] := buckets in use.
-__global__ __launch_bounds__(256) void k_bj_plan(const SjBQuery *__restrict__ qs, SjBState *state, int nq,
+// words[0] := buckets in use; the buckets of kBjChunk queries are listed together.
+constexpr int kBjChunk = 256;
+__global__ __launch_bounds__(kBjChunk) void k_bj_plan(const SjBQuery *__restrict__ qs, SjBState *state, int nq,
                                                  uint32_t *words) {
     __shared__ uint32_t s_w[4];
     __shared__ uint32_t s_base;
-    const int q = blockIdx.x * 256 + threadIdx.x;
+    const int q = blockIdx.x * kBjChunk + threadIdx.x;
     uint32_t nb = 0;
     if (q < nq) {
         bj_plan_query(qs[q], state[q]);
         nb = state[q].nb;
     }
     const uint32_t ex = block_excl_scan256(nb, s_w);
-    if (threadIdx.x == 255) s_base = atomicAdd(&words[0], ex + nb);
+    if (threadIdx.x == kBjChunk - 1) s_base = atomicAdd(&words[0], ex + nb);
     __syncthreads();
-    if (q < nq) state[q].from = s_base + ex;
+    if (q < nq) state[q].from = s_base;
 }
 
-// Lists the buckets of query blockIdx.x with their sizes.
+// Lists the buckets of query blockIdx.x with their sizes: first the first bucket of
+// each of the chunk's queries, then the second ones, and so on, so that few buckets
+// of a query are being finished at the same time.
 static_assert(kBjMaxBuckets == 512, "one bucket per thread");
 __global__ __launch_bounds__(512) void k_bj_list(const SjBQuery *__restrict__ qs, const SjBState *state,
-                                                 const uint32_t *sctr, const uint32_t *rctr, SjBucket *list) {
-    const uint32_t q = blockIdx.x, f = threadIdx.x;
+                                                 int nq, const uint32_t *sctr, const uint32_t *rctr, SjBucket *list) {
+    __shared__ uint32_t s_nb[kBjChunk];
+    const uint32_t q = blockIdx.x, f = threadIdx.x, q0 = q - q % kBjChunk;
+    if (f < (uint32_t)kBjChunk) s_nb[f] = q0 + f < (uint32_t)nq ? state[q0 + f].nb : 0u;
+    __syncthreads();
     const SjBState &st = state[q];
     if (f >= st.nb) return;
+    uint32_t at = st.from;
+    const uint32_t m = min((uint32_t)kBjChunk, (uint32_t)nq - q0);
+#pragma unroll 8
+    for (uint32_t i = 0; i < m; ++i) at += min(s_nb[i], f) + (q0 + i < q && s_nb[i] > f ? 1u : 0u);
     const size_t c = (size_t)(qs[q].bucket0 + f) * kCtrStride;
-    list[st.from + f] = SjBucket{q, f, min(sctr[c], kBjRows), min(rctr[c], kBjKeys)};
+    list[at] = SjBucket{q, f, min(sctr[c], kBjRows), min(rctr[c], kBjKeys)};
 }
 
 // Blocks [0, nst): S tiles; from nst on: build tiles.
@@ -207,34 +217,39 @@ __global__ __launch_bounds__(kSplitThreads) void k_bj_split(const SjBQuery *__re
                          FixedLayout{build ? kBjKeys : kBjRows}, build ? rctr : sctr, sh, FlagOverflow{&st.overflow});
 }
 
-// lookback over at most kBjMaxBuckets tiles, with the words of all predecessors
-// in flight together: a query's buckets run at the same time, so hardly one finds
-// an inclusive prefix near it, and a load per 64 predecessors is a chain of up to
-// eight.
-QO_DEV uint64_t bj_lookback(uint64_t *status, uint32_t f, uint32_t aggregate, DevCtl *ctl) {
-    constexpr int kWords = kBjMaxBuckets / kWave;
+// lookback over at most kBjMaxBuckets tiles from `near`, the words of the 64 before
+// f as read some time before.  With many queries an inclusive prefix is among them;
+// with few the words of all predecessors are read together (a query's buckets then
+// run at the same time, and a load per 64 of them is a chain of up to eight).
+constexpr int kBjWords = kBjMaxBuckets / kWave;
+QO_DEV uint64_t bj_word(const uint64_t *status, uint32_t f, int k) {
+    const int idx = (int)f - 1 - k * kWave - (int)lane_id();
+    return idx >= 0 ? ld_agent(&status[idx]) : kFlagInc;
+}
+QO_DEV uint64_t bj_lookback(uint64_t *status, uint32_t f, uint32_t aggregate, DevCtl *ctl, uint64_t near) {
     const unsigned lane = lane_id();
     uint64_t excl = 0;
     if (f > 0) {
         const uint32_t limit = ctl->spin_limit;
         for (uint32_t sleeps = 0;;) {  // wave-uniform: the branches depend on ballots only
-            uint64_t w[kWords];
-#pragma unroll
-            for (int k = 0; k < kWords; ++k) {
-                const int idx = (int)f - 1 - k * kWave - (int)lane;
-                w[k] = idx >= 0 ? ld_agent(&status[idx]) : kFlagInc;
-            }
+            uint64_t w[kBjWords];
             uint64_t sum = 0;
             bool done = false, empty = false;
-#pragma unroll
-            for (int k = 0; k < kWords; ++k) {
-                if (done || empty) continue;
-                const uint64_t inc = ballot(w[k] >> 62 == 2);
+            auto add = [&](uint64_t word) {
+                const uint64_t inc = ballot(word >> 62 == 2);
                 const unsigned first = inc ? (unsigned)__builtin_ctzll(inc) : 64u;
                 const uint64_t relevant = first >= 63 ? ~uint64_t(0) : ((uint64_t(2) << first) - 1);
-                empty = (ballot(w[k] >> 62 == 0) & relevant) != 0;
-                if (lane <= first) sum += w[k] & kValMask;
+                empty = (ballot(word >> 62 == 0) & relevant) != 0;
+                if (lane <= first) sum += word & kValMask;
                 done = inc != 0;
+            };
+            add(near);
+            if (!done && !empty) {
+#pragma unroll
+                for (int k = 1; k < kBjWords; ++k) w[k] = bj_word(status, f, k);
+#pragma unroll
+                for (int k = 1; k < kBjWords; ++k)
+                    if (!done && !empty) add(w[k]);
             }
             if (!empty) {
                 excl = wave_sum(sum);
@@ -245,6 +260,7 @@ QO_DEV uint64_t bj_lookback(uint64_t *status, uint32_t f, uint32_t aggregate, De
                 return 0;
             }
             __builtin_amdgcn_s_sleep(1);
+            near = bj_word(status, f, 0);
         }
     }
     if (lane == 0) st_agent(&status[f], kFlagInc | (excl + aggregate));
@@ -261,8 +277,10 @@ struct BjChained {
         // Successors need not wait for the placement.
         if (threadIdx.x == 0) st_agent(&status[f], (f ? kFlagAgg : kFlagInc) | total);
     }
-    QO_DEV uint64_t position(uint32_t total) const {
-        const uint64_t e = bj_lookback(status, f, total, ctl);
+    using Asked = uint64_t;
+    QO_DEV void ask(Asked &a) const { a = bj_word(status, f, 0); }
+    QO_DEV uint64_t position(uint32_t total, Asked a) const {
+        const uint64_t e = bj_lookback(status, f, total, ctl, a);
         if (f == st->nb - 1 && lane_id() == 0) st->rows = e + total;
         return e;
     }
@@ -270,9 +288,10 @@ struct BjChained {
 };
 
 // One listed bucket, taken by ticket: a query's buckets are listed in order, so
-// every predecessor in the look-back is already running or done.  Of its 513 us
-// for 512 queries 113 are the look-back and 37 the tickets (a ticket counter per
-// query, read after the list, 30 more; a load per 64 predecessors 25 more).  Rows
+// every predecessor in the look-back is already running or done.  465 us for 512
+// queries, 37 of them the tickets (a counter per query, read after the list, 30
+// more).  With the buckets listed query by query, so that a query's were all being
+// finished at once, and the look-back's words read where they are needed 513.  Rows
 // at positions that assume every tuple matches took 363, and left rows behind the
 // result where one did not.
 __global__ __launch_bounds__(kBjThreads, 8) void k_bj_finish(const SjBQuery *__restrict__ qs, SjBState *state,
@@ -387,7 +406,7 @@ int bj_plan_launch(const SjBatchPlan &p, uint32_t *any, hipStream_t st) {
         k_bj_split<<<nst + nrt, kSplitThreads, 0, st>>>(p.d_q, p.state, p.d_stiles, nst, p.d_rtiles, p.sbuckets, p.sctr,
                                                         p.rbuckets, p.rctr);
         QO_LAUNCHED();
-        k_bj_list<<<(unsigned)nq, 512, 0, st>>>(p.d_q, p.state, p.sctr, p.rctr, p.list);
+        k_bj_list<<<(unsigned)nq, 512, 0, st>>>(p.d_q, p.state, nq, p.sctr, p.rctr, p.list);
         QO_LAUNCHED();
         // One block per bucket a query may use (two to four times those in use; 2048
         // blocks that walk the list took a tenth longer).

@@ -26,9 +26,9 @@
 // matches otherwise.  More rows than the outputs hold: none is written.
 //
 // Whole calls, generic path -> this one: 2^28 S rows, half selected, 2^24 dense
-// build keys 5.64 -> 2.40 ms (split 0.96, second split 0.55, finish 0.64, build
+// build keys 5.64 -> 2.44 ms (split 0.96, second split 0.55, finish 0.67, build
 // 0.2); 12,000,008 S rows, half selected, 1,500,001 spread 31-bit keys 684 ->
-// 370 us; 16384 S rows, half selected, 4096 spread keys 204 -> 125 us (88 with the
+// 349 us; 16384 S rows, half selected, 4096 spread keys 204 -> 75 us (the
 // table built by one work-group).
 #include <algorithm>
 #include <cmath>
@@ -227,7 +227,9 @@ __global__ __launch_bounds__(256) void k_sj_offsets(SjBuckets A, uint32_t nsub, 
 struct SjKnown {
     uint32_t at;
     QO_DEV void begin(uint32_t) const {}
-    QO_DEV uint64_t position(uint32_t) const { return at; }
+    struct Asked {};
+    QO_DEV void ask(Asked &) const {}
+    QO_DEV uint64_t position(uint32_t, Asked) const { return at; }
     QO_DEV void repeated() const {}  // the table build saw to that
 };
 struct SjChained {
@@ -240,7 +242,9 @@ struct SjChained {
         // Successors need not wait for the placement.
         if (threadIdx.x == 0) st_agent(&status[f], (f ? kFlagAgg : kFlagInc) | total);
     }
-    QO_DEV uint64_t position(uint32_t total) const {
+    struct Asked {};
+    QO_DEV void ask(Asked &) const {}
+    QO_DEV uint64_t position(uint32_t total, Asked) const {
         const uint64_t e = lookback(status, f, total, ctl, flag, kSjWait);
         if (f == nb - 1 && lane_id() == 0) *d_count = e + total;
         return e;
@@ -301,7 +305,10 @@ struct SjPlan {
 };
 
 // Fewer S tuples than this are probed and sorted by the generic path, whose
-// small sort is one launch.
+// small sort is one launch.  At the line, 16383 S rows that way and 16384 this way,
+// us: 64 build keys spread 157 and 113, dense 141 and 96; 4096 spread 233 and 112,
+// dense 138 and 97.  (What breaks even lies below and was not looked for: those rows
+// fewer keep the path they had.)
 constexpr size_t kSjMinRows = size_t(1) << 14;
 constexpr uint64_t kSjMaxBuckets = 1u << (2 * kSjPartBits);
 

@@ -47,7 +47,7 @@ struct SjBState {             // zero before a launch
     uint32_t pass;            // sampled S tuples that pass the filter
     uint32_t pmin_inv, pmax;  // ~smallest and largest sampled s_payload, biased
     uint32_t kmin, last, sh, nb, pay_bits;
-    uint32_t from;            // first of its buckets in the list of those in use
+    uint32_t from;            // where its chunk of queries begins in the list of buckets in use
     uint32_t overflow, repeated;
     uint64_t rows;            // matches
 };
@@ -105,7 +105,7 @@ struct JoinBatchPlan {
     size_t part_ws_bytes = 0;
     // Bound by join_plan_bind:
     uint64_t *slots_all = nullptr;
-    uint32_t *small = nullptr;  // tickets, then per-query match counts
+    uint32_t *small = nullptr;  // tickets and flags (words 0-4), from word 64 per-query match counts
     BQuery *d_q = nullptr;
     RadixSeg *d_segs = nullptr;
     uint64_t *mkeys = nullptr, *kalt = nullptr;

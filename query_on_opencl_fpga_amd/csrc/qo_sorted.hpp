@@ -168,7 +168,8 @@ QO_DEV void sj_clear(SjLds<DENSE, NT> &s) {
 // Joins and writes one bucket: n tuples at src, keys in [kbase, kbase + 2^sh).
 // DENSE: `slots` is the bucket's slice of the key-range table (2^sh <= 2 NT
 // slots); else nr <= 2 NT build tuples at rsrc.  `start` says where the rows go:
-// begin(total) (every thread), position(total) (first wave only; the first row's
+// begin(total) (every thread), ask() (first wave only; what position() may read
+// ahead), position(total) (first wave only; the first row's
 // output position) and, for build tuples, repeated() when two have one key.
 // Called by all NT threads after sj_clear and a barrier.
 template <bool DENSE, int NT, class Start>
@@ -279,8 +280,10 @@ QO_DEV void sj_bucket(SjLds<DENSE, NT> &s, const uint64_t *__restrict__ src, uin
         s.slot[p] = (uint16_t)l;
     }
     __syncthreads();
+    typename Start::Asked asked;
     if (s.long_run) {  // block-uniform
         sj_sort_rows<DENSE, NT>(s, total, sb);
+        if (threadIdx.x < kWave) start.ask(asked);
     } else {
         // Position i of the rows in bin order: its rank in its bin's run by
         // s_payload, four rows of the run per step (reads past the run's end stay
@@ -305,6 +308,7 @@ QO_DEV void sj_bucket(SjLds<DENSE, NT> &s, const uint64_t *__restrict__ src, uin
             }
             dst[j] = (b0 + before) | (l << 16);
         }
+        if (threadIdx.x < kWave) start.ask(asked);  // on their way over the barrier and the move
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < IT; ++j) {
@@ -314,7 +318,7 @@ QO_DEV void sj_bucket(SjLds<DENSE, NT> &s, const uint64_t *__restrict__ src, uin
         }
     }
     if (threadIdx.x < kWave) {
-        const uint64_t e = start.position(total);
+        const uint64_t e = start.position(total, asked);
         if (threadIdx.x == 0) s.base = e;
     }
     __syncthreads();
