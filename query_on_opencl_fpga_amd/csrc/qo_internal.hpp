@@ -109,10 +109,12 @@ enum TuneOp {
 // PART_LDS (join only): partition, and probe hash-mixed tables through LDS slices.
 // PART_L2 (join only): by size, with every key-range table probed through L2
 // (no key-range LDS slices).
-// Group-bys up to this many groups aggregate in one LDS table per block (4096
-// slots, three quarters full at most), larger ones are partitioned first.
-constexpr size_t kGroupbyDirect = 3072;
 enum PartMode { PART_AUTO = 0, PART_ALWAYS = 1, PART_NEVER = 2, PART_LDS = 3, PART_L2 = 4 };
+// Group-bys up to this many groups aggregate in one LDS table per block, larger ones
+// of 2^20 tuples and more are partitioned first: from 2^20 tuples on a table of 4096
+// slots, three quarters full at most, holds that many.  (Fewer tuples take the tuned
+// table, 2048 slots by default, and what it does not hold goes to the global one.)
+constexpr size_t kGroupbyDirect = 3072;
 TuneParams tune_get(int op, size_t n);
 // The built-in default of an operator (used where no class is tuned).
 TuneParams tune_builtin(int op);

@@ -218,7 +218,8 @@ int qo_autotune(int op, int size_class, int reps, int *block, int *items, int *p
     double best = 1e30;
     Cand win = cands[0];
     for (const Cand &c : cands) {
-        if (op == TUNE_GROUPBY && c.items == 4096 && (size_t)props().lds_per_block < 4096 * 24 + 8) continue;
+        // A slot is 32 bytes with its packed word, and the kernel has up to 8 KB beside the table.
+        if (op == TUNE_GROUPBY && c.items == 4096 && (size_t)props().lds_per_block < 4096 * 32 + 8192 + 8) continue;
         QO_TRY(qo_tune_set(op, size_class, c.block, c.items, c.param));
         double t = 0;
         QO_TRY(w.prepare());
